@@ -21,6 +21,7 @@
 #include <stdint.h>
 
 #include "linalg3.h"
+#include "normal64.h"
 #include "philox.h"
 
 namespace mp {
@@ -66,20 +67,16 @@ template <>
 struct Num<double> {
     static __device__ inline void box_muller(uint32_t a, uint32_t b, double &z0, double &z1)
     {
-        const double u = ((double)a + 0.5) * 0x1p-32;
-        const double v = ((double)b + 0.5) * 0x1p-32;
-        const double r = sqrt(-2.0 * log(u));
-        const double th = 2.0 * kPi * v;
-        double s, c;
-        sincos(th, &s, &c);
-        z0 = r * c;
-        z1 = r * s;
+        box_muller64(a, b, z0, z1);
     }
 };
 
 // Applied field along z at stage time.  FP32 evaluates the phase from cycles
 // c = f_red * t in FP64; FP64 evaluates h sin(2 pi f t) with t = (n+1) dt as
-// the reference does (lib/field.cpp:37-54).
+// the reference does (lib/field.cpp:37-54).  The second stage's time is
+// t + dt (lib/integrators.cpp:372-405); the FP64 sine takes it as (n+2) dt, the
+// next step's first stage time up to one rounding of t, so that one sine serves
+// both (a square wave keeps t + dt, whose rounding decides its sign at an edge).
 template <typename T, int kShape>
 struct Applied;
 
@@ -100,8 +97,15 @@ struct Applied<double, kShape> {
     {
         const int s = kShape == kMixed ? shape : kShape;
         if (s == kConstant) return amp;
-        if (s == kSine) return amp * sin(2 * kPi * f * t);
+        if (s == kSine) return amp * sin_cycles(f * t);
         return amp * ((int)(t * f * 2) % 2 ? -1 : 1);
+    }
+    // the second stage of step n -> n+1, whose first stage time is t1
+    static __device__ inline double second(int shape, double amp, double f, double dt, double n,
+                                           double t1)
+    {
+        const int s = kShape == kMixed ? shape : kShape;
+        return at(shape, amp, f, s == kSine ? (n + 2.0) * dt : t1 + dt);
     }
 };
 
@@ -315,11 +319,25 @@ __global__ __launch_bounds__(kBlock) void heun_indep_kernel(IndepArgs<T> a,
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
 
-    float hc[5], hn[5];  // table entries of the current and next group
-    auto fields = [&](int64_t n, int u, double base, T &h1, T &h2) {
+    // the field at the five stage times of the current and the next group:
+    // table entries, or (FP64 sine) evaluated a group ahead
+    constexpr bool kGroupField = kTable || (sizeof(T) == 8 && kShape == kSine);
+    T hc[5], hn[5];
+    auto group_field = [&](int64_t g, T *h) {
         if constexpr (kTable) {
-            h1 = (T)hc[u];
-            h2 = (T)hc[u + 1];
+            const float *row = htab + 4 * (g - (n0 >> 2));
+#pragma unroll
+            for (int j = 0; j < 5; ++j) h[j] = (T)row[j];
+        } else if constexpr (kGroupField) {
+#pragma unroll
+            for (int j = 1; j < 5; ++j)
+                h[j] = Applied<T, kShape>::at(shape, amp, fred, (double)(4 * g + 1 + j) * dtd);
+        }
+    };
+    auto fields = [&](int64_t n, int u, double base, T &h1, T &h2) {
+        if constexpr (kGroupField) {
+            h1 = hc[u];
+            h2 = hc[u + 1];
         } else if constexpr (sizeof(T) == 4) {
             const double c1 = (base + (double)(u + 1)) * fdt;
             h1 = Applied<T, kShape>::at(shape, amp, c1);
@@ -327,24 +345,24 @@ __global__ __launch_bounds__(kBlock) void heun_indep_kernel(IndepArgs<T> a,
         } else {
             const double t1 = (base + (double)(u + 1)) * dtd;
             h1 = Applied<T, kShape>::at(shape, amp, fred, t1);
-            h2 = Applied<T, kShape>::at(shape, amp, fred, t1 + dtd);
+            h2 = Applied<T, kShape>::second(shape, amp, fred, dtd, base + (double)u, t1);
         }
     };
 
     T zc[12], zn[12];
     const int64_t g_begin = n0 >> 2, g_end = (n1 + 3) >> 2;
     if (!kArrayNoise) group_normals(g_begin, pid, a.tag, keys, sig, zc);
-    if constexpr (kTable) {
-#pragma unroll
-        for (int j = 0; j < 5; ++j) hc[j] = htab[j];
+    if constexpr (kGroupField) {
+        group_field(g_begin, hc);
+        if constexpr (!kTable)
+            hc[0] = Applied<T, kShape>::at(shape, amp, fred, (double)(4 * g_begin + 1) * dtd);
     }
     for (int64_t g = g_begin; g < g_end; ++g) {
         const double base = (double)(4 * g);
         if (!kArrayNoise) group_normals(g + 1, pid, a.tag, keys, sig, zn);
-        if constexpr (kTable) {
-            const float *nxt = htab + 4 * (g + 1 - g_begin);
-#pragma unroll
-            for (int j = 0; j < 5; ++j) hn[j] = nxt[j];
+        if constexpr (kGroupField) {
+            group_field(g + 1, hn);
+            if constexpr (!kTable) hn[0] = hc[4];
         }
         const bool fast = 4 * g >= n0 && 4 * g + 4 <= n1 && next_rec > 4 * g + 4;
         if (!kArrayNoise && fast) {
@@ -388,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void heun_indep_kernel(IndepArgs<T> a,
 #pragma unroll
             for (int i = 0; i < 12; ++i) zc[i] = zn[i];
         }
-        if constexpr (kTable) {
+        if constexpr (kGroupField) {
 #pragma unroll
             for (int j = 0; j < 5; ++j) hc[j] = hn[j];
         }
@@ -509,8 +527,8 @@ __global__ __launch_bounds__(2 * kWave) void heun_indep_pc_kernel(IndepArgs<T> a
                                 const double t1 = (base + (double)(u + 1)) * dtd;
                                 half[kk][12 + 2 * u][lane] =
                                     Applied<T, kShape>::at(shape, amp, fred, t1);
-                                half[kk][13 + 2 * u][lane] =
-                                    Applied<T, kShape>::at(shape, amp, fred, t1 + dtd);
+                                half[kk][13 + 2 * u][lane] = Applied<T, kShape>::second(
+                                    shape, amp, fred, dtd, base + (double)u, t1);
                             }
                         }
                     }
@@ -941,7 +959,7 @@ __global__ __launch_bounds__(kCache > 0 ? 256 : 1024, kLds > 0 ? 2 : 1) void heu
             } else {
                 const double t1 = (double)(n + 1) * dtd;
                 h1 = Applied<T, kShape>::at(shape, amp, fred, t1);
-                h2 = Applied<T, kShape>::at(shape, amp, fred, t1 + dtd);
+                h2 = Applied<T, kShape>::second(shape, amp, fred, dtd, (double)n, t1);
             }
             // stage 1
             if (lead) mb0[tid] = Vec4<T>{mx, my, mz, T(0)};
