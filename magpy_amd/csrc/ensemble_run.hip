@@ -69,26 +69,28 @@ std::vector<T> cast_vec(const std::vector<double> &v)
     return std::vector<T>(v.begin(), v.end());
 }
 
-// Which Heun kernel runs n_waves integrating waves: 0 the one-wave kernel,
-// 1 the two-wave kernel with the normals formed by the producing wave, 2 (FP32)
-// the two-wave kernel with Box-Muller in the integrating wave.  FP32: 2 while
-// the integrating waves are more than one per CU and at most one per SIMD, 1
-// at one per CU or fewer, else 0 (32,768-step launches: 65,536 particles
-// 3.63e11 / 3.02e11 / 2.72e11 for 2 / 1 / 0; 16,384: 0.94e11 / 1.21e11 /
-// 0.68e11; 131,072: 2.99e11 / 2.82e11 / 3.66e11).  FP64: 0, the one-wave
-// kernel is faster at every size measured (65,536 particles: 5.7e10 against
-// 4.3e10; 16,384: 1.50e10 against 1.44e10; 1,000: 1.37e9 against 1.20e9).
-// MAGPY_AMD_HEUN_TWO_WAVE=0/1/2 forces the choice (2 means 1 in FP64).
+// Which Heun kernel runs n_waves integrating waves: 0 the one-wave kernel;
+// FP32: 1 the two-wave kernel with the normals formed by the producing wave, 2
+// the same with Box-Muller in the integrating wave; FP64: 1 (or 2) the kernel
+// with three producing waves per integrating wave.  FP32: 2 while the
+// integrating waves are more than one per CU and at most one per SIMD, 1 at one
+// per CU or fewer, else 0 (32,768-step launches: 65,536 particles 3.63e11 /
+// 3.02e11 / 2.72e11 for 2 / 1 / 0; 16,384: 0.94e11 / 1.21e11 / 0.68e11; 131,072:
+// 2.99e11 / 2.82e11 / 3.66e11).  FP64: 1 up to two integrating waves per CU,
+// where the producing waves have SIMDs of their own (us per step, 1 / 0, sine
+// field: 1,000 particles 0.146 / 0.428, 16,384 0.157 / 0.439, 32,768 0.262 /
+// 0.434, 65,536 0.493 / 0.458, 131,072 0.986 / 0.838).
+// MAGPY_AMD_HEUN_TWO_WAVE=0/1/2 forces the choice.
 int two_wave_mode(int n_waves, bool fp32)
 {
     if (const char *env = std::getenv("MAGPY_AMD_HEUN_TWO_WAVE")) {
         const int v = std::atoi(env);
         return v <= 0 ? 0 : (v >= 2 && fp32) ? 2 : 1;
     }
-    if (!fp32) return 0;
     int dev = 0, cus = 0;
     MP_HIP(hipGetDevice(&dev));
     MP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (!fp32) return n_waves <= 2 * cus ? 1 : 0;
     if (n_waves > 4 * cus) return 0;
     return n_waves > cus ? 2 : 1;
 }
@@ -100,9 +102,10 @@ void launch_heun(const mp::IndepArgs<T> &a, int grid, hipStream_t s, const float
 {
     if constexpr (!kArray) {
         if (two_wave != 0) {
-            // one (integrating, producing) wave pair per workgroup; two or
-            // four pairs per workgroup measure the same or slower
-            const dim3 g2((unsigned)(grid * (mp::kBlock / mp::kWave))), b2(2 * mp::kWave);
+            // one integrating wave per workgroup (FP32: one (integrating,
+            // producing) pair; two or four pairs measure the same or slower)
+            const dim3 g2((unsigned)(grid * (mp::kBlock / mp::kWave))),
+                b2(sizeof(T) == 4 ? 2 * mp::kWave : 4 * mp::kWave);
             if constexpr (sizeof(T) == 4) {
                 auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g2, b2, 0, s, a, htab); };
                 if (htab) {
@@ -116,8 +119,9 @@ void launch_heun(const mp::IndepArgs<T> &a, int grid, hipStream_t s, const float
                 else go(mp::heun_indep_pc_kernel<T, kShape, false, kRenorm, false>);
                 return;
             }
-            hipLaunchKernelGGL((mp::heun_indep_pc_kernel<T, kShape, false, kRenorm, false>), g2,
-                               b2, 0, s, a, htab);
+            if constexpr (sizeof(T) == 8)
+                hipLaunchKernelGGL((mp::heun_indep_pc_kernel<T, kShape, false, kRenorm, false, 3>),
+                                   g2, b2, 0, s, a, htab);
             return;
         }
     }

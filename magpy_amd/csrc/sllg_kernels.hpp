@@ -432,12 +432,19 @@ __global__ __launch_bounds__(kBlock) void heun_indep_kernel(IndepArgs<T> a,
 // are too few to give each SIMD several integrating waves.  Every value is
 // computed by the same expression as in heun_indep_kernel, so the results
 // are the same bit for bit.
-// Ring halves of 4 groups (24 KB, FP32 with a table), 2 groups (20 KB, FP32
-// with per-lane fields) or 1 group (20 KB, FP64): four workgroups of a CU fit.
-template <typename T, bool kTable>
+// FP32: one producing wave and ring halves of 4 groups (24 KB, with a table) or
+// 2 (20 KB, per-lane fields), so four workgroups of a CU fit.  FP64: three
+// producing waves, whose noise takes 2.4 times the integrating wave's step, each
+// filling one group of a half of 3 (at most 60 KB, two workgroups of a CU).  A
+// group's rows are its normals, then the applied field: none with a table or an
+// FP64 constant field, the five stage times of an FP64 sine, else (h1, h2) of
+// each step.
+template <typename T, int kShape, bool kTable, int kProducers>
 struct HeunRing {
-    static constexpr int kGroups = sizeof(T) == 8 ? 1 : kTable ? 4 : 2;
-    static constexpr int kRows = kTable ? 12 : 20;   // normals, then (h1, h2) of each step
+    static constexpr int kGroups = sizeof(T) == 8 ? kProducers : kTable ? 4 : 2;
+    static constexpr bool kNoField = kTable || (sizeof(T) == 8 && kShape == kConstant);
+    static constexpr bool kSineRows = sizeof(T) == 8 && kShape == kSine;
+    static constexpr int kRows = 12 + (kNoField ? 0 : kSineRows ? 5 : 8);
 };
 
 // htab is deliberately not __restrict__: the integrator then reads it with
@@ -451,16 +458,19 @@ struct HeunRing {
 // Box-Muller work to the integrating wave fills the stalls of its step chain;
 // with fewer integrating waves than SIMDs the integrating wave runs alone and
 // the producer should carry it.
-template <typename T, int kShape, bool kTable, bool kRenorm, bool kBmInt>
-__global__ __launch_bounds__(2 * kWave) void heun_indep_pc_kernel(IndepArgs<T> a,
-                                                                  const float *htab)
+template <typename T, int kShape, bool kTable, bool kRenorm, bool kBmInt, int kProducers = 1>
+__global__ __launch_bounds__((1 + kProducers) * kWave) void heun_indep_pc_kernel(
+    IndepArgs<T> a, const float *htab)
 {
     static_assert(sizeof(T) == 4 || !kTable, "the shared field table is FP32");
     static_assert(sizeof(T) == 4 || !kBmInt, "Box-Muller in the integrating wave is FP32");
-    constexpr int K = HeunRing<T, kTable>::kGroups, R = HeunRing<T, kTable>::kRows;
+    using Ring = HeunRing<T, kShape, kTable, kProducers>;
+    constexpr int K = Ring::kGroups, R = Ring::kRows;
     __shared__ T ring[2][K][R][kWave];
     const int lane = threadIdx.x & (kWave - 1);
-    const bool producer = __builtin_amdgcn_readfirstlane(threadIdx.x) >= kWave;
+    // wave 0 integrates, waves 1 .. kProducers fill every kProducers-th group
+    const int role = (int)(__builtin_amdgcn_readfirstlane(threadIdx.x) / kWave);
+    const bool producer = role > 0;
     const int wave = blockIdx.x;
     const int p = wave * kWave + lane;
     const bool live = p < a.n;
@@ -492,7 +502,7 @@ __global__ __launch_bounds__(2 * kWave) void heun_indep_pc_kernel(IndepArgs<T> a
         if (producer) {
             if (c < n_chunks) {
                 T (*half)[R][kWave] = ring[c & 1];
-                for (int kk = 0; kk < K; ++kk) {
+                for (int kk = role - 1; kk < K; kk += kProducers) {
                     const int64_t g = g_begin + c * K + kk;
                     if (g >= g_end) break;
                     if constexpr (kBmInt) {
@@ -514,7 +524,12 @@ __global__ __launch_bounds__(2 * kWave) void heun_indep_pc_kernel(IndepArgs<T> a
 #pragma unroll
                         for (int i = 0; i < 12; ++i) half[kk][i][lane] = z[i];
                     }
-                    if constexpr (!kTable) {
+                    if constexpr (Ring::kSineRows) {
+#pragma unroll
+                        for (int j = 0; j < 5; ++j)
+                            half[kk][12 + j][lane] = Applied<T, kShape>::at(
+                                shape, amp, fred, (double)(4 * g + 1 + j) * dtd);
+                    } else if constexpr (!Ring::kNoField) {
                         const double base = (double)(4 * g);
 #pragma unroll
                         for (int u = 0; u < 4; ++u) {
@@ -550,6 +565,15 @@ __global__ __launch_bounds__(2 * kWave) void heun_indep_pc_kernel(IndepArgs<T> a
                     for (int u = 0; u < 4; ++u) {
                         hh1[u] = tg[u];
                         hh2[u] = tg[u + 1];
+                    }
+                } else if constexpr (Ring::kNoField) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) hh1[u] = hh2[u] = amp;
+                } else if constexpr (Ring::kSineRows) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        hh1[u] = half[kk][12 + u][lane];
+                        hh2[u] = half[kk][13 + u][lane];
                     }
                 } else {
 #pragma unroll
