@@ -22,6 +22,7 @@
 #include <new>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "host_util.hpp"
@@ -483,16 +484,23 @@ struct GroupRun : GroupBase {
         mp::ImplicitClusterArgs ia{
             mp::ClusterArgs<double>{a, d_px.p, d_py.p, d_pz.p, d_w.p, d_cbase.p, d_csize.p}, eps,
             max_iter, d_it.p, d_fl.p, interactions ? 1 : 0};
-        const size_t shmem = 3 * (size_t)block * sizeof(mp::Vec4<double>);
+        // positions and iterates, then a square and a flag per slot
+        const size_t shmem =
+            (size_t)block * (2 * sizeof(mp::Vec4<double>) + sizeof(double) + sizeof(int));
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), shmem, s, ia);
         };
-        switch (shape_kind) {
-        case mp::kSine: go(mp::implicit_cluster_kernel<mp::kSine, kArray>); break;
-        case mp::kSquare: go(mp::implicit_cluster_kernel<mp::kSquare, kArray>); break;
-        case mp::kConstant: go(mp::implicit_cluster_kernel<mp::kConstant, kArray>); break;
-        default: go(mp::implicit_cluster_kernel<mp::kMixed, kArray>); break;
-        }
+        auto shaped = [&](auto one_wave) {
+            constexpr bool W = decltype(one_wave)::value;
+            switch (shape_kind) {
+            case mp::kSine: go(mp::implicit_cluster_kernel<mp::kSine, kArray, W>); break;
+            case mp::kSquare: go(mp::implicit_cluster_kernel<mp::kSquare, kArray, W>); break;
+            case mp::kConstant: go(mp::implicit_cluster_kernel<mp::kConstant, kArray, W>); break;
+            default: go(mp::implicit_cluster_kernel<mp::kMixed, kArray, W>); break;
+            }
+        };
+        if (block == mp::kWave) shaped(std::true_type{});
+        else shaped(std::false_type{});
     }
 
     template <int L, bool kArray>

@@ -699,7 +699,7 @@ __device__ inline void dipolar_term(const Vec4<T> &pi, const Vec4<T> &pj, const 
     const T r2 = skip ? T(1) : fmad(dx, dx, fmad(dy, dy, dz * dz));
     T rinv;
     if constexpr (sizeof(T) == 4) rinv = __builtin_amdgcn_rsqf(r2);
-    else rinv = 1.0 / sqrt(r2);
+    else rinv = rsqrt_normal(r2);
     const T rinv2 = rinv * rinv;
     const T c = skip ? T(0) : pj.w * rinv2 * rinv;
     const T t = T(3) * fmad(mj.x, dx, fmad(mj.y, dy, mj.z * dz)) * rinv2;
@@ -1060,53 +1060,130 @@ struct ImplicitArgs {
     unsigned long long *newton_fail;    // [n]
 };
 
-__device__ inline void drift3(const double *m, double al, const double *h, double *d)
+// The Newton system of one particle at the iterate m: f = -F and J = dF/dm of
+//   F(m) = m - x0 - (a(m) dt + B(m) dW) / 2,
+// h the field at m and s = sr dW.  Drift and diffusion are the one bilinear map
+// L (llg_map), so F costs one L at v = h dt + s, and
+//   J = I - (dL/dm (m; h + s) + L(m, c) e0^T) / 2,
+// the field Jacobian being c e0^T; the drift term has no dt, and the two
+// diffusion-Jacobian entries that lib/llg.cpp:128, 156 take at m2 are added:
+// alpha (m0 - m2) s1 to row 0, 2 alpha (m2 - m1) s2 to row 2 of column 1.
+// dL_i/dm_j (m; g) = -eps_ijk g_k + alpha (2 g_i m_j - m_i g_j - delta_ij m.g).
+// 79 FP64 operations; the separate drift, diffusion and Jacobian arrays of the
+// reference's formulas were 230.
+struct NewtonSystem {
+    double f[3], J[9];
+};
+
+__device__ inline NewtonSystem midpoint_system(const double *m, const double *x0, const double *h,
+                                               const double *s, double dt, double al,
+                                               const double *c_half, const double *e0)
 {
-    d[0] = m[2] * h[1] - m[1] * h[2] + al * (h[0] * (m[1] * m[1] + m[2] * m[2]) - m[0] * (m[1] * h[1] + m[2] * h[2]));
-    d[1] = m[0] * h[2] - m[2] * h[0] + al * (h[1] * (m[0] * m[0] + m[2] * m[2]) - m[1] * (m[0] * h[0] + m[2] * h[2]));
-    d[2] = m[1] * h[0] - m[0] * h[1] + al * (h[2] * (m[0] * m[0] + m[1] * m[1]) - m[2] * (m[0] * h[0] + m[1] * h[1]));
+#pragma clang fp contract(off)
+    NewtonSystem n;
+    double lx, ly, lz;
+    llg_map(m[0], m[1], m[2], fmad(h[0], dt, s[0]), fmad(h[1], dt, s[1]), fmad(h[2], dt, s[2]), al,
+            lx, ly, lz);
+    n.f[0] = fmad(0.5, lx, x0[0] - m[0]);
+    n.f[1] = fmad(0.5, ly, x0[1] - m[1]);
+    n.f[2] = fmad(0.5, lz, x0[2] - m[2]);
+    const double g[3] = {h[0] + s[0], h[1] + s[1], h[2] + s[2]};
+    const double G[3] = {0.5 * g[0], 0.5 * g[1], 0.5 * g[2]};
+    const double P[3] = {al * m[0], al * m[1], al * m[2]};
+    double C[3];
+    llg_map(m[0], m[1], m[2], c_half[0], c_half[1], c_half[2], al, C[0], C[1], C[2]);
+    const double T = fmad(P[0], G[0], fmad(P[1], G[1], fmad(P[2], G[2], 1.0)));
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        n.J[4 * i] = fmad(-C[i], e0[i], fmad(-P[i], G[i], T));
+    // off the diagonal: -eps_ijk G_k with the sign of (i, j)
+    auto off = [&](int i, int j, double eps_g) {
+        return fmad(-g[i], P[j], fmad(P[i], G[j], fmad(-C[i], e0[j], eps_g)));
+    };
+    n.J[1] = off(0, 1, fmad(P[2] - P[0], 0.5 * s[1], G[2]));
+    n.J[2] = off(0, 2, -G[1]);
+    n.J[3] = off(1, 0, -G[2]);
+    n.J[5] = off(1, 2, G[0]);
+    n.J[6] = off(2, 0, G[1]);
+    n.J[7] = off(2, 1, fmad(P[1] - P[2], s[2], -G[0]));
+    return n;
 }
 
-__device__ inline void diffusion3(const double *m, double sr, double al, double *B)
+// J x = f by cofactors (x returned in f): the Newton matrices are I plus a small
+// part, for which one determinant and one reciprocal do, where LU takes five
+// dependent divisions.  Where the determinant cancels to 2^-24 of its terms, or
+// is not finite, solve3's pivoted LU decides, and a zero pivot returns false
+// with f unchanged, as LAPACK's dgesv leaves its right-hand side.
+__device__ inline bool newton_solve(NewtonSystem &n)
 {
-    B[0] = al * sr * (m[1] * m[1] + m[2] * m[2]);
-    B[1] = sr * (m[2] - al * m[0] * m[1]);
-    B[2] = -sr * (m[1] + al * m[0] * m[2]);
-    B[3] = -sr * (m[2] + al * m[0] * m[1]);
-    B[4] = al * sr * (m[0] * m[0] + m[2] * m[2]);
-    B[5] = sr * (m[0] - al * m[1] * m[2]);
-    B[6] = sr * (m[1] - al * m[0] * m[2]);
-    B[7] = -sr * (m[0] + al * m[1] * m[2]);
-    B[8] = al * sr * (m[0] * m[0] + m[1] * m[1]);
+#pragma clang fp contract(off)
+    const double *J = n.J;
+    // u = b x c, v = c x a, w = a x b of J's columns a, b, c
+    auto minor = [](double p, double q, double r, double t) { return fmad(p, q, -(r * t)); };
+    const double u0 = minor(J[4], J[8], J[7], J[5]), u1 = minor(J[7], J[2], J[1], J[8]),
+                 u2 = minor(J[1], J[5], J[4], J[2]);
+    const double v0 = minor(J[5], J[6], J[8], J[3]), v1 = minor(J[8], J[0], J[2], J[6]),
+                 v2 = minor(J[2], J[3], J[5], J[0]);
+    const double w0 = minor(J[3], J[7], J[6], J[4]), w1 = minor(J[6], J[1], J[0], J[7]),
+                 w2 = minor(J[0], J[4], J[3], J[1]);
+    const double t0 = J[0] * u0, t1 = J[3] * u1, t2 = J[6] * u2;
+    const double det = t0 + t1 + t2, size = fabs(t0) + fabs(t1) + fabs(t2);
+    if (!(fabs(det) > 0x1p-24 * size && size < 0x1p600)) return solve3(n.J, n.f);
+    const double r = rcp_normal(det);
+    const double f0 = n.f[0], f1 = n.f[1], f2 = n.f[2];
+    n.f[0] = fmad(u0, f0, fmad(u1, f1, u2 * f2)) * r;
+    n.f[1] = fmad(v0, f0, fmad(v1, f1, v2 * f2)) * r;
+    n.f[2] = fmad(w0, f0, fmad(w1, f1, w2 * f2)) * r;
+    return true;
 }
 
-// d(drift)/dm, row-major, hj = field Jacobian (row-major)
-__device__ inline void drift_jac3(const double *m, double a, const double *h, const double *hj, double *j)
+// The uniaxial anisotropy field and the applied field along z
+__device__ inline void single_field(const double *m, const double *e, double k, double applied,
+                                    double *h)
 {
-    j[0] = m[2] * hj[3] - m[1] * hj[6] + a * (-m[1] * h[1] - m[2] * h[2] + (m[1] * m[1] + m[2] * m[2]) * hj[0] - m[0] * (m[1] * hj[3] + m[2] * hj[6]));
-    j[1] = -h[2] + m[2] * hj[4] - m[1] * hj[7] + a * (2 * m[1] * h[0] + (m[1] * m[1] + m[2] * m[2]) * hj[1] - m[0] * (h[1] + m[1] * hj[4] + m[2] * hj[7]));
-    j[2] = h[1] + m[2] * hj[5] - m[1] * hj[8] + a * (2 * m[2] * h[0] + (m[1] * m[1] + m[2] * m[2]) * hj[2] - m[0] * (h[2] + m[1] * hj[5] + m[2] * hj[8]));
-    j[3] = h[2] - m[2] * hj[0] + m[0] * hj[6] + a * (2 * m[0] * h[1] + (m[0] * m[0] + m[2] * m[2]) * hj[3] - m[1] * (h[0] + m[0] * hj[0] + m[2] * hj[6]));
-    j[4] = -m[2] * hj[1] + m[0] * hj[7] + a * (-m[0] * h[0] - m[2] * h[2] + (m[0] * m[0] + m[2] * m[2]) * hj[4] - m[1] * (m[0] * hj[1] + m[2] * hj[7]));
-    j[5] = -h[0] - m[2] * hj[2] + m[0] * hj[8] + a * (2 * m[2] * h[1] + (m[0] * m[0] + m[2] * m[2]) * hj[5] - m[1] * (h[2] + m[0] * hj[2] + m[2] * hj[8]));
-    j[6] = -h[1] + m[1] * hj[0] - m[0] * hj[3] + a * (2 * m[0] * h[2] + (m[0] * m[0] + m[1] * m[1]) * hj[6] - m[2] * (h[0] + m[0] * hj[0] + m[1] * hj[3]));
-    j[7] = h[0] + m[1] * hj[1] - m[0] * hj[4] + a * (2 * m[1] * h[2] + (m[0] * m[0] + m[1] * m[1]) * hj[7] - m[2] * (h[1] + m[0] * hj[1] + m[1] * hj[4]));
-    j[8] = m[1] * hj[2] - m[0] * hj[5] + a * (-m[0] * h[0] - m[1] * h[1] + (m[0] * m[0] + m[1] * m[1]) * hj[8] - m[2] * (m[0] * hj[2] + m[1] * hj[5]));
+#pragma clang fp contract(off)
+    const double d = fmad(m[0], e[0], fmad(m[1], e[1], m[2] * e[2])) * k;
+    h[0] = d * e[0];
+    h[1] = d * e[1];
+    h[2] = fmad(d, e[2], applied);
 }
 
-// jb[z + 3y + 9x] = dB[x][y]/dm[z] as lib/llg.cpp:118-158 writes it
-__device__ inline void diffusion_jac3(const double *m, double sr, double al, double *jb)
+// The Euler guess x0/2 + (a dt + B dW)/2 (lib/integrators.cpp:605-614)
+__device__ inline void midpoint_guess(const double *x0, const double *h, const double *s, double dt,
+                                      double al, double *y)
 {
-    jb[0] = 0;                  jb[1] = 2 * al * sr * m[1];  jb[2] = 2 * al * sr * m[2];
-    jb[3] = -al * sr * m[1];    jb[4] = -al * sr * m[2];     jb[5] = sr;
-    jb[6] = -al * sr * m[2];    jb[7] = -sr;                 jb[8] = -al * sr * m[0];
-    jb[9] = -al * sr * m[1];    jb[10] = -al * sr * m[0];    jb[11] = -sr;
-    jb[12] = 2 * al * sr * m[0]; jb[13] = 0;                 jb[14] = 2 * al * sr * m[2];
-    jb[15] = sr;                jb[16] = -al * sr * m[2];    jb[17] = -al * sr * m[1];
-    jb[18] = -al * sr * m[2];   jb[19] = sr;                 jb[20] = -al * sr * m[0];
-    jb[21] = -sr;               jb[22] = -al * sr * m[2];    jb[23] = -al * sr * m[1];
-    jb[24] = 2 * al * sr * m[0]; jb[25] = 2 * al * sr * m[2]; jb[26] = 0;
+#pragma clang fp contract(off)
+    double lx, ly, lz;
+    llg_map(x0[0], x0[1], x0[2], fmad(h[0], dt, s[0]), fmad(h[1], dt, s[1]), fmad(h[2], dt, s[2]),
+            al, lx, ly, lz);
+    y[0] = 0.5 * (lx + x0[0]);
+    y[1] = 0.5 * (ly + x0[1]);
+    y[2] = 0.5 * (lz + x0[2]);
 }
+
+// Wiener normals of consecutive steps, one Philox call at a time
+struct StepNormals {
+    double z[4];
+    uint64_t have = UINT64_MAX;
+    __device__ inline void get(int64_t n, uint32_t pid, uint32_t tag, const PhiloxKeys &keys,
+                               double *w)
+    {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint64_t j = 3 * (uint64_t)n + d;
+            const uint64_t c = j >> 2;
+            if (c != have) {
+                const u32x4 r =
+                    philox4x32_10(u32x4{(uint32_t)c, (uint32_t)(c >> 32), pid, tag}, keys);
+                Num<double>::box_muller(r.x, r.y, z[0], z[1]);
+                Num<double>::box_muller(r.z, r.w, z[2], z[3]);
+                have = c;
+            }
+            const int jj = (int)(j & 3);
+            w[d] = jj == 0 ? z[0] : jj == 1 ? z[1] : jj == 2 ? z[2] : z[3];
+        }
+    }
+};
 
 template <int kShape, bool kArrayNoise>
 __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
@@ -1128,18 +1205,13 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
     const uint32_t pid = a.pid[q];
     const double ah = sqrt(2 * 1000.0 * fabs(log(dt)));
     const double sdt = sqrt(dt);
-    // field Jacobian k e e^T (lib/field.cpp:159-174)
-    double hj[9];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) hj[i * 3 + j] = k * e[i] * e[j];
+    // half the field Jacobian k e e^T (lib/field.cpp:159-174) as c e^T
+    const double c_half[3] = {0.5 * k * e[0], 0.5 * k * e[1], 0.5 * k * e[2]};
 
     unsigned long long iters = 0, fails = 0;
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
-    double zbuf[4];
-    uint64_t have = UINT64_MAX;
+    StepNormals normals;
 
     for (int64_t n = a.n0; n < a.n1; ++n) {
         double w[3];
@@ -1147,85 +1219,36 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
             const double *src = a.noise + ((size_t)n * (size_t)a.n + (size_t)q) * 3;
             w[0] = src[0]; w[1] = src[1]; w[2] = src[2];
         } else {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const uint64_t j = 3 * (uint64_t)n + d;
-                const uint64_t c = j >> 2;
-                if (c != have) {
-                    const u32x4 r = philox4x32_10(u32x4{(uint32_t)c, (uint32_t)(c >> 32), pid, a.tag}, keys);
-                    Num<double>::box_muller(r.x, r.y, zbuf[0], zbuf[1]);
-                    Num<double>::box_muller(r.z, r.w, zbuf[2], zbuf[3]);
-                    have = c;
-                }
-                const int jj = (int)(j & 3);
-                w[d] = jj == 0 ? zbuf[0] : jj == 1 ? zbuf[1] : jj == 2 ? zbuf[2] : zbuf[3];
-            }
+            normals.get(n, pid, a.tag, keys, w);
         }
         const double t = (double)(n + 1) * dt;
-        double dwm[3];
+        double sw[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) dwm[d] = fmax(-ah, fmin(ah, w[d])) * sdt;
+        for (int d = 0; d < 3; ++d) sw[d] = sr * (fmax(-ah, fmin(ah, w[d])) * sdt);
 
-        // Euler guess from sde(x0, t) (lib/integrators.cpp:605-614)
-        double h[3], dr[3], B[9];
-        {
-            const double dot = (x0[0] * e[0] + x0[1] * e[1] + x0[2] * e[2]) * k;
-            h[0] = dot * e[0];
-            h[1] = dot * e[1];
-            h[2] = dot * e[2] + Applied<double, kShape>::at(shape, amp, fred, t);
-        }
-        drift3(x0, al, h, dr);
-        diffusion3(x0, sr, al, B);
-        double y[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            double g = dr[i] * dt;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) g += B[i * 3 + j] * dwm[j];
-            y[i] = (g + x0[i]) / 2;
-        }
+        double h[3], y[3];
+        single_field(x0, e, k, Applied<double, kShape>::at(shape, amp, fred, t), h);
+        midpoint_guess(x0, h, sw, dt, al, y);
         const double happ_mid = Applied<double, kShape>::at(shape, amp, fred, t + dt / 2);
         const double tol = ia.eps * sqrt(y[0] * y[0] + y[1] * y[1] + y[2] * y[2]);
-        double err = 2 * tol;
+        // |delta| > tol, tested on squares after the first iteration
+        bool over = 2 * tol > tol;
+        const double tol2 = tol * tol;
         int iter = ia.max_iter;
         bool singular = false;
-        while ((err > tol) && (iter-- > 0)) {
-            const double xt[3] = {y[0], y[1], y[2]};
-            const double dot = (xt[0] * e[0] + xt[1] * e[1] + xt[2] * e[2]) * k;
-            h[0] = dot * e[0];
-            h[1] = dot * e[1];
-            h[2] = dot * e[2] + happ_mid;
-            drift3(xt, al, h, dr);
-            diffusion3(xt, sr, al, B);
-            double J[9], jb[27], F[3];
-            drift_jac3(xt, al, h, hj, J);
-            diffusion_jac3(xt, sr, al, jb);
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                F[i] = xt[i] - 0.5 * dr[i] * dt - x0[i];
-#pragma unroll
-                for (int j = 0; j < 3; ++j) F[i] -= 0.5 * B[i * 3 + j] * dwm[j];
-            }
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-#pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    double v = (double)(i == j) - 0.5 * J[i * 3 + j];
-#pragma unroll
-                    for (int kk = 0; kk < 3; ++kk) v -= 0.5 * jb[i * 9 + kk * 3 + j] * dwm[kk];
-                    J[i * 3 + j] = v;
-                }
-            double dlt[3] = {-F[0], -F[1], -F[2]};
+        while (over && (iter-- > 0)) {
+            single_field(y, e, k, happ_mid, h);
+            NewtonSystem ns = midpoint_system(y, x0, h, sw, dt, al, c_half, e);
             ++iters;
-            if (!solve3(J, dlt)) {  // LAPACK_ERR: x_root left at -F
-                y[0] = dlt[0]; y[1] = dlt[1]; y[2] = dlt[2];
+            if (!newton_solve(ns)) {  // LAPACK_ERR: x_root left at -F
+                y[0] = ns.f[0]; y[1] = ns.f[1]; y[2] = ns.f[2];
                 singular = true;
                 break;
             }
-            err = sqrt(dlt[0] * dlt[0] + dlt[1] * dlt[1] + dlt[2] * dlt[2]);
-            y[0] = dlt[0] + xt[0];
-            y[1] = dlt[1] + xt[1];
-            y[2] = dlt[2] + xt[2];
+            over = fmad(ns.f[0], ns.f[0], fmad(ns.f[1], ns.f[1], ns.f[2] * ns.f[2])) > tol2;
+            y[0] += ns.f[0];
+            y[1] += ns.f[1];
+            y[2] += ns.f[2];
         }
         if (singular || iter == -1) ++fails;
 #pragma unroll
@@ -1293,8 +1316,24 @@ struct ImplicitClusterArgs {
 
 constexpr int kImplicitClusterBlock = 256;   // largest workgroup, so largest cluster
 
-template <int kShape, bool kArrayNoise>
-__global__ __launch_bounds__(kImplicitClusterBlock) void implicit_cluster_kernel(
+// Order LDS accesses of the workgroup: a barrier, or, where the workgroup is one
+// wave (whose LDS accesses complete in order), only the compiler's order.
+template <bool kOneWave>
+__device__ inline void lds_sync()
+{
+    if constexpr (kOneWave) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
+// kOneWave: the workgroup is one wave (clusters of at most 64 particles), so
+// an iteration needs no barrier.
+template <int kShape, bool kArrayNoise, bool kOneWave>
+__global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void implicit_cluster_kernel(
     ImplicitClusterArgs ia)
 {
     const ClusterArgs<double> &ca = ia.c;
@@ -1303,7 +1342,8 @@ __global__ __launch_bounds__(kImplicitClusterBlock) void implicit_cluster_kernel
     const int slots = blockDim.x;
     Vec4<double> *pos = reinterpret_cast<Vec4<double> *>(smem_raw);
     Vec4<double> *mb = pos + slots;    // the states the field is taken from
-    Vec4<double> *red = mb + slots;    // vectors whose cluster norm is taken
+    double *red = reinterpret_cast<double *>(mb + slots);  // squares whose cluster sum is taken
+    int *sing = reinterpret_cast<int *>(red + slots);      // a cluster's first slot: singular block
 
     const int tid = threadIdx.x;
     const int p = blockIdx.x * slots + tid;   // the grid covers all slots exactly
@@ -1324,29 +1364,60 @@ __global__ __launch_bounds__(kImplicitClusterBlock) void implicit_cluster_kernel
     const double ah = sqrt(2 * 1000.0 * fabs(log(dt)));
     const double sdt = sqrt(dt);
     pos[tid] = Vec4<double>{ca.px[p], ca.py[p], ca.pz[p], ca.w[p]};
+    sing[tid] = 0;
 
     // hj + 3n of the 3N x 3N field Jacobian J[i][j] = k_{i/3} e[i] e[j] for
     // i/3 == j/3 (lib/field.cpp:159-174): flat index f = 3n + q, row f / 3N,
     // column f % 3N.  For every n < N that row is 0, 1 or 2, i.e. particle 0's
-    // block row, nonzero in columns 0-2 only.
-    double hj[9];
+    // block row, nonzero in columns 0-2 only: row r of the 3 x 3 slice is
+    // k e[i] e^T of particle 0 where n + r = i N, else zero, so the slice is
+    // c e^T with c_r = k e[i] or 0.
+    double c_half[3], e0[3];
     {
         const int nn = live ? cn : 1, idx = live ? tid - cb : 0;
         const int first = blockIdx.x * slots + cb;
         const double k0 = a.k[first];
-        const double e0[3] = {a.ex[first], a.ey[first], a.ez[first]};
+        e0[0] = a.ex[first];
+        e0[1] = a.ey[first];
+        e0[2] = a.ez[first];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const int f = 3 * idx + q, i = f / (3 * nn), j = f % (3 * nn);
-            hj[q] = (i < 3 && j < 3) ? k0 * e0[i < 3 ? i : 0] * e0[j < 3 ? j : 0] : 0.0;
+        for (int r = 0; r < 3; ++r) {
+            const int i = (idx + r) / nn;
+            const double ei = i == 0 ? e0[0] : i == 1 ? e0[1] : e0[2];
+            c_half[r] = (idx + r) % nn == 0 && i < 3 ? 0.5 * k0 * ei : 0.0;
         }
     }
 
     unsigned long long iters = 0, fails = 0;
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
-    double zbuf[4];
-    uint64_t have = UINT64_MAX;
+    StepNormals normals;
+
+    // the sum of red over the cluster's slots, as two sums added at the end
+    auto cluster_sum = [&]() {
+        double s0 = 0.0, s1 = 0.0;
+        int j = cb;
+        for (; j + 4 <= ce; j += 4) {
+            s0 += red[j];
+            s1 += red[j + 1];
+            s0 += red[j + 2];
+            s1 += red[j + 3];
+        }
+        for (; j < ce; ++j) s0 += red[j];
+        return s0 + s1;
+    };
+    auto square = [](const double *v) { return fmad(v[0], v[0], fmad(v[1], v[1], v[2] * v[2])); };
+    // the field of the state m, the dipolar sum of the states in mb added
+    auto field = [&](const double *m, double applied, double *h) {
+        single_field(m, e, k, applied, h);
+        if (ia.interactions) {
+            double d[3];
+            dipolar_field<double, 1>(pos, mb, tid, cb, ce, 0, d[0], d[1], d[2]);
+            h[0] += d[0];
+            h[1] += d[1];
+            h[2] += d[2];
+        }
+    };
 
     for (int64_t n = a.n0; n < a.n1; ++n) {
         double w[3];
@@ -1354,137 +1425,71 @@ __global__ __launch_bounds__(kImplicitClusterBlock) void implicit_cluster_kernel
             const double *src = a.noise + ((size_t)n * (size_t)a.n + (size_t)p) * 3;
             w[0] = src[0]; w[1] = src[1]; w[2] = src[2];
         } else {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const uint64_t j = 3 * (uint64_t)n + d;
-                const uint64_t c = j >> 2;
-                if (c != have) {
-                    const u32x4 r = philox4x32_10(u32x4{(uint32_t)c, (uint32_t)(c >> 32), pid, a.tag}, keys);
-                    Num<double>::box_muller(r.x, r.y, zbuf[0], zbuf[1]);
-                    Num<double>::box_muller(r.z, r.w, zbuf[2], zbuf[3]);
-                    have = c;
-                }
-                const int jj = (int)(j & 3);
-                w[d] = jj == 0 ? zbuf[0] : jj == 1 ? zbuf[1] : jj == 2 ? zbuf[2] : zbuf[3];
-            }
+            normals.get(n, pid, a.tag, keys, w);
         }
         const double t = (double)(n + 1) * dt;
-        double dwm[3];
+        double sw[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) dwm[d] = fmax(-ah, fmin(ah, w[d])) * sdt;
+        for (int d = 0; d < 3; ++d) sw[d] = sr * (fmax(-ah, fmin(ah, w[d])) * sdt);
 
-        // Euler guess from sde(x0, t), the field including the cluster's
-        // dipolar sum at x0 (lib/integrators.cpp:605-614)
+        // Euler guess, the field including the cluster's dipolar sum at x0
         mb[tid] = Vec4<double>{x0[0], x0[1], x0[2], 0.0};
-        __syncthreads();
-        double h[3], hd[3] = {0.0, 0.0, 0.0}, dr[3], B[9], y[3];
-        if (ia.interactions) dipolar_field<double, 1>(pos, mb, tid, cb, ce, 0, hd[0], hd[1], hd[2]);
-        {
-            const double dot = (x0[0] * e[0] + x0[1] * e[1] + x0[2] * e[2]) * k;
-            h[0] = dot * e[0];
-            h[1] = dot * e[1];
-            h[2] = dot * e[2] + Applied<double, kShape>::at(shape, amp, fred, t);
-            if (ia.interactions) {
-                h[0] = h[0] + hd[0];
-                h[1] = h[1] + hd[1];
-                h[2] = h[2] + hd[2];
-            }
-        }
-        drift3(x0, al, h, dr);
-        diffusion3(x0, sr, al, B);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            double g = dr[i] * dt;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) g += B[i * 3 + j] * dwm[j];
-            y[i] = (g + x0[i]) / 2;
-        }
-        red[tid] = Vec4<double>{y[0], y[1], y[2], 0.0};
-        __syncthreads();   // every lane's guess field is taken: mb may change
-        double ss = 0.0;
-        for (int j = cb; j < ce; ++j) {
-            const Vec4<double> v = red[j];
-            ss += v.x * v.x;
-            ss += v.y * v.y;
-            ss += v.z * v.z;
-        }
-        const double tol = ia.eps * sqrt(ss);
+        lds_sync<kOneWave>();
+        double h[3], y[3];
+        field(x0, Applied<double, kShape>::at(shape, amp, fred, t), h);
+        midpoint_guess(x0, h, sw, dt, al, y);
+        red[tid] = square(y);
+        lds_sync<kOneWave>();   // every lane's guess field is taken: mb may change
+        const double tol = ia.eps * sqrt(cluster_sum());
+        const double tol2 = tol * tol;
         mb[tid] = Vec4<double>{y[0], y[1], y[2], 0.0};
         const double happ_mid = Applied<double, kShape>::at(shape, amp, fred, t + dt / 2);
-        double err = 2 * tol;
         int iter = ia.max_iter;
         bool singular = false;
-        bool go = live && (err > tol) && (iter-- > 0);
-        while (__syncthreads_or(go)) {
-            const double xt[3] = {y[0], y[1], y[2]};
+        bool go = live && (2 * tol > tol) && (iter-- > 0);
+        auto any_go = [&]() {
+            if constexpr (kOneWave) {
+                lds_sync<true>();
+                return __any(go) != 0;
+            } else {
+                return __syncthreads_or(go) != 0;
+            }
+        };
+        while (any_go()) {
             double dlt[3] = {0.0, 0.0, 0.0}, nf[3] = {0.0, 0.0, 0.0};
             bool ok = true;
             if (go) {
-                const double dot = (xt[0] * e[0] + xt[1] * e[1] + xt[2] * e[2]) * k;
-                h[0] = dot * e[0];
-                h[1] = dot * e[1];
-                h[2] = dot * e[2] + happ_mid;
-                if (ia.interactions) {
-                    dipolar_field<double, 1>(pos, mb, tid, cb, ce, 0, hd[0], hd[1], hd[2]);
-                    h[0] = h[0] + hd[0];
-                    h[1] = h[1] + hd[1];
-                    h[2] = h[2] + hd[2];
-                }
-                drift3(xt, al, h, dr);
-                diffusion3(xt, sr, al, B);
-                double J[9], jb[27], F[3];
-                drift_jac3(xt, al, h, hj, J);
-                diffusion_jac3(xt, sr, al, jb);
+                field(y, happ_mid, h);
+                NewtonSystem ns = midpoint_system(y, x0, h, sw, dt, al, c_half, e0);
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    F[i] = xt[i] - 0.5 * dr[i] * dt - x0[i];
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) F[i] -= 0.5 * B[i * 3 + j] * dwm[j];
-                }
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        double v = (double)(i == j) - 0.5 * J[i * 3 + j];
-#pragma unroll
-                        for (int kk = 0; kk < 3; ++kk) v -= 0.5 * jb[i * 9 + kk * 3 + j] * dwm[kk];
-                        J[i * 3 + j] = v;
-                    }
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    dlt[i] = -F[i];
-                    nf[i] = -F[i];
-                }
+                for (int i = 0; i < 3; ++i) nf[i] = ns.f[i];
                 ++iters;
-                ok = solve3(J, dlt);
+                ok = newton_solve(ns);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) dlt[i] = ns.f[i];
             }
-            __syncthreads();   // the iterates' field and the last norm are read
-            if (go) red[tid] = Vec4<double>{dlt[0], dlt[1], dlt[2], ok ? 0.0 : 1.0};
-            __syncthreads();
+            lds_sync<kOneWave>();   // the iterates' field and the last norm are read
             if (go) {
-                double s2 = 0.0;
-                bool sing = false;
-                for (int j = cb; j < ce; ++j) {
-                    const Vec4<double> v = red[j];
-                    s2 += v.x * v.x;
-                    s2 += v.y * v.y;
-                    s2 += v.z * v.z;
-                    sing = sing || v.w != 0.0;
-                }
-                if (sing) {   // LAPACK_ERR: x_root left at -F
+                red[tid] = square(dlt);
+                if (!ok) sing[cb] = 1;
+            }
+            lds_sync<kOneWave>();
+            if (go) {
+                if (sing[cb] != 0) {   // LAPACK_ERR: x_root left at -F
                     y[0] = nf[0]; y[1] = nf[1]; y[2] = nf[2];
                     singular = true;
                     go = false;
                 } else {
-                    err = sqrt(s2);
-                    y[0] = dlt[0] + xt[0];
-                    y[1] = dlt[1] + xt[1];
-                    y[2] = dlt[2] + xt[2];
+                    const bool over = cluster_sum() > tol2;   // |delta| > tol
+                    y[0] += dlt[0];
+                    y[1] += dlt[1];
+                    y[2] += dlt[2];
                     mb[tid] = Vec4<double>{y[0], y[1], y[2], 0.0};
-                    go = (err > tol) && (iter-- > 0);
+                    go = over && (iter-- > 0);
                 }
             }
         }
+        if (singular) sing[cb] = 0;   // its readers are past the loop's last barrier
         if (live && (singular || iter == -1)) ++fails;
 #pragma unroll
         for (int i = 0; i < 3; ++i) x0[i] = 2 * y[i] - x0[i];
