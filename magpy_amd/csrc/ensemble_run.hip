@@ -64,6 +64,15 @@ int64_t steps_per_launch(int scheme, int precision)
     return precision == MP_PRECISION_FP32 ? (1 << 17) : (1 << 16);
 }
 
+// compute units of the current device
+int device_cus()
+{
+    int dev = 0, cus = 0;
+    MP_HIP(hipGetDevice(&dev));
+    MP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return cus;
+}
+
 template <typename T>
 std::vector<T> cast_vec(const std::vector<double> &v)
 {
@@ -88,9 +97,7 @@ int two_wave_mode(int n_waves, bool fp32)
         const int v = std::atoi(env);
         return v <= 0 ? 0 : (v >= 2 && fp32) ? 2 : 1;
     }
-    int dev = 0, cus = 0;
-    MP_HIP(hipGetDevice(&dev));
-    MP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int cus = device_cus();
     if (!fp32) return n_waves <= 2 * cus ? 1 : 0;
     if (n_waves > 4 * cus) return 0;
     return n_waves > cus ? 2 : 1;
@@ -208,11 +215,18 @@ struct GroupBase {
 // Cluster packing: members of a group sorted by size (largest first), each
 // placed in the first block with room; a member never straddles blocks.
 // Returns slot -> particle (-1 padding), and per slot the block-relative
-// start lane of its member and the member size.
+// start lane of its member and the member size.  A member takes a multiple of
+// `align` slots: those past its size are its helpers (slot_particle -1, with the
+// member's start and size), so every member starts on a multiple of align.
+// Blocks come out largest member first.  The dispatcher deals workgroups round
+// the XCDs, their CUs and SIMDs, so those `run` apart share a SIMD; a
+// workgroup's time goes with its largest member, and every second run of blocks
+// is reversed so that a SIMD gets a long and a short one.
 void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int block,
-                   std::vector<int64_t> &slot_particle, std::vector<int> &cbase,
-                   std::vector<int> &csize)
+                   int align, size_t run, std::vector<int64_t> &slot_particle,
+                   std::vector<int> &cbase, std::vector<int> &csize)
 {
+    auto taken = [align](int size) { return (size + align - 1) / align * align; };
     std::vector<size_t> order(members.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
@@ -222,7 +236,7 @@ void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int 
     std::vector<std::vector<size_t>> content;    // members per block
     size_t first_open = 0;
     for (size_t oi : order) {
-        const int sz = (int)(members[oi].second - members[oi].first);
+        const int sz = taken((int)(members[oi].second - members[oi].first));
         size_t bi = first_open;
         while (bi < fill.size() && fill[bi] + sz > block) ++bi;
         if (bi == fill.size()) {
@@ -233,6 +247,9 @@ void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int 
         content[bi].push_back(oi);
         while (first_open < fill.size() && fill[first_open] == block) ++first_open;
     }
+    for (size_t b = run; b < content.size(); b += 2 * run)
+        std::reverse(content.begin() + (ptrdiff_t)b,
+                     content.begin() + (ptrdiff_t)std::min(content.size(), b + run));
     const size_t nslots = fill.size() * (size_t)block;
     slot_particle.assign(nslots, -1);
     cbase.assign(nslots, 0);
@@ -241,15 +258,23 @@ void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int 
         int lane = 0;
         for (size_t oi : content[bi]) {
             const int sz = (int)(members[oi].second - members[oi].first);
-            for (int j = 0; j < sz; ++j) {
+            for (int j = 0; j < taken(sz); ++j) {
                 const size_t slot = bi * (size_t)block + (size_t)(lane + j);
-                slot_particle[slot] = members[oi].first + j;
+                if (j < sz) slot_particle[slot] = members[oi].first + j;
                 cbase[slot] = lane;
                 csize[slot] = sz;
             }
-            lane += sz;
+            lane += taken(sz);
         }
     }
+}
+
+// Lanes of the implicit cluster kernel that share their pair sums (shared_field)
+int field_targets(const std::vector<std::pair<int64_t, int64_t>> &members)
+{
+    int64_t nmax = 1;
+    for (const auto &m : members) nmax = std::max(nmax, m.second - m.first);
+    return nmax > 8 ? 4 : 2;
 }
 
 template <typename T>
@@ -261,6 +286,7 @@ struct GroupRun : GroupBase {
     bool interactions = true;  // clusters: dipolar sums (the implicit scheme may run without)
     int two_wave = 0;          // Heun kernel: 0 one wave, 1/2 two waves (two_wave_mode)
     int lanes = 1;             // lanes per cluster slot (1 or 2)
+    int targets = 1;           // implicit clusters: lanes that share their pair sums
     int64_t S = 0, s_next = 0, spl = 1;
     std::vector<int64_t> sched, slot_particle;
     DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_mx, d_my, d_mz, d_samples;
@@ -308,7 +334,11 @@ struct GroupRun : GroupBase {
             }
             block = cluster_block;
             lanes = cluster_lanes;
-            pack_clusters(members, block / lanes, slot_particle, cbase, csize);
+            // workgroups that fill every SIMD once
+            const size_t run =
+                (size_t)std::max(1, 4 * device_cus() / ((block + mp::kWave - 1) / mp::kWave));
+            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT) targets = field_targets(members);
+            pack_clusters(members, block / lanes, targets, run, slot_particle, cbase, csize);
         } else {
             slot_particle.assign(plan.perm.begin() + b, plan.perm.begin() + e);
         }
@@ -484,23 +514,31 @@ struct GroupRun : GroupBase {
         mp::ImplicitClusterArgs ia{
             mp::ClusterArgs<double>{a, d_px.p, d_py.p, d_pz.p, d_w.p, d_cbase.p, d_csize.p}, eps,
             max_iter, d_it.p, d_fl.p, interactions ? 1 : 0};
-        // positions and iterates, then a square and a flag per slot
-        const size_t shmem =
-            (size_t)block * (2 * sizeof(mp::Vec4<double>) + sizeof(double) + sizeof(int));
+        // a source per slot, a sum per `targets` slots, a flag per slot
+        const size_t shmem = (size_t)block * (sizeof(mp::Source) + sizeof(int)) +
+                             (size_t)(block / targets) * sizeof(double);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), shmem, s, ia);
         };
-        auto shaped = [&](auto one_wave) {
+        auto shaped = [&](auto one_wave, auto kt) {
             constexpr bool W = decltype(one_wave)::value;
+            constexpr int KT = decltype(kt)::value;
             switch (shape_kind) {
-            case mp::kSine: go(mp::implicit_cluster_kernel<mp::kSine, kArray, W>); break;
-            case mp::kSquare: go(mp::implicit_cluster_kernel<mp::kSquare, kArray, W>); break;
-            case mp::kConstant: go(mp::implicit_cluster_kernel<mp::kConstant, kArray, W>); break;
-            default: go(mp::implicit_cluster_kernel<mp::kMixed, kArray, W>); break;
+            case mp::kSine: go(mp::implicit_cluster_kernel<mp::kSine, kArray, W, KT>); break;
+            case mp::kSquare: go(mp::implicit_cluster_kernel<mp::kSquare, kArray, W, KT>); break;
+            case mp::kConstant: go(mp::implicit_cluster_kernel<mp::kConstant, kArray, W, KT>); break;
+            default: go(mp::implicit_cluster_kernel<mp::kMixed, kArray, W, KT>); break;
             }
         };
-        if (block == mp::kWave) shaped(std::true_type{});
-        else shaped(std::false_type{});
+        using Two = std::integral_constant<int, 2>;
+        using Four = std::integral_constant<int, 4>;
+        if (block == mp::kWave) {
+            if (targets == 2) shaped(std::true_type{}, Two{});
+            else shaped(std::true_type{}, Four{});
+        } else {
+            if (targets == 2) shaped(std::false_type{}, Two{});
+            else shaped(std::false_type{}, Four{});
+        }
     }
 
     template <int L, bool kArray>
@@ -1139,9 +1177,7 @@ ClusterLayout cluster_layout(int64_t nmax, int64_t particles, ClusterLimits lim 
     } else if (const int forced = env_cluster_lanes()) {
         l.lanes = forced;
     } else {
-        int dev = 0, cus = 0;
-        MP_HIP(hipGetDevice(&dev));
-        MP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const int cus = device_cus();
         l.lanes = particles < (int64_t)kSplitBelowWavesPerCU * mp::kWave * cus ? 2 : 1;
     }
     if (cluster_min_block(nmax, l.lanes, lim.max_block) == 0) l.lanes = 1;

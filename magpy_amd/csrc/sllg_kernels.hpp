@@ -1161,27 +1161,44 @@ __device__ inline void midpoint_guess(const double *x0, const double *h, const d
     y[2] = 0.5 * (lz + x0[2]);
 }
 
-// Wiener normals of consecutive steps, one Philox call at a time
+// Wiener normals of consecutive steps n0, n0 + 1, ...: a step takes at most one
+// new Philox call.  The round keys are formed again at each call, so that they
+// hold no registers through the Newton iterations.
 struct StepNormals {
-    double z[4];
-    uint64_t have = UINT64_MAX;
-    __device__ inline void get(int64_t n, uint32_t pid, uint32_t tag, const PhiloxKeys &keys,
-                               double *w)
+    uint32_t key0, key1, pid, tag;
+    double z[4];   // the last call's normals
+
+    __device__ inline StepNormals(uint32_t k0, uint32_t k1, uint32_t particle, uint32_t t,
+                                  int64_t n0)
+        : key0(k0), key1(k1), pid(particle), tag(t)
     {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const uint64_t j = 3 * (uint64_t)n + d;
-            const uint64_t c = j >> 2;
-            if (c != have) {
-                const u32x4 r =
-                    philox4x32_10(u32x4{(uint32_t)c, (uint32_t)(c >> 32), pid, tag}, keys);
-                Num<double>::box_muller(r.x, r.y, z[0], z[1]);
-                Num<double>::box_muller(r.z, r.w, z[2], z[3]);
-                have = c;
-            }
-            const int jj = (int)(j & 3);
-            w[d] = jj == 0 ? z[0] : jj == 1 ? z[1] : jj == 2 ? z[2] : z[3];
+        call(3 * (uint64_t)n0 >> 2, z);
+    }
+    __device__ inline void call(uint64_t c, double *out) const
+    {
+        uint32_t a = key0, b = key1;
+        asm volatile("" : "+v"(a), "+v"(b));
+        PhiloxKeys keys;
+        keys.init(a, b);
+        const u32x4 r = philox4x32_10(u32x4{(uint32_t)c, (uint32_t)(c >> 32), pid, tag}, keys);
+        Num<double>::box_muller(r.x, r.y, out[0], out[1]);
+        Num<double>::box_muller(r.z, r.w, out[2], out[3]);
+    }
+    __device__ inline void get(int64_t n, double *w)
+    {
+        const uint64_t j = 3 * (uint64_t)n;
+        const int o = (int)(j & 3);   // the step's first normal is component o of its call
+        if (o == 1) {
+            w[0] = z[1]; w[1] = z[2]; w[2] = z[3];
+            return;
         }
+        double zn[4];
+        call((j + 2) >> 2, zn);
+        w[0] = o == 0 ? zn[0] : o == 2 ? z[2] : z[3];
+        w[1] = o == 0 ? zn[1] : o == 2 ? z[3] : zn[0];
+        w[2] = o == 0 ? zn[2] : o == 2 ? zn[0] : zn[1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[i] = zn[i];
     }
 };
 
@@ -1200,9 +1217,7 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
     const double fred = a.fred[q];
     const int shape = a.shape[q];
     const double msw = a.msw[q];
-    PhiloxKeys keys;
-    keys.init(a.key0[q], a.key1[q]);
-    const uint32_t pid = a.pid[q];
+    StepNormals normals(a.key0[q], a.key1[q], a.pid[q], a.tag, a.n0);
     const double ah = sqrt(2 * 1000.0 * fabs(log(dt)));
     const double sdt = sqrt(dt);
     // half the field Jacobian k e e^T (lib/field.cpp:159-174) as c e^T
@@ -1211,7 +1226,6 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
     unsigned long long iters = 0, fails = 0;
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
-    StepNormals normals;
 
     for (int64_t n = a.n0; n < a.n1; ++n) {
         double w[3];
@@ -1219,7 +1233,7 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
             const double *src = a.noise + ((size_t)n * (size_t)a.n + (size_t)q) * 3;
             w[0] = src[0]; w[1] = src[1]; w[2] = src[2];
         } else {
-            normals.get(n, pid, a.tag, keys, w);
+            normals.get(n, w);
         }
         const double t = (double)(n + 1) * dt;
         double sw[3];
@@ -1316,6 +1330,120 @@ struct ImplicitClusterArgs {
 
 constexpr int kImplicitClusterBlock = 256;   // largest workgroup, so largest cluster
 
+// The dipolar field of kT = 2 or 4 particles at once.  kT neighbouring lanes of a
+// cluster (which starts on a multiple of kT; past its size come helper lanes
+// without a particle) share their pair sums: lane q sums the sources at offsets
+// congruent to q for all kT particles, and the lanes exchange the sums that are
+// the others'.  A source read from LDS then serves kT pair terms, which are
+// independent work.  A source was two 32-byte vectors per term; it is 48 bytes
+// for kT terms.  Bound: FP64 issue, ~33 instructions per term, under the card's
+// power limit (2.1 GHz).  kT = 4 is the faster from 9 particles up; in smaller
+// clusters helper lanes and idle residues cost more than the reads (us per
+// iteration, kT 2 / 4: 65,536 dimers 1.64 / 3.5, 8,192 of 8 2.18 / 2.20, 2,048
+// of 64 13.4 / 13.0).  4,096 clusters of 2 to 64, 32 steps, on a warm card:
+// 11.4 -> 10.65 ms a pass; one dimer, 1,000 steps: 24.6 -> 21.0 ms.
+struct Source {
+    double px, py, pz, mx, my, mz;   // position, w m
+};
+
+// One term of the field at (x, y, z): M / r^3 (3 (u.n) n - u), M = |w m|
+__device__ inline void source_term(double x, double y, double z, const Source &q, bool skip,
+                                   double *h)
+{
+#pragma clang fp contract(off)
+    const double dx = q.px - x, dy = q.py - y, dz = q.pz - z;
+    const double r2 = skip ? 1.0 : fmad(dx, dx, fmad(dy, dy, dz * dz));
+    const double rinv = rsqrt_normal(r2);
+    const double rinv2 = rinv * rinv;
+    const double c = skip ? 0.0 : rinv2 * rinv;
+    const double t = 3.0 * fmad(q.mx, dx, fmad(q.my, dy, q.mz * dz)) * rinv2;
+    h[0] = fmad(c, fmad(t, dx, -q.mx), h[0]);
+    h[1] = fmad(c, fmad(t, dy, -q.my), h[1]);
+    h[2] = fmad(c, fmad(t, dz, -q.mz), h[2]);
+}
+
+// the value of lane ^ kXor, kXor = 1, 2 or 3
+template <int kXor>
+__device__ inline double swap_lanes(double v)
+{
+    constexpr int kPerm = kXor == 1 ? 0xb1 : kXor == 2 ? 0x4e : 0x1b;   // quad_perm
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), kPerm, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), kPerm, 0xf, 0xf, true));
+}
+
+// A particle's place and those of the lanes ^ 1, ^ 2, ^ 3
+template <int kT>
+struct Places {
+    double x[kT][3];
+    __device__ inline explicit Places(const double *own)
+    {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            x[0][d] = own[d];
+            x[1][d] = swap_lanes<1>(own[d]);
+            if constexpr (kT == 4) {
+                x[2][d] = swap_lanes<2>(own[d]);
+                x[3][d] = swap_lanes<3>(own[d]);
+            }
+        }
+    }
+};
+
+// Adds to h the field at the calling lane's particle from the sources [b, e) of
+// its cluster.  All lanes of a cluster call it together.  The sum is taken as
+// (r0 + r1) + (r2 + r3) with r the sums over the sources at offsets congruent
+// mod 4, for either kT, so that a member's result does not depend on the rest of
+// the ensemble.
+template <int kT>
+__device__ inline void shared_field(const Source *src, int tid, int b, int e, const Places<kT> &at,
+                                    double *h)
+{
+    // s[t]: particle t's sum over this lane's sources; kT = 2 keeps those at
+    // offsets congruent mod 4 apart, in s[t] and s[2 + t]
+    double s[4][3];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) s[t][d] = 0.0;
+    auto term = [&](const Source &q, int t, bool skip, double *sum) {
+        source_term(at.x[t][0], at.x[t][1], at.x[t][2], q, skip, sum);
+    };
+    int j = b + (tid & (kT - 1));
+    if constexpr (kT == 4) {
+        for (; j < e; j += 4) {
+            const Source q = src[j];
+            term(q, 0, j == tid, s[0]);
+#pragma unroll
+            for (int t = 1; t < 4; ++t) term(q, t, false, s[t]);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            h[d] += (s[0][d] + swap_lanes<1>(s[1][d])) +
+                    (swap_lanes<2>(s[2][d]) + swap_lanes<3>(s[3][d]));
+    } else {
+        for (; j + 2 < e; j += 4) {
+            const Source q0 = src[j], q1 = src[j + 2];
+            term(q0, 0, j == tid, s[0]);
+            term(q0, 1, false, s[1]);
+            term(q1, 0, j + 2 == tid, s[2]);
+            term(q1, 1, false, s[3]);
+        }
+        if (j < e) {
+            const Source q = src[j];
+            term(q, 1, false, s[1]);
+            if (j != tid) term(q, 0, false, s[0]);   // a dimer's lanes skip their own particle
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) s[0][d] += swap_lanes<1>(s[1][d]);
+        if (e - b > 2) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) s[0][d] += s[2][d] + swap_lanes<1>(s[3][d]);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) h[d] += s[0][d];
+    }
+}
+
 // Order LDS accesses of the workgroup: a barrier, or, where the workgroup is one
 // wave (whose LDS accesses complete in order), only the compiler's order.
 template <bool kOneWave>
@@ -1331,25 +1459,27 @@ __device__ inline void lds_sync()
 }
 
 // kOneWave: the workgroup is one wave (clusters of at most 64 particles), so
-// an iteration needs no barrier.
-template <int kShape, bool kArrayNoise, bool kOneWave>
-__global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void implicit_cluster_kernel(
+// an iteration needs no barrier.  Held to the registers of three waves per SIMD:
+// 4,096 clusters of 2 to 64 are 2,124 one-wave workgroups, which two per SIMD
+// leave in a second, nearly empty round (11.35 against 10.85 ms a pass).
+template <int kShape, bool kArrayNoise, bool kOneWave, int kT>
+__global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock, 3) void implicit_cluster_kernel(
     ImplicitClusterArgs ia)
 {
     const ClusterArgs<double> &ca = ia.c;
     const IndepArgs<double> &a = ca.base;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int slots = blockDim.x;
-    Vec4<double> *pos = reinterpret_cast<Vec4<double> *>(smem_raw);
-    Vec4<double> *mb = pos + slots;    // the states the field is taken from
-    double *red = reinterpret_cast<double *>(mb + slots);  // squares whose cluster sum is taken
-    int *sing = reinterpret_cast<int *>(red + slots);      // a cluster's first slot: singular block
+    Source *src = reinterpret_cast<Source *>(smem_raw);     // the states the field is taken from
+    double *red = reinterpret_cast<double *>(src + slots);  // sums of kT lanes' squares
+    int *sing = reinterpret_cast<int *>(red + slots / kT);  // a cluster's first slot: singular block
 
     const int tid = threadIdx.x;
     const int p = blockIdx.x * slots + tid;   // the grid covers all slots exactly
+    // padding: cn = 0; a helper lane: past the end of its cluster
     const int cn = ca.csize[p];
-    const bool live = cn > 0;
-    const int cb = live ? ca.cbase[p] : tid, ce = live ? cb + cn : tid;
+    const int cb = cn > 0 ? ca.cbase[p] : tid, ce = cb + cn;
+    const bool live = tid < ce;
     const bool leader = live && tid == cb;
 
     double x0[3] = {a.mx[p], a.my[p], a.mz[p]};
@@ -1358,12 +1488,20 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
     const double sr = a.sr[p], fred = a.fred[p];
     const int shape = a.shape[p];
     const double msw = a.msw[p];
-    PhiloxKeys keys;
-    keys.init(a.key0[p], a.key1[p]);
-    const uint32_t pid = a.pid[p];
+    StepNormals normals(a.key0[p], a.key1[p], a.pid[p], a.tag, a.n0);
     const double ah = sqrt(2 * 1000.0 * fabs(log(dt)));
     const double sdt = sqrt(dt);
-    pos[tid] = Vec4<double>{ca.px[p], ca.py[p], ca.pz[p], ca.w[p]};
+    // (a helper's place: away from any particle, so that its unused sums are finite)
+    const double own[3] = {live ? ca.px[p] : 1e9, ca.py[p], ca.pz[p]}, wt = ca.w[p];
+    const Places<kT> at(own);
+    src[tid].px = own[0];
+    src[tid].py = own[1];
+    src[tid].pz = own[2];
+    auto publish = [&](const double *m) {
+        src[tid].mx = wt * m[0];
+        src[tid].my = wt * m[1];
+        src[tid].mz = wt * m[2];
+    };
     sing[tid] = 0;
 
     // hj + 3n of the 3N x 3N field Jacobian J[i][j] = k_{i/3} e[i] e[j] for
@@ -1391,32 +1529,37 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
     unsigned long long iters = 0, fails = 0;
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
-    StepNormals normals;
 
-    // the sum of red over the cluster's slots, as two sums added at the end
-    auto cluster_sum = [&]() {
-        double s0 = 0.0, s1 = 0.0;
-        int j = cb;
-        for (; j + 4 <= ce; j += 4) {
-            s0 += red[j];
-            s1 += red[j + 1];
-            s0 += red[j + 2];
-            s1 += red[j + 3];
-        }
-        for (; j < ce; ++j) s0 += red[j];
-        return s0 + s1;
+    // The sum over the cluster of |v|^2: kT lanes add theirs by lane swaps and
+    // the first stores the sum (put_square), then every lane adds the cluster's
+    // sums (cluster_sum): up to 64 of four lanes each, eight LDS reads in flight,
+    // or the few of two.
+    auto put_square = [&](const double *v) {
+        double q = live ? fmad(v[0], v[0], fmad(v[1], v[1], v[2] * v[2])) : 0.0;
+        q += swap_lanes<1>(q);
+        if constexpr (kT == 4) q += swap_lanes<2>(q);
+        if ((tid & (kT - 1)) == 0) red[tid / kT] = q;
     };
-    auto square = [](const double *v) { return fmad(v[0], v[0], fmad(v[1], v[1], v[2] * v[2])); };
-    // the field of the state m, the dipolar sum of the states in mb added
+    auto cluster_sum = [&]() {
+        double sum = 0.0;
+        if constexpr (kT == 2) {
+            for (int k = cb; k < ce; k += 2) sum += red[k / 2];
+            return sum;
+        }
+        for (int k = cb; k < ce; k += 8 * kT) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = red[(k + u * kT < ce ? k + u * kT : cb) / kT];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = k + u * kT < ce ? v[u] : 0.0;
+            sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        }
+        return sum;
+    };
+    // the field of the state m, the dipolar sum of the published states added
     auto field = [&](const double *m, double applied, double *h) {
         single_field(m, e, k, applied, h);
-        if (ia.interactions) {
-            double d[3];
-            dipolar_field<double, 1>(pos, mb, tid, cb, ce, 0, d[0], d[1], d[2]);
-            h[0] += d[0];
-            h[1] += d[1];
-            h[2] += d[2];
-        }
+        if (ia.interactions) shared_field<kT>(src, tid, cb, ce, at, h);
     };
 
     for (int64_t n = a.n0; n < a.n1; ++n) {
@@ -1425,7 +1568,7 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
             const double *src = a.noise + ((size_t)n * (size_t)a.n + (size_t)p) * 3;
             w[0] = src[0]; w[1] = src[1]; w[2] = src[2];
         } else {
-            normals.get(n, pid, a.tag, keys, w);
+            normals.get(n, w);
         }
         const double t = (double)(n + 1) * dt;
         double sw[3];
@@ -1433,20 +1576,21 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
         for (int d = 0; d < 3; ++d) sw[d] = sr * (fmax(-ah, fmin(ah, w[d])) * sdt);
 
         // Euler guess, the field including the cluster's dipolar sum at x0
-        mb[tid] = Vec4<double>{x0[0], x0[1], x0[2], 0.0};
+        publish(x0);
         lds_sync<kOneWave>();
         double h[3], y[3];
         field(x0, Applied<double, kShape>::at(shape, amp, fred, t), h);
         midpoint_guess(x0, h, sw, dt, al, y);
-        red[tid] = square(y);
-        lds_sync<kOneWave>();   // every lane's guess field is taken: mb may change
+        put_square(y);
+        lds_sync<kOneWave>();   // every lane's guess field is taken
         const double tol = ia.eps * sqrt(cluster_sum());
         const double tol2 = tol * tol;
-        mb[tid] = Vec4<double>{y[0], y[1], y[2], 0.0};
+        publish(y);
         const double happ_mid = Applied<double, kShape>::at(shape, amp, fred, t + dt / 2);
         int iter = ia.max_iter;
         bool singular = false;
-        bool go = live && (2 * tol > tol) && (iter-- > 0);
+        // a helper lane goes with its cluster (it sums for its neighbour)
+        bool go = cn > 0 && (2 * tol > tol) && (iter-- > 0);
         auto any_go = [&]() {
             if constexpr (kOneWave) {
                 lds_sync<true>();
@@ -1470,8 +1614,8 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
             }
             lds_sync<kOneWave>();   // the iterates' field and the last norm are read
             if (go) {
-                red[tid] = square(dlt);
-                if (!ok) sing[cb] = 1;
+                put_square(dlt);
+                if (live && !ok) sing[cb] = 1;
             }
             lds_sync<kOneWave>();
             if (go) {
@@ -1484,7 +1628,7 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock) void impl
                     y[0] += dlt[0];
                     y[1] += dlt[1];
                     y[2] += dlt[2];
-                    mb[tid] = Vec4<double>{y[0], y[1], y[2], 0.0};
+                    publish(y);
                     go = over && (iter-- > 0);
                 }
             }
