@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <limits>
 #include <map>
 #include <memory>
@@ -183,6 +184,7 @@ struct Plan {
     std::vector<std::vector<int64_t>> sched; // per group
     std::vector<int64_t> group_steps;        // per group
     std::vector<int64_t> member_of;          // per original particle
+    std::vector<int> group_of;               // per member
     std::vector<simulation::ReducedMember> red;
 };
 
@@ -193,9 +195,12 @@ struct HostCopy {
     std::vector<int32_t> shape;
 };
 
-// Results of one group copied back to the host, per slot.
+// Results of one launch set copied back to the host, per slot.  Samples and sums
+// of a group taken at or before the run's start step are not recorded (their
+// entries are unspecified or zero).
 struct GroupOut {
     std::vector<int64_t> particle_of; // slot -> particle (-1 = padding)
+    std::vector<int> group_of;        // slot -> schedule group
     std::vector<double> state;        // [slots][3]
     std::vector<uint32_t> status;
     std::vector<double> samples;      // [S][3][slots] (empty when not recorded)
@@ -209,6 +214,7 @@ struct GroupBase {
     virtual void enqueue(int64_t upto, hipStream_t s) = 0;
     virtual void state(std::vector<double> &out) = 0;  // [slots][3]
     virtual const std::vector<int64_t> &slots() const = 0;
+    virtual const std::vector<int> &set() const = 0;   // its schedule groups
     virtual GroupOut collect(hipStream_t s) = 0;
 };
 
@@ -277,6 +283,114 @@ int field_targets(const std::vector<std::pair<int64_t, int64_t>> &members)
     return nmax > 8 ? 4 : 2;
 }
 
+// The applied field of a schedule group: whether all of its particles see the
+// same one (shape, reduced amplitude, cycles per step), and which.
+struct GroupField {
+    bool uniform = true;
+    int shape = 0;
+    double amp = 0.0, fdt = 0.0;
+};
+
+GroupField group_field(const simulation::EnsembleSpec &sp, const Plan &plan, int gi)
+{
+    GroupField f;
+    bool first = true;
+    for (int64_t i = plan.group_begin[(size_t)gi]; i < plan.group_begin[(size_t)gi + 1]; ++i) {
+        const int64_t m = plan.member_of[(size_t)plan.perm[(size_t)i]];
+        const simulation::ReducedMember &r = plan.red[(size_t)m];
+        const GroupField x{true, sp.field_shape[m], r.happ, r.fapp * r.dt};
+        if (first) f = x;
+        else if (x.shape != f.shape || x.amp != f.amp || x.fdt != f.fdt) f.uniform = false;
+        first = false;
+    }
+    return f;
+}
+
+// The sample steps a launch set records and, with several groups in it, which
+// record each group's samples are.
+std::vector<int64_t> union_schedule(const Plan &plan, const std::vector<int> &set, int64_t start,
+                                    std::vector<std::vector<int32_t>> &pick)
+{
+    pick.clear();
+    if (set.size() == 1) return plan.sched[(size_t)set[0]];
+    std::vector<int64_t> u;
+    for (int gi : set)
+        for (int64_t k : plan.sched[(size_t)gi])
+            if (k > start) u.push_back(k);
+    std::sort(u.begin(), u.end());
+    u.erase(std::unique(u.begin(), u.end()), u.end());
+    for (int gi : set) {
+        std::vector<int32_t> row;
+        for (int64_t k : plan.sched[(size_t)gi])
+            row.push_back(k > start ? (int32_t)(std::lower_bound(u.begin(), u.end(), k) - u.begin())
+                                    : -1);
+        pick.push_back(std::move(row));
+    }
+    return u;
+}
+
+// Which schedule groups share a launch.  An ensemble whose members differ in
+// anisotropy or damping has a reduced step per member, and where sample times
+// fall on step boundaries the rounding of each decides its sample steps, so it
+// can have a schedule group per member: one launch of one particle after the
+// other (300 members, 2,000 FP64 steps: 178 ms).  A launch set records the union
+// of its groups' sample steps, which differ by a step here and there, and each
+// member's samples are picked from it.  Sets hold groups of equal step count whose
+// kernels run the same code for them: FP64 and the implicit scheme, whose lanes
+// all evaluate their own field; FP32 constant fields; and FP32 groups of
+// independent particles that read their field from a table, as many rows of it.
+// Not in a set: schedules too unlike (records beyond three times the samples),
+// more than 1 GiB of records (the set is cut there), FP32 groups with per-lane
+// fields, and runs in caller-bounded memory.
+std::vector<std::vector<int>> launch_sets(const simulation::EnsembleSpec &sp, const Plan &plan,
+                                          bool clusters, bool bounded_memory)
+{
+    const int G = (int)plan.sched.size();
+    std::vector<std::vector<int>> sets;
+    const bool fp32 = sp.precision == MP_PRECISION_FP32 && sp.scheme == MP_SCHEME_HEUN;
+    std::map<std::pair<int, int64_t>, std::vector<int>> alike;   // (kind, steps) -> groups
+    for (int g = 0; g < G; ++g) {
+        int kind = 0;
+        if (fp32) {
+            const GroupField f = group_field(sp, plan, g);
+            kind = !f.uniform ? -1 : f.shape == MP_FIELD_CONSTANT ? 1 : clusters ? -1 : 2;
+            if (sp.noise == MP_NOISE_ARRAY) kind = kind == 2 ? -1 : kind;
+        }
+        if (bounded_memory || G == 1) kind = -1;
+        if (kind < 0) sets.push_back({g});
+        else alike[{kind, plan.group_steps[(size_t)g]}].push_back(g);
+    }
+    const int64_t table_lanes = 4 * (int64_t)device_cus() * mp::kWave;  // two_wave_mode's bound
+    for (auto &[key, gs] : alike) {
+        const int64_t S = sp.max_samples, most = 3 * S + 8;
+        std::vector<int> cur;
+        std::vector<int64_t> steps;      // the records of cur
+        int64_t lanes = 0;
+        for (int g : gs) {
+            const int64_t len = plan.group_begin[(size_t)g + 1] - plan.group_begin[(size_t)g];
+            std::vector<int64_t> u;
+            std::set_union(steps.begin(), steps.end(), plan.sched[(size_t)g].begin(),
+                           plan.sched[(size_t)g].end(), std::back_inserter(u));
+            u.erase(std::unique(u.begin(), u.end()), u.end());
+            const bool fits = (int64_t)u.size() <= most &&
+                              (int64_t)u.size() * 3 * (lanes + len) * (fp32 ? 4 : 8) <= (1ll << 30) &&
+                              (key.first != 2 || lanes + len <= table_lanes);
+            if (!cur.empty() && !fits) {
+                sets.push_back(std::move(cur));
+                cur.clear();
+                u = plan.sched[(size_t)g];
+                lanes = 0;
+            }
+            cur.push_back(g);
+            steps = std::move(u);
+            lanes += len;
+        }
+        if (!cur.empty()) sets.push_back(std::move(cur));
+    }
+    std::sort(sets.begin(), sets.end());
+    return sets;
+}
+
 template <typename T>
 struct GroupRun : GroupBase {
     int n = 0, grid = 0, block = mp::kBlock, n_waves = 0, scheme = 0, shape_kind = -1;
@@ -287,8 +401,14 @@ struct GroupRun : GroupBase {
     int two_wave = 0;          // Heun kernel: 0 one wave, 1/2 two waves (two_wave_mode)
     int lanes = 1;             // lanes per cluster slot (1 or 2)
     int targets = 1;           // implicit clusters: lanes that share their pair sums
-    int64_t S = 0, s_next = 0, spl = 1;
+    // The schedule groups of this launch set.  With several, the kernels record
+    // the union of their sample steps (S of them, S_out samples per group) and
+    // pick[g][s] is the record of group g's sample s (-1: at or before the start).
+    std::vector<int> groups;
+    int64_t S = 0, S_out = 0, s_next = 0, spl = 1;
     std::vector<int64_t> sched, slot_particle;
+    std::vector<int> slot_group;              // index into groups (-1: padding)
+    std::vector<std::vector<int32_t>> pick;
     DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_mx, d_my, d_mz, d_samples;
     DevBuf<T> d_px, d_py, d_pz, d_w;
     DevBuf<double> d_fred, d_fdt, d_dtd, d_msw, d_noise, d_partial, d_ens;
@@ -296,23 +416,24 @@ struct GroupRun : GroupBase {
     DevBuf<uint32_t> d_key0, d_key1, d_pid, d_status;
     DevBuf<int64_t> d_sched;
     DevBuf<unsigned long long> d_it, d_fl;
-    DevBuf<float> d_htab;      // uniform applied field of one launch (FP32 Heun)
+    DevBuf<float> d_htab;      // applied field of one launch (FP32 Heun), a row per field
     bool uniform_field = false;
-    int field_shape0 = 0;
-    double happ0 = 0.0, fdt0 = 0.0;
+    DevBuf<int> d_field_shape;                // per row of d_htab
+    DevBuf<double> d_field_amp, d_field_fdt;
+    int64_t tab_stride = 0;
+    DevBuf<int64_t> d_toff;                   // per slot: start of its row (several rows)
+    DevBuf<int32_t> d_pick, d_slot_group;
     mp::IndepArgs<T> a{};
 
     // cluster_block == 0: one slot per particle of the group (independent
     // particles); otherwise members packed into blocks of cluster_block lanes,
     // cluster_lanes (1 or 2) lanes per slot.
-    GroupRun(const simulation::EnsembleSpec &sp, const Plan &plan, int gi, bool traj, bool ens,
-             int cluster_block, int cluster_lanes = 1)
+    GroupRun(const simulation::EnsembleSpec &sp, const Plan &plan, const std::vector<int> &set,
+             bool traj, bool ens, int cluster_block, int cluster_lanes = 1)
+        : groups(set)
     {
-        const int64_t b = plan.group_begin[(size_t)gi], e = plan.group_begin[(size_t)gi + 1];
         const int64_t P = sp.member_offsets[sp.n_members];
-        sched = plan.sched[(size_t)gi];
-        S = (int64_t)sched.size();
-        n_total = plan.group_steps[(size_t)gi];
+        n_total = plan.group_steps[(size_t)set[0]];
         scheme = sp.scheme;
         eps = sp.implicit_tol;
         max_iter = sp.implicit_max_iter > 0 ? sp.implicit_max_iter : 1000;
@@ -322,16 +443,21 @@ struct GroupRun : GroupBase {
         want_ens = ens;
         spl = steps_per_launch(sp.scheme, sp.precision);
         n_done = std::min(sp.start_step, n_total);
+        S_out = (int64_t)plan.sched[(size_t)set[0]].size();
+        sched = union_schedule(plan, set, n_done, pick);
+        S = (int64_t)sched.size();
         cluster = cluster_block > 0;
         std::vector<int> cbase, csize;
         if (cluster) {
             std::vector<std::pair<int64_t, int64_t>> members;  // particle ranges
-            for (int64_t i = b; i < e;) {
-                const int64_t m = plan.member_of[(size_t)plan.perm[(size_t)i]];
-                const int64_t len = sp.member_offsets[m + 1] - sp.member_offsets[m];
-                members.emplace_back(sp.member_offsets[m], sp.member_offsets[m] + len);
-                i += len;
-            }
+            for (int gi : set)
+                for (int64_t i = plan.group_begin[(size_t)gi];
+                     i < plan.group_begin[(size_t)gi + 1];) {
+                    const int64_t m = plan.member_of[(size_t)plan.perm[(size_t)i]];
+                    const int64_t len = sp.member_offsets[m + 1] - sp.member_offsets[m];
+                    members.emplace_back(sp.member_offsets[m], sp.member_offsets[m] + len);
+                    i += len;
+                }
             block = cluster_block;
             lanes = cluster_lanes;
             // workgroups that fill every SIMD once
@@ -340,9 +466,18 @@ struct GroupRun : GroupBase {
             if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT) targets = field_targets(members);
             pack_clusters(members, block / lanes, targets, run, slot_particle, cbase, csize);
         } else {
-            slot_particle.assign(plan.perm.begin() + b, plan.perm.begin() + e);
+            for (int gi : set)
+                slot_particle.insert(slot_particle.end(),
+                                     plan.perm.begin() + plan.group_begin[(size_t)gi],
+                                     plan.perm.begin() + plan.group_begin[(size_t)gi + 1]);
         }
         n = (int)slot_particle.size();
+        slot_group.assign((size_t)n, -1);
+        for (int i = 0; i < n; ++i) {
+            if (slot_particle[(size_t)i] < 0) continue;
+            const int g = plan.group_of[(size_t)plan.member_of[(size_t)slot_particle[(size_t)i]]];
+            slot_group[(size_t)i] = (int)(std::lower_bound(set.begin(), set.end(), g) - set.begin());
+        }
 
         std::vector<double> ex(n, 0.0), ey(n, 0.0), ez(n, 1.0), k(n, 0.0), al(n, 0.0), dt(n, 0.0),
             sig(n, 0.0), sr(n, 0.0), happ(n, 0.0), fred(n, 0.0), fdt(n, 0.0), msw(n, 0.0),
@@ -388,23 +523,39 @@ struct GroupRun : GroupBase {
             }
             if (first) {
                 shape_kind = shape[i];
-                field_shape0 = shape[i];
-                happ0 = happ[i];
-                fdt0 = fdt[i];
                 first = false;
             } else if (shape_kind != shape[i]) {
                 shape_kind = (int)mp::kMixed;
             }
         }
-        // one shared field table when every particle sees the same applied field
+        // the applied field from a table, where every particle of a schedule group
+        // sees the same one (a constant needs none: its table is its amplitude)
         uniform_field = sizeof(T) == 4 && scheme == MP_SCHEME_HEUN && !first;
-        for (int i = 0; i < n && uniform_field; ++i)
-            if (slot_particle[(size_t)i] >= 0)
-                uniform_field = shape[i] == field_shape0 && happ[i] == happ0 && fdt[i] == fdt0;
+        for (int gi : set) uniform_field = uniform_field && group_field(sp, plan, gi).uniform;
+        if (set.size() > 1 && shape_kind == (int)mp::kConstant) uniform_field = false;
         if (uniform_field) {
             // groups of four aligned below n0, one entry past the last step, and
             // the next group's prefetch: 4 * groups + 5 <= spl + 12
-            d_htab.alloc((size_t)spl + 16);
+            if (set.size() > 1)   // at most 64 MB of rows, or rows of 4,096 steps
+                spl = std::min(spl, std::max((int64_t)4096, ((int64_t)1 << 24) / (int64_t)set.size()));
+            tab_stride = spl + 16;
+            std::vector<int> row_shape;
+            std::vector<double> row_amp, row_fdt;
+            for (int gi : set) {
+                const GroupField f = group_field(sp, plan, gi);
+                row_shape.push_back(f.shape);
+                row_amp.push_back(f.amp);
+                row_fdt.push_back(f.fdt);
+            }
+            d_field_shape.upload(row_shape);
+            d_field_amp.upload(row_amp);
+            d_field_fdt.upload(row_fdt);
+            d_htab.alloc((size_t)tab_stride * set.size());
+            if (set.size() > 1) {
+                std::vector<int64_t> toff((size_t)n, 0);
+                for (int i = 0; i < n; ++i) toff[(size_t)i] = tab_stride * slot_group[(size_t)i];
+                d_toff.upload(toff);
+            }
         }
         d_ex.upload(cast_vec<T>(ex));
         d_ey.upload(cast_vec<T>(ey));
@@ -441,15 +592,25 @@ struct GroupRun : GroupBase {
         // cluster slots come in whole blocks of block / lanes
         grid = cluster ? n / (block / lanes) : (n + block - 1) / block;
         n_waves = (grid * block) / mp::kWave;
+        const bool several = set.size() > 1;
         two_wave = !cluster && !array_noise && scheme == MP_SCHEME_HEUN
                        ? two_wave_mode(n_waves, sizeof(T) == 4)
                        : 0;
-        if (want_traj) d_samples.alloc((size_t)S * 3 * (size_t)n);
+        // the one-wave kernel reads one table row
+        if (several && uniform_field) two_wave = std::max(two_wave, 1);
+        if (want_traj || (several && want_ens)) d_samples.alloc((size_t)S * 3 * (size_t)n);
         if (want_ens) {
             // each recorded sample writes all of its (component, wave) slots;
-            // slots of samples taken at step 0 are replaced on the host
-            d_partial.alloc((size_t)S * 3 * (size_t)n_waves);
-            d_ens.alloc((size_t)S * 3);
+            // slots of samples taken at step 0 are replaced on the host.  Several
+            // schedules: the sums are taken from the samples
+            if (!several) d_partial.alloc((size_t)S * 3 * (size_t)n_waves);
+            d_ens.alloc((size_t)S_out * 3);
+            if (several) {
+                std::vector<int32_t> flat;
+                for (const auto &row : pick) flat.insert(flat.end(), row.begin(), row.end());
+                d_pick.upload(flat);
+                d_slot_group.upload(std::vector<int32_t>(slot_group.begin(), slot_group.end()));
+            }
         }
         if (array_noise) {
             std::vector<double> nz((size_t)n_total * (size_t)n * 3, 0.0);
@@ -474,14 +635,16 @@ struct GroupRun : GroupBase {
         a.status = d_status.p;
         a.sched = d_sched.p;
         a.S = S;
-        a.samples = want_traj ? d_samples.p : nullptr;
-        a.ens_partial = want_ens ? d_partial.p : nullptr;
+        a.samples = d_samples.p;
+        a.ens_partial = d_partial.p;
         a.tag = sp.noise_tag;
         a.renorm = sp.renorm ? 1 : 0;
         a.noise = array_noise ? d_noise.p : nullptr;
+        a.toff = d_toff.p;
     }
 
     const std::vector<int64_t> &slots() const override { return slot_particle; }
+    const std::vector<int> &set() const override { return groups; }
 
     void launch_cluster(hipStream_t s, const float *htab)
     {
@@ -610,10 +773,12 @@ struct GroupRun : GroupBase {
             if (uniform_field) {
                 const int64_t g0 = n_done >> 2, g1 = (n1 + 3) >> 2;
                 const int64_t count = 4 * (g1 - g0) + 5;
-                require((size_t)count <= d_htab.n, "field table too small");
-                hipLaunchKernelGGL(mp::field_table_kernel, dim3((unsigned)((count + 255) / 256)),
-                                   dim3(256), 0, s, field_shape0, happ0, fdt0, 4 * g0, count,
-                                   d_htab.p);
+                require(count <= tab_stride, "field table too small");
+                const int64_t per_row = (count + 255) / 256;
+                hipLaunchKernelGGL(mp::field_table_kernel,
+                                   dim3((unsigned)(per_row * (int64_t)groups.size())), dim3(256), 0,
+                                   s, d_field_shape.p, d_field_amp.p, d_field_fdt.p, 4 * g0, count,
+                                   (int)per_row, tab_stride, d_htab.p);
                 MP_HIP(hipGetLastError());
                 htab = d_htab.p;
             }
@@ -649,9 +814,19 @@ struct GroupRun : GroupBase {
     {
         GroupOut o;
         o.particle_of = slot_particle;
+        o.group_of.resize((size_t)n);
+        for (int i = 0; i < n; ++i)
+            o.group_of[(size_t)i] =
+                slot_group[(size_t)i] < 0 ? groups[0] : groups[(size_t)slot_group[(size_t)i]];
+        const bool several = groups.size() > 1;
         if (want_ens) {
-            hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
-                               s, d_partial.p, n_waves, S * 3, d_ens.p);
+            if (several)
+                hipLaunchKernelGGL(mp::ens_pick_kernel<T>, dim3((unsigned)(S_out * 3)),
+                                   dim3(mp::kBlock), 0, s, d_samples.p, d_pick.p, d_slot_group.p,
+                                   d_msw.p, n, (int)S_out, d_ens.p);
+            else
+                hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)),
+                                   dim3(mp::kBlock), 0, s, d_partial.p, n_waves, S * 3, d_ens.p);
             MP_HIP(hipGetLastError());
         }
         MP_HIP(hipStreamSynchronize(s));
@@ -669,10 +844,23 @@ struct GroupRun : GroupBase {
             std::vector<T> hs(d_samples.n);
             if (!hs.empty())
                 MP_HIP(hipMemcpy(hs.data(), d_samples.p, hs.size() * sizeof(T), hipMemcpyDeviceToHost));
-            o.samples.assign(hs.begin(), hs.end());
+            if (several) {
+                o.samples.resize((size_t)S_out * 3 * (size_t)n);
+                for (int64_t sa = 0; sa < S_out; ++sa)
+                    for (int d = 0; d < 3; ++d)
+                        for (int i = 0; i < n; ++i) {
+                            const int g = slot_group[(size_t)i];
+                            const int32_t u = g < 0 ? -1 : pick[(size_t)g][(size_t)sa];
+                            if (u >= 0)
+                                o.samples[((size_t)sa * 3 + d) * (size_t)n + (size_t)i] =
+                                    (double)hs[((size_t)u * 3 + d) * (size_t)n + (size_t)i];
+                        }
+            } else {
+                o.samples.assign(hs.begin(), hs.end());
+            }
         }
         if (want_ens) {
-            o.ens.resize((size_t)S * 3);
+            o.ens.resize((size_t)S_out * 3);
             MP_HIP(hipMemcpy(o.ens.data(), d_ens.p, o.ens.size() * sizeof(double),
                              hipMemcpyDeviceToHost));
         }
@@ -895,6 +1083,11 @@ struct ReplicaRun : GroupBase {
     }
 
     const std::vector<int64_t> &slots() const override { return slot_particle; }
+    const std::vector<int> &set() const override
+    {
+        static const std::vector<int> only{0};
+        return only;
+    }
 
     void enqueue(int64_t upto, hipStream_t s) override
     {
@@ -949,6 +1142,7 @@ struct ReplicaRun : GroupBase {
     {
         GroupOut o;
         o.particle_of = slot_particle;
+        o.group_of.assign(slot_particle.size(), 0);
         if (want_ens) {
             hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
                                s, d_partial.p, n_waves, S * 3, d_ens.p);
@@ -1224,9 +1418,9 @@ ClusterLayout autotune_cluster_layout(const simulation::EnsembleSpec &sp, const 
         for (int b = b0; b != 0 && b <= 1024; b *= 2) {
             std::unique_ptr<GroupBase> g;
             if (sp.precision == MP_PRECISION_FP32)
-                g.reset(new GroupRun<float>(sp, plan, 0, false, false, b, lanes));
+                g.reset(new GroupRun<float>(sp, plan, {0}, false, false, b, lanes));
             else
-                g.reset(new GroupRun<double>(sp, plan, 0, false, false, b, lanes));
+                g.reset(new GroupRun<double>(sp, plan, {0}, false, false, b, lanes));
             g->enqueue(g->n_done + 4, s);  // warm the code object
             MP_HIP(hipEventRecord(e0, s));
             g->enqueue(g->n_done + trial_steps, s);
@@ -1291,7 +1485,9 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     std::map<std::pair<double, double>, int> step_key;        // (dt, end) -> schedule
     std::vector<std::vector<int64_t>> scheds;                 // schedule + step count
     std::map<std::vector<int64_t>, int> sched_to_group;
-    std::vector<int> member_group((size_t)sp.n_members), group_sched;
+    std::vector<int> &member_group = plan.group_of;
+    std::vector<int> group_sched;
+    member_group.resize((size_t)sp.n_members);
     for (int64_t m = 0; m < sp.n_members; ++m) {
         const int64_t b = sp.member_offsets[m], e = sp.member_offsets[m + 1];
         plan.red.push_back(simulation::reduce_member(
@@ -1324,11 +1520,13 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     }
     const int G = (int)group_sched.size();
     plan.group_begin.assign((size_t)G + 1, 0);
+    std::vector<std::vector<int64_t>> group_members((size_t)G);
+    for (int64_t m = 0; m < sp.n_members; ++m)
+        group_members[(size_t)member_group[(size_t)m]].push_back(m);
     for (int g = 0; g < G; ++g) {
-        for (int64_t m = 0; m < sp.n_members; ++m)
-            if (member_group[(size_t)m] == g)
-                for (int64_t p = sp.member_offsets[m]; p < sp.member_offsets[m + 1]; ++p)
-                    plan.perm.push_back(p);
+        for (int64_t m : group_members[(size_t)g])
+            for (int64_t p = sp.member_offsets[m]; p < sp.member_offsets[m + 1]; ++p)
+                plan.perm.push_back(p);
         plan.group_begin[(size_t)g + 1] = (int64_t)plan.perm.size();
         std::vector<int64_t> k = scheds[(size_t)group_sched[(size_t)g]];
         const int64_t steps = k.back();
@@ -1393,13 +1591,13 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     ss->dipolar = cluster_block && sp.interactions ? MP_DIPOLAR_PAIRS : 0;
     ss->cluster_block = cluster_block;
     ss->cluster_lanes = cluster_block ? layout.lanes : 0;
-    for (int g = 0; g < G; ++g) {
+    for (const std::vector<int> &set : launch_sets(sp, plan, cluster_block != 0, in_arena)) {
         if (sp.precision == MP_PRECISION_FP32 && sp.scheme == MP_SCHEME_HEUN)
             ss->groups.emplace_back(
-                new GroupRun<float>(sp, plan, g, traj, ens, cluster_block, layout.lanes));
+                new GroupRun<float>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
         else
             ss->groups.emplace_back(
-                new GroupRun<double>(sp, plan, g, traj, ens, cluster_block, layout.lanes));
+                new GroupRun<double>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
     }
     return ss.release();
 }
@@ -1441,10 +1639,9 @@ void session_finish(mp_session *ss, mp_ensemble_out &out)
     if (want_traj) traj.assign((size_t)S * 3 * (size_t)P, 0.0);
     if (out.ens_m && ss->want_ens) ens.assign((size_t)S * 3, 0.0);
     int64_t newton_iters = 0, newton_fail = 0;
-    for (size_t gi = 0; gi < ss->groups.size(); ++gi) {
-        GroupOut o = ss->groups[gi]->collect(ss->sg.s);
+    for (auto &run : ss->groups) {
+        GroupOut o = run->collect(ss->sg.s);
         const int n = (int)o.particle_of.size();
-        const std::vector<int64_t> &sched = plan.sched[gi];
         for (int i = 0; i < n; ++i) {
             const int64_t p = o.particle_of[(size_t)i];
             if (p < 0) continue;
@@ -1461,29 +1658,38 @@ void session_finish(mp_session *ss, mp_ensemble_out &out)
                 for (int i = 0; i < n; ++i) {
                     const int64_t p = o.particle_of[(size_t)i];
                     if (p < 0) continue;
+                    const int64_t k = plan.sched[(size_t)o.group_of[(size_t)i]][(size_t)s];
                     for (int d = 0; d < 3; ++d)
                         traj[((size_t)s * 3 + d) * (size_t)P + (size_t)p] =
-                            sched[(size_t)s] < h.start ? nan
-                            : sched[(size_t)s] == h.start
+                            k < h.start ? nan
+                            : k == h.start
                                 ? h.m0[(size_t)p * 3 + d]
                                 : o.samples[((size_t)s * 3 + d) * (size_t)n + (size_t)i];
                 }
         if (!ens.empty())
-            for (int64_t s = 0; s < S; ++s)
-                for (int d = 0; d < 3; ++d) {
-                    double v = o.ens[(size_t)s * 3 + d];
-                    if (sched[(size_t)s] < h.start) {
-                        v = nan;
-                    } else if (sched[(size_t)s] == h.start) {
-                        v = 0.0;
-                        for (int i = 0; i < n; ++i) {
-                            const int64_t p = o.particle_of[(size_t)i];
-                            if (p < 0) continue;
-                            v += h.m0[(size_t)p * 3 + d] * h.ms[(size_t)plan.member_of[(size_t)p]];
-                        }
-                    }
-                    ens[(size_t)s * 3 + d] += v;
+            for (int64_t s = 0; s < S; ++s) {
+                // what the set's groups recorded of sample s, and the start states
+                // of those that took it at the start step
+                bool known = true, all = true;
+                double v[3] = {0.0, 0.0, 0.0};
+                for (int gi : run->set()) {
+                    const int64_t k = plan.sched[(size_t)gi][(size_t)s];
+                    known = known && k >= h.start;
+                    all = all && k > h.start;
                 }
+                if (known && !all)
+                    for (int i = 0; i < n; ++i) {
+                        const int64_t p = o.particle_of[(size_t)i];
+                        if (p < 0 || plan.sched[(size_t)o.group_of[(size_t)i]][(size_t)s] > h.start)
+                            continue;
+                        const double w = h.ms[(size_t)plan.member_of[(size_t)p]];
+                        for (int d = 0; d < 3; ++d) v[d] += h.m0[(size_t)p * 3 + d] * w;
+                    }
+                const bool recorded = all || run->set().size() > 1;
+                for (int d = 0; d < 3; ++d)
+                    ens[(size_t)s * 3 + d] +=
+                        !known ? nan : v[d] + (recorded ? o.ens[(size_t)s * 3 + d] : 0.0);
+            }
     }
 
     // ---- results in SI units (lib/simulation.cpp:610-621)

@@ -104,6 +104,7 @@ struct Applied<double, kShape> {
     static __device__ inline double second(int shape, double amp, double f, double dt, double n,
                                            double t1)
     {
+#pragma clang fp contract(off)
         const int s = kShape == kMixed ? shape : kShape;
         return at(shape, amp, f, s == kSine ? (n + 2.0) * dt : t1 + dt);
     }
@@ -173,6 +174,7 @@ struct IndepArgs {
     uint32_t tag;
     int renorm;
     const double *noise;    // [steps][n][3] (array noise) or null
+    const int64_t *toff;    // start of the particle's field-table row, or null (one row)
 };
 
 template <typename T>
@@ -492,6 +494,10 @@ __global__ __launch_bounds__((1 + kProducers) * kWave) void heun_indep_pc_kernel
     const T k = a.k[q], al = a.alpha[q], dt = a.dt[q];
     const T kex = k * ex, key = k * ey, kez = k * ez, edx = ex * dt, edy = ey * dt, edz = ez * dt;
     const double msw = a.msw[q];
+    const float *row = htab;   // the particle's field table
+    if constexpr (kTable) {
+        if (a.toff != nullptr) row += a.toff[q];
+    }
     const float cbm = Num<float>::kRadius2 * (float)(sig * sig);   // FP32 Box-Muller radius scale
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
@@ -560,7 +566,7 @@ __global__ __launch_bounds__((1 + kProducers) * kWave) void heun_indep_pc_kernel
                 for (int i = 0; i < 12; ++i) zz[i] = half[kk][i][lane];
                 if constexpr (kTable) {
                     const int64_t gt = gc + kk < g_end ? gc + kk : g_end - 1;
-                    const float *tg = htab + 4 * (gt - g_begin);
+                    const float *tg = row + 4 * (gt - g_begin);
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         hh1[u] = tg[u];
@@ -650,19 +656,23 @@ __global__ __launch_bounds__((1 + kProducers) * kWave) void heun_indep_pc_kernel
     }
 }
 
-// Applied field of a uniform launch: out[i] = h(t_{base+1+i}), i < count,
-// evaluated in FP64 from the cycle count c = f_red t reduced to [0,1).
-static __global__ void field_table_kernel(int shape, double amp, double fdt, int64_t base, int64_t count,
-                                   float *out)
+// Applied field tables of a launch, one row per field: out[row * stride + i] =
+// h(t_{base+1+i}), i < count, evaluated in FP64 from the cycle count c = f_red t
+// reduced to [0,1).  per_row workgroups fill a row.
+static __global__ void field_table_kernel(const int *shape, const double *amp, const double *fdt,
+                                          int64_t base, int64_t count, int per_row, int64_t stride,
+                                          float *out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int row = blockIdx.x / per_row;
+    const int64_t i = (int64_t)(blockIdx.x % per_row) * blockDim.x + threadIdx.x;
     if (i >= count) return;
-    const double c = (double)(base + 1 + i) * fdt;
+    const double c = (double)(base + 1 + i) * fdt[row];
     const double fr = c - floor(c);
-    double h = amp;
-    if (shape == kSine) h = amp * sinpi(2.0 * fr);
-    else if (shape == kSquare) h = fr >= 0.5 ? -amp : amp;
-    out[i] = (float)h;
+    const double a = amp[row];
+    double h = a;
+    if (shape[row] == kSine) h = a * sinpi(2.0 * fr);
+    else if (shape[row] == kSquare) h = fr >= 0.5 ? -a : a;
+    out[row * stride + i] = (float)h;
 }
 
 // ------------------------------------------------------------------ interacting clusters
@@ -1679,6 +1689,33 @@ static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int
         __syncthreads();
     }
     if (threadIdx.x == 0) out[r] = buf[0];
+}
+
+// Ensemble sums of a launch set of several schedules: out[s][c] = sum over slots
+// of Ms m, each slot's sample s being record pick[group][s] (-1: none), in a
+// fixed order.  Bound by the read of the records once.
+template <typename T>
+static __global__ __launch_bounds__(kBlock) void ens_pick_kernel(const T *samples,
+                                                                 const int32_t *pick,
+                                                                 const int32_t *slot_group,
+                                                                 const double *msw, int n, int S,
+                                                                 double *out)
+{
+    const int s = blockIdx.x / 3, c = blockIdx.x % 3;
+    __shared__ double buf[kBlock];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += kBlock) {
+        const int g = slot_group[i];
+        const int u = g < 0 ? -1 : pick[(size_t)g * S + s];
+        if (u >= 0) acc += (double)samples[((size_t)u * 3 + c) * (size_t)n + i] * msw[i];
+    }
+    buf[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) buf[threadIdx.x] += buf[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.x] = buf[0];
 }
 
 // normals j0 .. j0+n-1 of one particle's stream, one lane per normal
