@@ -91,13 +91,26 @@ void validate(const mp_adjoint_spec &sp)
             "precision must be MP_PRECISION_FP32 or MP_PRECISION_FP64");
 }
 
+// steps per forward launch, 0 when the environment does not say
 int64_t env_steps_per_launch()
 {
     if (const char *env = std::getenv("MAGPY_AMD_ADJOINT_STEPS_PER_LAUNCH")) {
         long long v = std::atoll(env);
         if (v > 0) return (int64_t)v;
     }
-    return 1 << 16;
+    return 0;
+}
+
+// Segments of C steps per forward launch: about 2^16 steps.  A run of fewer than
+// four such blocks is cut into four, so that the maps of one block overlap the
+// forward steps of the next, as long as a block's maps (a lane per segment and
+// particle) keep two waves on each SIMD of the card (2^17 lanes).
+int64_t block_segments(int64_t particles, int64_t segments, int64_t C)
+{
+    if (const int64_t env = env_steps_per_launch()) return std::max<int64_t>(1, env / C);
+    const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 16) / C);
+    const int64_t fill = (((int64_t)1 << 17) + particles - 1) / particles;
+    return std::min(most, std::max((segments + 3) / 4, fill));
 }
 
 // lanes (segment x particle) per adjoint-map launch
@@ -107,7 +120,7 @@ int64_t env_batch_lanes()
         long long v = std::atoll(env);
         if (v > 0) return (int64_t)v;
     }
-    return 1 << 18;
+    return 1 << 20;
 }
 
 struct AdjointBase {
@@ -201,8 +214,8 @@ struct AdjointRun final : AdjointBase {
         C = sp.checkpoint_interval;
         S = sp.n_samples;
         n_ck = (N + C - 1) / C;
-        spl = std::max<int64_t>(C, env_steps_per_launch() / C * C);
-        segs_per_block = spl / C;
+        segs_per_block = block_segments(P, n_ck, C);
+        spl = segs_per_block * C;
         shape.assign(sp.radius_shape, sp.radius_shape + P);
         m0.assign(sp.magnetisation_direction, sp.magnetisation_direction + 3 * P);
         sched.assign(sp.sample_steps, sp.sample_steps + S);
@@ -213,13 +226,13 @@ struct AdjointRun final : AdjointBase {
         sp.seed = nullptr;
         pt.build(sched, N, C);
         n_waves = (int)((P + mp::kWave - 1) / mp::kWave);
-        // transfer batches: about 2^18 lanes (4,096 waves; 2^18 to 2^21
-        // measure the same), scratch at most 8 GiB, the block's segments
-        // split evenly
+        // transfer batches: up to 2^20 lanes (launches of a few waves per SIMD
+        // leave their last round half empty), scratch at most 8 GiB, the block's
+        // segments split evenly
         const int64_t seg_len = std::min(C, N);
         const int64_t by_lanes = std::max<int64_t>(1, env_batch_lanes() / P);
         const int64_t by_bytes = std::max<int64_t>(
-            1, ((int64_t)8 << 30) / (seg_len * mp::kScratchRows * P * (int64_t)sizeof(T)));
+            1, ((int64_t)8 << 30) / ((seg_len + 3) / 4 * 3 * P * (int64_t)sizeof(T)));
         const int64_t most = std::min({segs_per_block, by_lanes, by_bytes});
         const int64_t n_batches = (segs_per_block + most - 1) / most;
         batch_segs = (segs_per_block + n_batches - 1) / n_batches;
@@ -294,7 +307,7 @@ struct AdjointRun final : AdjointBase {
     {
         if (scratch.p) return;
         const int64_t seg_len = std::min(C, N);
-        scratch.alloc((size_t)seg_len * mp::kScratchRows * (size_t)(batch_segs * P));
+        scratch.alloc((size_t)((seg_len + 3) / 4) * 3 * (size_t)(batch_segs * P));
         scratch_bytes = (int64_t)(scratch.n * sizeof(T));
         pieces.alloc((size_t)max_batch_pieces * mp::kTransfer * P);
         acc.alloc((size_t)mp::kTransfer * P);
@@ -314,7 +327,6 @@ struct AdjointRun final : AdjointBase {
         a.tag = sp.noise_tag;
         a.dt = (T)q[0];
         a.alpha = (T)q[2];
-        a.happ = (T)q[3];
         a.mx = mx.p;
         a.my = my.p;
         a.mz = mz.p;
@@ -330,12 +342,12 @@ struct AdjointRun final : AdjointBase {
         return a;
     }
 
-    void table(DevBuf<T> &tab, hipStream_t st, int64_t base, int64_t count)
+    void table(DevBuf<T> &tab, hipStream_t st, T amp, int64_t base, int64_t count)
     {
         require((size_t)count <= tab.n, "field table too small");
         const double fdt = sp.field_frequency * sp.time_step;
         hipLaunchKernelGGL(mp::path_field_table_kernel<T>, dim3((unsigned)((count + 255) / 256)),
-                           dim3(256), 0, st, fdt, base, count, tab.p);
+                           dim3(256), 0, st, fdt, amp, base, count, tab.p);
         MP_HIP(hipGetLastError());
     }
 
@@ -432,7 +444,7 @@ struct AdjointRun final : AdjointBase {
     void record_batch(int64_t j0, int64_t j1, int64_t ck_base, const T *ck_block)
     {
         const int64_t n_a = j0 * C, n_end = std::min(N, j1 * C);
-        table(ftab_tr, tr.s, n_a, n_end - n_a + 2);
+        table(ftab_tr, tr.s, T(1), n_a, n_end - n_a + 2);
         const int64_t piece0 = pt.seg_first[(size_t)j0];
         const int64_t piece1 = j1 < n_ck ? pt.seg_first[(size_t)j1] : (int64_t)pt.start.size();
         mp::TransferArgs<T> t{};
@@ -494,7 +506,7 @@ struct AdjointRun final : AdjointBase {
             // the maps of block k - 2 must be done with this checkpoint buffer
             if (tr_pending[buf]) MP_HIP(hipStreamWaitEvent(sg.s, ev_tr[buf], 0));
             timed(fwd_ms, sg.s, [&] {
-                table(ftab, sg.s, n0, n1 - n0 + 5);
+                table(ftab, sg.s, (T)q[3], n0, n1 - n0 + 5);
                 a.tab0 = n0;
                 a.n0 = n0;
                 a.n1 = n1;

@@ -16,9 +16,9 @@
 // sample step and c_f at the end, and between sample steps it is a linear
 // map of its end value.  Those maps (transfers, below) are computed right
 // after each forward batch, for all segments of the batch in parallel: a
-// lane per (segment, particle) recomputes its segment from the checkpoint
-// into scratch ([C][6][lanes]: states and normals, read back only by the lane
-// that wrote it) and carries three basis adjoints back through it.  They are folded into one
+// lane per (segment, particle) recomputes its segment from the checkpoint,
+// keeping every fourth state in scratch ([C / 4][3][lanes], read back only by the
+// lane that wrote it), and carries three basis adjoints back through it.  They are folded into one
 // transfer per sampling interval, and a reverse pass with given weights is
 // then a short scan over the intervals.
 //
@@ -58,9 +58,9 @@ struct PathArgs {
     const T *sig;                   // sr sqrt(dt) per particle
     const uint32_t *key0, *key1;    // Philox key (member seed) per particle
     uint32_t tag;
-    T dt, alpha, happ;
+    T dt, alpha;
     T *mx, *my, *mz;                // state
-    const T *ftab;                  // ftab[i] = s_{tab0 + i}
+    const T *ftab;                  // ftab[i] = happ s_{tab0 + i}
     int64_t tab0;
     int64_t n_steps;                // N
     int64_t ck_every;               // C (a multiple of 4)
@@ -88,15 +88,23 @@ __device__ inline V3<T> group_w(const T z[12], int i)
 }
 
 // field h(m, s) and v = dt h + sig w (fused multiply-adds fixed by the
-// source, as in llg_map, so the recompute reproduces the forward pass)
+// source, as in llg_map, so the recompute reproduces the forward pass); sw is
+// sig w and hs is happ s, rounded products either way
+template <typename T>
+__device__ inline V3<T> path_v_scaled(const V3<T> &m, const V3<T> &e, const V3<T> &sw, T dt, T hs)
+{
+#pragma clang fp contract(off)
+    const T me = fmad(m.x, e.x, fmad(m.y, e.y, m.z * e.z));
+    return V3<T>{fmad(dt, me * e.x, sw.x), fmad(dt, me * e.y, sw.y),
+                 fmad(dt, fmad(me, e.z, hs), sw.z)};
+}
+
 template <typename T>
 __device__ inline V3<T> path_v(const V3<T> &m, const V3<T> &e, const V3<T> &w, T dt, T sig,
                                T happ, T s)
 {
 #pragma clang fp contract(off)
-    const T me = fmad(m.x, e.x, fmad(m.y, e.y, m.z * e.z));
-    return V3<T>{fmad(dt, me * e.x, sig * w.x), fmad(dt, me * e.y, sig * w.y),
-                 fmad(dt, fmad(me, e.z, happ * s), sig * w.z)};
+    return path_v_scaled(m, e, V3<T>{sig * w.x, sig * w.y, sig * w.z}, dt, happ * s);
 }
 
 template <typename T>
@@ -108,15 +116,24 @@ __device__ inline V3<T> path_L(const V3<T> &m, const V3<T> &v, T al)
 }
 
 template <typename T>
+__device__ inline V3<T> path_step_scaled(const V3<T> &m, const V3<T> &e, const V3<T> &sw, T dt,
+                                         T al, T hs1, T hs2)
+{
+#pragma clang fp contract(off)
+    const V3<T> a1 = path_L(m, path_v_scaled(m, e, sw, dt, hs1), al);
+    const V3<T> mt{m.x + a1.x, m.y + a1.y, m.z + a1.z};
+    const V3<T> a2 = path_L(mt, path_v_scaled(mt, e, sw, dt, hs2), al);
+    return V3<T>{fmad(T(0.5), a1.x + a2.x, m.x), fmad(T(0.5), a1.y + a2.y, m.y),
+                 fmad(T(0.5), a1.z + a2.z, m.z)};
+}
+
+template <typename T>
 __device__ inline V3<T> path_step(const V3<T> &m, const V3<T> &e, const V3<T> &w, T dt, T sig,
                                   T al, T happ, T s1, T s2)
 {
 #pragma clang fp contract(off)
-    const V3<T> a1 = path_L(m, path_v(m, e, w, dt, sig, happ, s1), al);
-    const V3<T> mt{m.x + a1.x, m.y + a1.y, m.z + a1.z};
-    const V3<T> a2 = path_L(mt, path_v(mt, e, w, dt, sig, happ, s2), al);
-    return V3<T>{fmad(T(0.5), a1.x + a2.x, m.x), fmad(T(0.5), a1.y + a2.y, m.y),
-                 fmad(T(0.5), a1.z + a2.z, m.z)};
+    return path_step_scaled(m, e, V3<T>{sig * w.x, sig * w.y, sig * w.z}, dt, al, happ * s1,
+                            happ * s2);
 }
 
 // Unscaled Wiener normals of step group g (steps 4g..4g+3): w of step 4g+i
@@ -165,7 +182,9 @@ struct FwdRing {
 // integrates from the other half, and the two swap halves at a barrier every
 // kGroups groups.  The integrating wave thus carries only the Heun steps; it
 // reads the group's five field values once and keeps the next sample step in
-// a register.
+// a register.  A lone wave issues an instruction every ~5.5 cycles whatever it
+// is, so its instructions bound the kernel: the producer scales the normals by
+// sig and the table holds happ s (0.158 -> 0.149 us per step).
 template <typename T>
 __global__ __launch_bounds__(2 * kWave) void path_forward_kernel(PathArgs<T> a)
 {
@@ -184,7 +203,7 @@ __global__ __launch_bounds__(2 * kWave) void path_forward_kernel(PathArgs<T> a)
     keys.init(a.key0[p], a.key1[p]);
     V3<T> m{a.mx[p], a.my[p], a.mz[p]};
     const V3<T> e{a.ex[p], a.ey[p], a.ez[p]};
-    const T sig = a.sig[p], dt = a.dt, al = a.alpha, ha = a.happ;
+    const T sig = a.sig[p], dt = a.dt, al = a.alpha;
     int64_t s = a.s_next;
     int64_t next_rec = s < a.S ? a.sched[s] : INT64_MAX;
     int64_t ck_n = (a.n0 + a.ck_every - 1) / a.ck_every * a.ck_every;
@@ -203,7 +222,7 @@ __global__ __launch_bounds__(2 * kWave) void path_forward_kernel(PathArgs<T> a)
                     T z[12];
                     path_group_normals<T>(g, a.tag, keys, z);
 #pragma unroll
-                    for (int q = 0; q < 12; ++q) half[k][q][lane] = z[q];
+                    for (int q = 0; q < 12; ++q) half[k][q][lane] = sig * z[q];
                 }
             }
         } else if (c > 0) {
@@ -222,10 +241,10 @@ __global__ __launch_bounds__(2 * kWave) void path_forward_kernel(PathArgs<T> a)
                     ck_n += a.ck_every;
                 }
                 if (nb + 4 <= a.n1 && next_rec >= nb + 4) {
-                    m = path_step(m, e, V3<T>{zc[0], zc[1], zc[2]}, dt, sig, al, ha, f0, f1);
-                    m = path_step(m, e, V3<T>{zc[3], zc[4], zc[5]}, dt, sig, al, ha, f1, f2);
-                    m = path_step(m, e, V3<T>{zc[6], zc[7], zc[8]}, dt, sig, al, ha, f2, f3);
-                    m = path_step(m, e, V3<T>{zc[9], zc[10], zc[11]}, dt, sig, al, ha, f3, f4);
+                    m = path_step_scaled(m, e, V3<T>{zc[0], zc[1], zc[2]}, dt, al, f0, f1);
+                    m = path_step_scaled(m, e, V3<T>{zc[3], zc[4], zc[5]}, dt, al, f1, f2);
+                    m = path_step_scaled(m, e, V3<T>{zc[6], zc[7], zc[8]}, dt, al, f2, f3);
+                    m = path_step_scaled(m, e, V3<T>{zc[9], zc[10], zc[11]}, dt, al, f3, f4);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -237,7 +256,7 @@ __global__ __launch_bounds__(2 * kWave) void path_forward_kernel(PathArgs<T> a)
                         }
                         const T sa = i == 0 ? f0 : i == 1 ? f1 : i == 2 ? f2 : f3;
                         const T sb = i == 0 ? f1 : i == 1 ? f2 : i == 2 ? f3 : f4;
-                        m = path_step(m, e, group_w(zc, i), dt, sig, al, ha, sa, sb);
+                        m = path_step_scaled(m, e, group_w(zc, i), dt, al, sa, sb);
                     }
                 }
             }
@@ -362,23 +381,28 @@ struct TransferArgs {
     int64_t n_steps, ck_every;
     const T *ck;                    // checkpoints of this batch's segments [seg][3][n]
     int64_t seg0, n_segs;           // global index of the first segment, segments in batch
-    T *scratch;                     // [C][kScratchRows][n_segs * n]
+    T *scratch;                     // [ceil(C / 4)][3][n_segs * n]
     const int32_t *seg_first_piece, *seg_n_pieces;   // per segment of the batch
     const int64_t *piece_start;     // first step of each piece (run-wide index)
     int64_t piece_base;             // run-wide index of the batch's first piece
     double *pieces;                 // [piece - piece_base][21][n]
 };
 
-// Rows of scratch per step: the state m_n (3), then the unscaled normals w_n
-// (3), so that the reverse sweep needs no second pass of the generator.
-constexpr int kScratchRows = 6;
-
-// One lane per (segment, particle), particle fastest.
-// Register budget of four waves per SIMD (128 VGPRs, a few spills outside the
-// step body): 4% faster than the three waves the unconstrained kernel gets.
+// One lane per (segment, particle), particle fastest.  The segment is walked in
+// the 4-step groups of the Wiener stream: the forward sweep keeps the state at
+// each group's start (12 bytes per group and lane of FP32), and the reverse
+// sweep forms the group's normals again and steps through it once more, so that
+// its states and normals are in registers.  Keeping every step's state and
+// normals instead (24 bytes per step, written and read back through HBM) waited
+// on those reads.  Bound: VALU issue, ~640 instructions per step.  16,384
+// particles, FP32: 20,000 steps 10.9 -> 8.5 ms with the forward pass, 200,000
+// steps 84 -> 61 ms; 3,000 particles, FP64, 20,000 steps: 24.2 -> 9.8 ms.
+// The next group's state and field values load while a group is worked on.
+// Registers: three waves per SIMD in FP32 (168; four spill: 4.05 against 3.16
+// ms per 163,840 lanes and 1,000 steps), two in FP64.
 template <typename T>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void
-path_transfer_kernel(TransferArgs<T> a)
+__global__ __launch_bounds__(kWave, sizeof(T) == 4 ? 3 : 2) void path_transfer_kernel(
+    TransferArgs<T> a)
 {
     const int64_t lanes = a.n_segs * (int64_t)a.n;
     const int64_t gid0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -389,31 +413,51 @@ path_transfer_kernel(TransferArgs<T> a)
     const int64_t seg = a.seg0 + sl;
     const int64_t n_a = seg * a.ck_every;
     const int64_t n_b = n_a + a.ck_every < a.n_steps ? n_a + a.ck_every : a.n_steps;
+    const int n_groups = (int)((n_b - n_a + 3) >> 2);      // n_a is a multiple of 4
     const V3<T> e{a.ex[p], a.ey[p], a.ez[p]};
     const T sig = a.sig[p], dt = a.dt, al = a.alpha, ha = a.happ;
-    PhiloxKeys keys;
-    keys.init(a.key0[p], a.key1[p]);
-    T z[12];
-    // 1. the segment's states m_{n_a} .. m_{n_b - 1} and their normals
-    //    (n_a is a multiple of 4)
+    const uint32_t key0 = a.key0[p], key1 = a.key1[p];
+    // a group's normals; the round keys are formed again, to hold no registers
+    auto normals = [&](int g, T *z) {
+        uint32_t k0 = key0, k1 = key1;
+        asm volatile("" : "+v"(k0), "+v"(k1));
+        PhiloxKeys keys;
+        keys.init(k0, k1);
+        path_group_normals<T>((n_a >> 2) + g, a.tag, keys, z);
+    };
+    // the field at the five stage times of a group; past the last step those of
+    // the table's end, which no step uses
+    const T *tab = a.ftab + (n_a + 1 - a.tab0);
+    const int last = (int)(n_b - n_a);
+    auto fields = [&](int g, T *f) {
+#pragma unroll
+        for (int j = 0; j < 5; ++j) f[j] = tab[4 * g + j < last ? 4 * g + j : last];
+    };
+    T *row = a.scratch + gid;
+    // 1. the state at each group's start
     V3<T> m = load3(a.ck + (size_t)sl * 3 * P, P, p);
-    for (int64_t n = n_a; n < n_b; ++n) {
-        const int i = (int)(n & 3);
-        if (i == 0) path_group_normals<T>(n >> 2, a.tag, keys, z);
-        const V3<T> w = group_w(z, i);
-        if (live) {
-            T *row = a.scratch + (size_t)(n - n_a) * kScratchRows * L;
-            store3(row, L, (int)gid, m);
-            store3(row + 3 * L, L, (int)gid, w);
-        }
-        m = path_step(m, e, w, dt, sig, al, ha, a.ftab[n + 1 - a.tab0], a.ftab[n + 2 - a.tab0]);
+    T f[5], fn[5];
+    fields(0, fn);
+    for (int g = 0; g < n_groups; ++g) {
+        if (live) store3(row, L, 0, m);
+        row += 3 * L;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) f[j] = fn[j];
+        if (g + 1 == n_groups) break;   // the last group's steps are taken below
+        fields(g + 1, fn);
+        T z[12];
+        normals(g, z);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            m = path_step(m, e, V3<T>{z[3 * i], z[3 * i + 1], z[3 * i + 2]}, dt, sig, al, ha, f[i],
+                          f[i + 1]);
     }
     // 2. three adjoint channels (lambda = e_x, e_y, e_z at the end of each
     //    piece) back through the segment; a piece ends at every sample step.
     //    Parameter terms gather in gs (the state type) and move to g (double)
     //    every 4 steps and at piece ends.
     V3<T> lam[3];
-    double g[3][4];
+    double g64[3][4];
     T gs[3][4];
     auto clear_gs = [&]() {
 #pragma unroll
@@ -425,7 +469,7 @@ path_transfer_kernel(TransferArgs<T> a)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) g[c][q] += (double)gs[c][q];
+            for (int q = 0; q < 4; ++q) g64[c][q] += (double)gs[c][q];
         clear_gs();
     };
     auto reset = [&]() {
@@ -433,45 +477,58 @@ path_transfer_kernel(TransferArgs<T> a)
         for (int c = 0; c < 3; ++c) {
             lam[c] = V3<T>{T(c == 0), T(c == 1), T(c == 2)};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) g[c][q] = 0.0;
+            for (int q = 0; q < 4; ++q) g64[c][q] = 0.0;
         }
         clear_gs();
     };
     reset();
     int piece = a.seg_first_piece[sl] + a.seg_n_pieces[sl] - 1;
     int64_t piece_begin = a.piece_start[piece];
-    // the rows of step n - 1 load while step n runs
-    const T *row = a.scratch + (size_t)(n_b - 1 - n_a) * kScratchRows * L;
-    V3<T> mm_next = load3(row, L, (int)gid), w_next = load3(row + 3 * L, L, (int)gid);
-    for (int64_t n = n_b - 1; n >= n_a; --n) {
-        const V3<T> mm = mm_next, w = w_next;
-        if (n > n_a) {
-            row -= kScratchRows * L;
-            mm_next = load3(row, L, (int)gid);
-            w_next = load3(row + 3 * L, L, (int)gid);
+    V3<T> m_next = m;   // the last group's start
+    row -= 3 * L;
+    for (int g = n_groups - 1; g >= 0; --g) {
+        V3<T> ms[4];
+        ms[0] = m_next;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) f[j] = fn[j];
+        if (g + 1 == n_groups) fields(g, f);
+        if (g > 0) {
+            row -= 3 * L;
+            m_next = load3(row, L, 0);
+            fields(g - 1, fn);
         }
-        const StepFwd<T> f = step_forward(mm, e, w, dt, sig, al, ha, a.ftab[n + 1 - a.tab0],
-                                          a.ftab[n + 2 - a.tab0]);
+        T z[12];
+        normals(g, z);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) lam[c] = step_adjoint(f, e, dt, al, ha, lam[c], gs[c]);
-        if ((n & 3) == 0) flush();
-        if (n == piece_begin) {
-            flush();
-            if (live) {
-                double *out = a.pieces + (size_t)(piece - a.piece_base) * kTransfer * P + p;
+        for (int i = 0; i < 3; ++i)
+            ms[i + 1] = path_step(ms[i], e, V3<T>{z[3 * i], z[3 * i + 1], z[3 * i + 2]}, dt, sig, al,
+                                  ha, f[i], f[i + 1]);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    out[(3 * r + 0) * P] = (double)(r == 0 ? lam[0].x : r == 1 ? lam[0].y : lam[0].z);
-                    out[(3 * r + 1) * P] = (double)(r == 0 ? lam[1].x : r == 1 ? lam[1].y : lam[1].z);
-                    out[(3 * r + 2) * P] = (double)(r == 0 ? lam[2].x : r == 1 ? lam[2].y : lam[2].z);
+        for (int i = 3; i >= 0; --i) {
+            if (4 * g + i >= last) continue;   // past the segment's end
+            const StepFwd<T> fw = step_forward(ms[i], e, V3<T>{z[3 * i], z[3 * i + 1], z[3 * i + 2]},
+                                               dt, sig, al, ha, f[i], f[i + 1]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) lam[c] = step_adjoint(fw, e, dt, al, ha, lam[c], gs[c]);
+            if (i == 0) flush();
+            if (n_a + 4 * g + i == piece_begin) {
+                flush();
+                if (live) {
+                    double *out = a.pieces + (size_t)(piece - a.piece_base) * kTransfer * P + p;
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        out[(3 * r + 0) * P] = (double)(r == 0 ? lam[0].x : r == 1 ? lam[0].y : lam[0].z);
+                        out[(3 * r + 1) * P] = (double)(r == 0 ? lam[1].x : r == 1 ? lam[1].y : lam[1].z);
+                        out[(3 * r + 2) * P] = (double)(r == 0 ? lam[2].x : r == 1 ? lam[2].y : lam[2].z);
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) out[(9 + 3 * q + c) * P] = g64[c][q];
                 }
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) out[(9 + 3 * q + c) * P] = g[c][q];
+                reset();
+                if (piece > a.seg_first_piece[sl]) piece_begin = a.piece_start[--piece];
             }
-            reset();
-            if (piece > a.seg_first_piece[sl]) piece_begin = a.piece_start[--piece];
         }
     }
 }
@@ -574,15 +631,15 @@ __global__ __launch_bounds__(kWave) void path_scan_kernel(ScanArgs a)
     for (int q = 0; q < 4; ++q) a.g[q * P + p] = g[q];
 }
 
-// Field table: out[i] = sin(2 pi frac((base + i) fdt)), FP64 phase reduction.
+// Field table: out[i] = amp sin(2 pi frac((base + i) fdt)), FP64 phase reduction.
 template <typename T>
-__global__ void path_field_table_kernel(double fdt, int64_t base, int64_t count, T *out)
+__global__ void path_field_table_kernel(double fdt, T amp, int64_t base, int64_t count, T *out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
     double c = (double)(base + i) * fdt;
     c -= floor(c);
-    out[i] = (T)sin(2.0 * kPi * c);
+    out[i] = amp * (T)sin(2.0 * kPi * c);
 }
 
 }  // namespace mp
