@@ -231,7 +231,7 @@ int mp_wiener_normals(uint64_t seed, uint32_t particle, uint32_t tag, uint64_t j
  *   J = sum_s grad_ens_mz[s] * ens_mz[s] + grad_final_mz * final_mz
  * with respect to theta through the trajectories (the vector-Jacobian
  * product).  While a recording forward pass runs, the adjoint's linear maps
- * between sample steps are computed from states kept every
+ * between sample steps are computed from states kept at least every
  * checkpoint_interval steps (recomputed in between) and held per sampling
  * interval in device memory (21 doubles per particle per interval), so the
  * reverse pass for any weights is a short scan.  No counterpart in the reference,

@@ -101,16 +101,33 @@ int64_t env_steps_per_launch()
     return 0;
 }
 
+// Length of the segments whose maps are computed in parallel: the checkpoint
+// interval, or the smallest whole part of it that is a multiple of 4 steps and at
+// least 200.  Short segments give small ensembles more lanes (300 particles,
+// 20,000 steps: 4.6 -> 3.7 ms) and let the maps' waves, some of which share a SIMD
+// with a forward wave, even out; each costs a transfer of 168 bytes per particle.
+// Above 2^16 particles one segment of every particle fills the card, and the states
+// kept for shorter ones (two blocks of up to 2^16 steps) would take over 1 GiB.
+int64_t segment_steps(int64_t particles, int64_t checkpoint_interval)
+{
+    if (particles > (int64_t)1 << 16) return checkpoint_interval;
+    const int64_t groups = checkpoint_interval / 4;
+    for (int64_t parts = groups; parts > 1; --parts)
+        if (groups % parts == 0 && checkpoint_interval / parts >= 200)
+            return checkpoint_interval / parts;
+    return checkpoint_interval;
+}
+
 // Segments of C steps per forward launch: about 2^16 steps.  A run of fewer than
-// four such blocks is cut into four, so that the maps of one block overlap the
+// eight such blocks is cut into eight, so that the maps of one block overlap the
 // forward steps of the next, as long as a block's maps (a lane per segment and
-// particle) keep two waves on each SIMD of the card (2^17 lanes).
+// particle) keep three waves on each SIMD of the card.
 int64_t block_segments(int64_t particles, int64_t segments, int64_t C)
 {
     if (const int64_t env = env_steps_per_launch()) return std::max<int64_t>(1, env / C);
     const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 16) / C);
-    const int64_t fill = (((int64_t)1 << 17) + particles - 1) / particles;
-    return std::min(most, std::max((segments + 3) / 4, fill));
+    const int64_t fill = (3 * ((int64_t)1 << 16) + particles - 1) / particles;
+    return std::min(most, std::max((segments + 7) / 8, fill));
 }
 
 // lanes (segment x particle) per adjoint-map launch
@@ -211,7 +228,7 @@ struct AdjointRun final : AdjointBase {
         device = s.device;
         P = sp.n_particles;
         N = sp.n_steps;
-        C = sp.checkpoint_interval;
+        C = segment_steps(P, sp.checkpoint_interval);
         S = sp.n_samples;
         n_ck = (N + C - 1) / C;
         segs_per_block = block_segments(P, n_ck, C);

@@ -395,8 +395,8 @@ struct TransferArgs {
 // its states and normals are in registers.  Keeping every step's state and
 // normals instead (24 bytes per step, written and read back through HBM) waited
 // on those reads.  Bound: VALU issue, ~640 instructions per step.  16,384
-// particles, FP32: 20,000 steps 10.9 -> 8.5 ms with the forward pass, 200,000
-// steps 84 -> 61 ms; 3,000 particles, FP64, 20,000 steps: 24.2 -> 9.8 ms.
+// particles, FP32: 20,000 steps 10.8 -> 7.1 ms with the forward pass, 200,000
+// steps 84 -> 57.8 ms; 3,000 particles, FP64, 20,000 steps: 24.2 -> 8.1 ms.
 // The next group's state and field values load while a group is worked on.
 // Registers: three waves per SIMD in FP32 (168; four spill: 4.05 against 3.16
 // ms per 163,840 lanes and 1,000 steps), two in FP64.
@@ -558,10 +558,20 @@ __global__ __launch_bounds__(kWave) void path_compose_kernel(ComposeArgs a)
     double acc[kTransfer];
 #pragma unroll
     for (int q = 0; q < kTransfer; ++q) acc[q] = a.acc[q * P + p];
+    // the next piece loads while this one is folded (the kernel waits on little
+    // else: a wave per 64 particles)
+    double nx[kTransfer];
+    auto load = [&](int k) {
+        const double *from = a.pieces + (size_t)(k < a.n_pieces ? k : a.n_pieces - 1) * kTransfer * P + p;
+#pragma unroll
+        for (int q = 0; q < kTransfer; ++q) nx[q] = from[q * P];
+    };
+    load(0);
     for (int k = 0; k < a.n_pieces; ++k) {
         double x[kTransfer];
 #pragma unroll
-        for (int q = 0; q < kTransfer; ++q) x[q] = a.pieces[((size_t)k * kTransfer + q) * P + p];
+        for (int q = 0; q < kTransfer; ++q) x[q] = nx[q];
+        load(k + 1);
         if (a.piece_new[k]) {
             if (a.piece_iv[k] > 0)
 #pragma unroll
