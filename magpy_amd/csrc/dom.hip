@@ -63,36 +63,38 @@ void dom_run(const mp_dom_spec &sp, double *time, double *field, double *mz, uin
     require(sp.device >= 0 && sp.device < count, "device index out of range");
     MP_HIP(hipSetDevice(sp.device));
 
-    std::vector<double> happ(P), up(P), down(P), hk(P);
+    // the eight inputs of the kernels one after the other, in one copy
+    std::vector<double> in(8 * (size_t)P);
+    double *const row[8] = {in.data(),         in.data() + P,     in.data() + 2 * P,
+                            in.data() + 3 * P, in.data() + 4 * P, in.data() + 5 * P,
+                            in.data() + 6 * P, in.data() + 7 * P};
+    const double hk0 = 2.0 * sp.anisotropy[0] / kMU0 / sp.magnetisation[0];
     for (int64_t p = 0; p < P; ++p) {
-        hk[p] = 2.0 * sp.anisotropy[p] / kMU0 / sp.magnetisation[p];
-        happ[p] = sp.field_amplitude / hk[p];
-        up[p] = sp.initial_probabilities[2 * p];
-        down[p] = sp.initial_probabilities[2 * p + 1];
+        const double hk = 2.0 * sp.anisotropy[p] / kMU0 / sp.magnetisation[p];
+        row[0][p] = sp.anisotropy[p];
+        row[1][p] = sp.volume[p];
+        row[2][p] = sp.temperature[p];
+        row[3][p] = sp.magnetisation[p];
+        row[4][p] = sp.damping[p];
+        row[5][p] = sp.field_amplitude / hk;
+        row[6][p] = sp.initial_probabilities[2 * p];
+        row[7][p] = sp.initial_probabilities[2 * p + 1];
     }
-    auto vec = [&](const double *x) { return std::vector<double>(x, x + P); };
-    DevBuf<double> dk, dv, dt, dms, dal, dh, dup, ddown, dmz;
-    dk.upload(vec(sp.anisotropy));
-    dv.upload(vec(sp.volume));
-    dt.upload(vec(sp.temperature));
-    dms.upload(vec(sp.magnetisation));
-    dal.upload(vec(sp.damping));
-    dh.upload(happ);
-    dup.upload(up);
-    ddown.upload(down);
+    DevBuf<double> din, dmz;
+    din.upload(in);
     dmz.alloc((size_t)S * P);
     DevBuf<uint32_t> dst(P);
     DevBuf<int64_t> dsteps(P);
     mp::DomArgs a{};
     a.n = (int)P;
-    a.k = dk.p;
-    a.v = dv.p;
-    a.temp = dt.p;
-    a.ms = dms.p;
-    a.alpha = dal.p;
-    a.happ = dh.p;
-    a.p_up = dup.p;
-    a.p_down = ddown.p;
+    a.k = din.p;
+    a.v = din.p + P;
+    a.temp = din.p + 2 * P;
+    a.ms = din.p + 3 * P;
+    a.alpha = din.p + 4 * P;
+    a.happ = din.p + 5 * P;
+    a.p_up = din.p + 6 * P;
+    a.p_down = din.p + 7 * P;
     a.shape = sp.field_shape;
     a.freq = sp.field_frequency;
     a.n_components = sp.field_n_components;
@@ -142,11 +144,17 @@ void dom_run(const mp_dom_spec &sp, double *time, double *field, double *mz, uin
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (kernel_ms) *kernel_ms = ms;
-    std::vector<double> h((size_t)S * P);
-    MP_HIP(hipMemcpy(h.data(), dmz.p, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    if (mz)
-        for (int64_t p = 0; p < P; ++p)
-            for (int64_t s = 0; s < S; ++s) mz[p * S + s] = h[(size_t)s * P + p];
+    if (mz) {
+        // [S][P] to the caller's [P][S], in tiles that stay in cache
+        constexpr int64_t kTile = 32;
+        std::unique_ptr<double[]> h(new double[(size_t)S * P]);
+        MP_HIP(hipMemcpy(h.get(), dmz.p, (size_t)S * P * sizeof(double), hipMemcpyDeviceToHost));
+        for (int64_t p0 = 0; p0 < P; p0 += kTile)
+            for (int64_t s0 = 0; s0 < S; s0 += kTile)
+                for (int64_t p = p0; p < std::min(P, p0 + kTile); ++p)
+                    for (int64_t s = s0; s < std::min(S, s0 + kTile); ++s)
+                        mz[p * S + s] = h[(size_t)(s * P + p)];
+    }
     if (status) MP_HIP(hipMemcpy(status, dst.p, P * sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (steps) MP_HIP(hipMemcpy(steps, dsteps.p, P * sizeof(int64_t), hipMemcpyDeviceToHost));
     // time and field of particle 0 as the reference returns them: the
@@ -156,8 +164,8 @@ void dom_run(const mp_dom_spec &sp, double *time, double *field, double *mz, uin
         const double t = s == 0 ? 0.0 : (double)s * ts;
         if (time) time[s] = t;
         if (field)
-            field[s] = dom_field_host(sp.field_shape, happ[0], sp.field_frequency,
-                                      sp.field_n_components, t) * hk[0];
+            field[s] = dom_field_host(sp.field_shape, row[5][0], sp.field_frequency,
+                                      sp.field_n_components, t) * hk0;
     }
 }
 

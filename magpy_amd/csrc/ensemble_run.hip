@@ -195,27 +195,63 @@ struct HostCopy {
     std::vector<int32_t> shape;
 };
 
-// Results of one launch set copied back to the host, per slot.  Samples and sums
-// of a group taken at or before the run's start step are not recorded (their
-// entries are unspecified or zero).
+// Results of one launch set copied back to the host: states and samples go
+// straight to the caller's arrays, the rest is per slot.  Sums of a sample that a
+// group took at or before the run's start step are unspecified or zero.
 struct GroupOut {
-    std::vector<int64_t> particle_of; // slot -> particle (-1 = padding)
-    std::vector<int> group_of;        // slot -> schedule group
-    std::vector<double> state;        // [slots][3]
     std::vector<uint32_t> status;
-    std::vector<double> samples;      // [S][3][slots] (empty when not recorded)
     std::vector<double> ens;          // [S][3]        (empty when not recorded)
     int64_t newton_iters = 0, newton_fail = 0;
+};
+
+// Where the samples of a launch set go: the caller's [P][S] arrays (any may be
+// null), and what a sample at or before the start step is (the start state as
+// given, or unknown).
+struct SampleSink {
+    double *dst[3];
+    const Plan &plan;
+    const HostCopy &host;
+
+    // Samples of every slot from the records src [records][3][n]; slot_particle[i]
+    // is the particle (-1: padding) and record(i, s) the record of its sample s.
+    // Tiles of particles and samples keep both sides in cache.
+    template <typename T, typename Record>
+    void take(const T *src, const std::vector<int64_t> &slot_particle, Record record) const
+    {
+        constexpr int64_t kTile = 16;
+        const int64_t n = (int64_t)slot_particle.size(), S = host.S;
+        const double nan = std::numeric_limits<double>::quiet_NaN();
+        for (int64_t i0 = 0; i0 < n; i0 += kTile)
+            for (int64_t s0 = 0; s0 < S; s0 += kTile)
+                for (int64_t i = i0; i < std::min(n, i0 + kTile); ++i) {
+                    const int64_t p = slot_particle[(size_t)i];
+                    if (p < 0) continue;
+                    const int64_t m = plan.member_of[(size_t)p];
+                    const double ms = host.ms[(size_t)m];
+                    const std::vector<int64_t> &k = plan.sched[(size_t)plan.group_of[(size_t)m]];
+                    for (int64_t sa = s0; sa < std::min(S, s0 + kTile); ++sa) {
+                        const int64_t at = k[(size_t)sa];
+                        const T *row = at > host.start ? src + record(i, sa) * 3 * n + i : nullptr;
+                        for (int d = 0; d < 3; ++d) {
+                            if (!dst[d]) continue;
+                            const double v = row != nullptr       ? (double)row[d * n]
+                                             : at == host.start ? host.m0[(size_t)p * 3 + d]
+                                                                  : nan;
+                            dst[d][p * S + sa] = v * ms;
+                        }
+                    }
+                }
+    }
 };
 
 struct GroupBase {
     int64_t n_done = 0, n_total = 0, launches = 0;
     virtual ~GroupBase() = default;
     virtual void enqueue(int64_t upto, hipStream_t s) = 0;
-    virtual void state(std::vector<double> &out) = 0;  // [slots][3]
+    virtual void state(double *out) = 0;               // its particles' rows of [P][3]
     virtual const std::vector<int64_t> &slots() const = 0;
     virtual const std::vector<int> &set() const = 0;   // its schedule groups
-    virtual GroupOut collect(hipStream_t s) = 0;
+    virtual GroupOut collect(hipStream_t s, double *state_out, const SampleSink *samples) = 0;
 };
 
 // Cluster packing: members of a group sorted by size (largest first), each
@@ -409,13 +445,13 @@ struct GroupRun : GroupBase {
     std::vector<int64_t> sched, slot_particle;
     std::vector<int> slot_group;              // index into groups (-1: padding)
     std::vector<std::vector<int32_t>> pick;
-    DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_mx, d_my, d_mz, d_samples;
+    DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_m, d_samples;   // d_m: x, y, z, each n
     DevBuf<T> d_px, d_py, d_pz, d_w;
     DevBuf<double> d_fred, d_fdt, d_dtd, d_msw, d_noise, d_partial, d_ens;
     DevBuf<int> d_shape, d_cbase, d_csize;
     DevBuf<uint32_t> d_key0, d_key1, d_pid, d_status;
     DevBuf<int64_t> d_sched;
-    DevBuf<unsigned long long> d_it, d_fl;
+    DevBuf<unsigned long long> d_newton;      // per slot: iterations, then failures
     DevBuf<float> d_htab;      // applied field of one launch (FP32 Heun), a row per field
     bool uniform_field = false;
     DevBuf<int> d_field_shape;                // per row of d_htab
@@ -481,10 +517,11 @@ struct GroupRun : GroupBase {
 
         std::vector<double> ex(n, 0.0), ey(n, 0.0), ez(n, 1.0), k(n, 0.0), al(n, 0.0), dt(n, 0.0),
             sig(n, 0.0), sr(n, 0.0), happ(n, 0.0), fred(n, 0.0), fdt(n, 0.0), msw(n, 0.0),
-            mx(n, 0.0), my(n, 0.0), mz(n, 1.0), px(n, 0.0), py(n, 0.0), pz(n, 0.0), w(n, 0.0);
+            m_now(3 * (size_t)n, 0.0), px(n, 0.0), py(n, 0.0), pz(n, 0.0), w(n, 0.0);
         std::vector<int> shape(n, MP_FIELD_CONSTANT);
         std::vector<uint32_t> key0(n, 0), key1(n, 0), pid(n, 0);
         bool first = true;
+        std::fill(m_now.begin() + 2 * (ptrdiff_t)n, m_now.end(), 1.0);
         for (int i = 0; i < n; ++i) {
             const int64_t p = slot_particle[(size_t)i];
             if (p < 0) continue;
@@ -495,9 +532,7 @@ struct GroupRun : GroupBase {
             ey[i] = sp.anisotropy_axis[3 * p + 1];
             ez[i] = sp.anisotropy_axis[3 * p + 2];
             const double *m0 = sp.start_state ? sp.start_state : sp.magnetisation_direction;
-            mx[i] = m0[3 * p];
-            my[i] = m0[3 * p + 1];
-            mz[i] = m0[3 * p + 2];
+            for (int d = 0; d < 3; ++d) m_now[(size_t)d * n + i] = m0[3 * p + d];
             k[i] = r.k_red[(size_t)lp];
             al[i] = sp.damping[m];
             dt[i] = r.dt;
@@ -566,9 +601,7 @@ struct GroupRun : GroupBase {
         d_sig.upload(cast_vec<T>(sig));
         d_sr.upload(cast_vec<T>(sr));
         d_happ.upload(cast_vec<T>(happ));
-        d_mx.upload(cast_vec<T>(mx));
-        d_my.upload(cast_vec<T>(my));
-        d_mz.upload(cast_vec<T>(mz));
+        d_m.upload(cast_vec<T>(m_now));
         d_fred.upload(fred);
         d_fdt.upload(fdt);
         d_dtd.upload(dt);
@@ -579,8 +612,8 @@ struct GroupRun : GroupBase {
         d_pid.upload(pid);
         d_status.upload(std::vector<uint32_t>((size_t)n, 0));
         d_sched.upload(sched);
-        d_it.upload(std::vector<unsigned long long>((size_t)n, 0));
-        d_fl.upload(std::vector<unsigned long long>((size_t)n, 0));
+        if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT)
+            d_newton.upload(std::vector<unsigned long long>(2 * (size_t)n, 0));
         if (cluster) {
             d_px.upload(cast_vec<T>(px));
             d_py.upload(cast_vec<T>(py));
@@ -631,7 +664,7 @@ struct GroupRun : GroupBase {
         a.shape = d_shape.p;
         a.key0 = d_key0.p; a.key1 = d_key1.p; a.pid = d_pid.p;
         a.msw = d_msw.p;
-        a.mx = d_mx.p; a.my = d_my.p; a.mz = d_mz.p;
+        a.mx = d_m.p; a.my = d_m.p + n; a.mz = d_m.p + 2 * (size_t)n;
         a.status = d_status.p;
         a.sched = d_sched.p;
         a.S = S;
@@ -645,6 +678,9 @@ struct GroupRun : GroupBase {
 
     const std::vector<int64_t> &slots() const override { return slot_particle; }
     const std::vector<int> &set() const override { return groups; }
+
+    unsigned long long *newton_iters() const { return d_newton.p; }
+    unsigned long long *newton_fails() const { return d_newton.p ? d_newton.p + n : nullptr; }
 
     void launch_cluster(hipStream_t s, const float *htab)
     {
@@ -676,7 +712,7 @@ struct GroupRun : GroupBase {
     {
         mp::ImplicitClusterArgs ia{
             mp::ClusterArgs<double>{a, d_px.p, d_py.p, d_pz.p, d_w.p, d_cbase.p, d_csize.p}, eps,
-            max_iter, d_it.p, d_fl.p, interactions ? 1 : 0};
+            max_iter, newton_iters(), newton_fails(), interactions ? 1 : 0};
         // a source per slot, a sum per `targets` slots, a flag per slot
         const size_t shmem = (size_t)block * (sizeof(mp::Source) + sizeof(int)) +
                              (size_t)(block / targets) * sizeof(double);
@@ -785,10 +821,10 @@ struct GroupRun : GroupBase {
             if (cluster)
                 launch_cluster(s, htab);
             else if (array_noise)
-                launch_shape<T, true>(shape_kind, a, scheme, eps, max_iter, d_it.p, d_fl.p, grid, s,
+                launch_shape<T, true>(shape_kind, a, scheme, eps, max_iter, newton_iters(), newton_fails(), grid, s,
                                       htab, false);
             else
-                launch_shape<T, false>(shape_kind, a, scheme, eps, max_iter, d_it.p, d_fl.p, grid, s,
+                launch_shape<T, false>(shape_kind, a, scheme, eps, max_iter, newton_iters(), newton_fails(), grid, s,
                                        htab, two_wave);
             MP_HIP(hipGetLastError());
             ++launches;
@@ -796,28 +832,20 @@ struct GroupRun : GroupBase {
         }
     }
 
-    void state(std::vector<double> &out) override
+    void state(double *out) override
     {
-        std::vector<T> hx((size_t)n), hy((size_t)n), hz((size_t)n);
-        MP_HIP(hipMemcpy(hx.data(), d_mx.p, n * sizeof(T), hipMemcpyDeviceToHost));
-        MP_HIP(hipMemcpy(hy.data(), d_my.p, n * sizeof(T), hipMemcpyDeviceToHost));
-        MP_HIP(hipMemcpy(hz.data(), d_mz.p, n * sizeof(T), hipMemcpyDeviceToHost));
-        out.resize((size_t)n * 3);
+        std::unique_ptr<T[]> h(new T[3 * (size_t)n]);
+        MP_HIP(hipMemcpy(h.get(), d_m.p, 3 * (size_t)n * sizeof(T), hipMemcpyDeviceToHost));
         for (int i = 0; i < n; ++i) {
-            out[(size_t)i * 3] = (double)hx[(size_t)i];
-            out[(size_t)i * 3 + 1] = (double)hy[(size_t)i];
-            out[(size_t)i * 3 + 2] = (double)hz[(size_t)i];
+            const int64_t p = slot_particle[(size_t)i];
+            if (p < 0) continue;
+            for (int d = 0; d < 3; ++d) out[3 * p + d] = (double)h[(size_t)d * n + i];
         }
     }
 
-    GroupOut collect(hipStream_t s) override
+    GroupOut collect(hipStream_t s, double *state_out, const SampleSink *sink) override
     {
         GroupOut o;
-        o.particle_of = slot_particle;
-        o.group_of.resize((size_t)n);
-        for (int i = 0; i < n; ++i)
-            o.group_of[(size_t)i] =
-                slot_group[(size_t)i] < 0 ? groups[0] : groups[(size_t)slot_group[(size_t)i]];
         const bool several = groups.size() > 1;
         if (want_ens) {
             if (several)
@@ -830,34 +858,29 @@ struct GroupRun : GroupBase {
             MP_HIP(hipGetLastError());
         }
         MP_HIP(hipStreamSynchronize(s));
-        state(o.state);
+        if (state_out) state(state_out);
         o.status.resize((size_t)n);
         MP_HIP(hipMemcpy(o.status.data(), d_status.p, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
-        std::vector<unsigned long long> it((size_t)n), fl((size_t)n);
-        MP_HIP(hipMemcpy(it.data(), d_it.p, n * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-        MP_HIP(hipMemcpy(fl.data(), d_fl.p, n * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-        for (int i = 0; i < n; ++i) {
-            o.newton_iters += (int64_t)it[(size_t)i];
-            o.newton_fail += (int64_t)fl[(size_t)i];
-        }
-        if (want_traj) {
-            std::vector<T> hs(d_samples.n);
-            if (!hs.empty())
-                MP_HIP(hipMemcpy(hs.data(), d_samples.p, hs.size() * sizeof(T), hipMemcpyDeviceToHost));
-            if (several) {
-                o.samples.resize((size_t)S_out * 3 * (size_t)n);
-                for (int64_t sa = 0; sa < S_out; ++sa)
-                    for (int d = 0; d < 3; ++d)
-                        for (int i = 0; i < n; ++i) {
-                            const int g = slot_group[(size_t)i];
-                            const int32_t u = g < 0 ? -1 : pick[(size_t)g][(size_t)sa];
-                            if (u >= 0)
-                                o.samples[((size_t)sa * 3 + d) * (size_t)n + (size_t)i] =
-                                    (double)hs[((size_t)u * 3 + d) * (size_t)n + (size_t)i];
-                        }
-            } else {
-                o.samples.assign(hs.begin(), hs.end());
+        if (d_newton.p) {
+            std::vector<unsigned long long> c(2 * (size_t)n);
+            MP_HIP(hipMemcpy(c.data(), d_newton.p, c.size() * sizeof(unsigned long long),
+                             hipMemcpyDeviceToHost));
+            for (int i = 0; i < n; ++i) {
+                o.newton_iters += (int64_t)c[(size_t)i];
+                o.newton_fail += (int64_t)c[(size_t)(n + i)];
             }
+        }
+        if (sink != nullptr && want_traj) {
+            std::unique_ptr<T[]> h(new T[d_samples.n]);
+            if (d_samples.n)
+                MP_HIP(hipMemcpy(h.get(), d_samples.p, d_samples.n * sizeof(T),
+                                 hipMemcpyDeviceToHost));
+            if (several)
+                sink->take(h.get(), slot_particle, [&](int64_t i, int64_t sa) {
+                    return (int64_t)pick[(size_t)slot_group[(size_t)i]][(size_t)sa];
+                });
+            else
+                sink->take(h.get(), slot_particle, [](int64_t, int64_t sa) { return sa; });
         }
         if (want_ens) {
             o.ens.resize((size_t)S_out * 3);
@@ -1127,38 +1150,44 @@ struct ReplicaRun : GroupBase {
         }
     }
 
-    void state(std::vector<double> &out) override
+    // The device packs the live columns to [reps n][3] in a buffer that is free
+    // between steps (the increments, or the field); the host widens them piece by
+    // piece.  4,096 x 512: 22 -> 6 ms against the padded rows repacked on the host.
+    void state(double *out) override
     {
-        std::vector<float> hm((size_t)rows * ld);
-        MP_HIP(hipMemcpy(hm.data(), d_m.p, hm.size() * sizeof(float), hipMemcpyDeviceToHost));
-        out.resize((size_t)reps * n * 3);
-        for (int rr = 0; rr < reps; ++rr)
-            for (int p = 0; p < n; ++p)
-                for (int c = 0; c < 3; ++c)
-                    out[((size_t)rr * n + p) * 3 + c] = hm[(size_t)rr * ld + mp::replica_col(p, c)];
+        const int64_t total = 3 * (int64_t)reps * n, piece = (int64_t)1 << 20;
+        float *packed = fused ? d_nz.p : d_h.p;
+        hipLaunchKernelGGL(mp::replica_pack_kernel, dim3((unsigned)((reps * n + 255) / 256)),
+                           dim3(256), 0, nullptr, a, packed);
+        MP_HIP(hipGetLastError());
+        std::unique_ptr<float[]> h(new float[(size_t)std::min(total, piece)]);
+        for (int64_t o = 0; o < total; o += piece) {
+            const int64_t len = std::min(piece, total - o);
+            MP_HIP(hipMemcpy(h.get(), packed + o, (size_t)len * sizeof(float),
+                             hipMemcpyDeviceToHost));
+            for (int64_t i = 0; i < len; ++i) out[o + i] = (double)h[(size_t)i];
+        }
     }
 
-    GroupOut collect(hipStream_t s) override
+    GroupOut collect(hipStream_t s, double *state_out, const SampleSink *sink) override
     {
         GroupOut o;
-        o.particle_of = slot_particle;
-        o.group_of.assign(slot_particle.size(), 0);
         if (want_ens) {
             hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
                                s, d_partial.p, n_waves, S * 3, d_ens.p);
             MP_HIP(hipGetLastError());
         }
         MP_HIP(hipStreamSynchronize(s));
-        state(o.state);
+        if (state_out) state(state_out);
         o.status.resize((size_t)reps * n);
         MP_HIP(hipMemcpy(o.status.data(), d_status.p, o.status.size() * sizeof(uint32_t),
                          hipMemcpyDeviceToHost));
-        if (want_traj) {
-            std::vector<float> hs(d_samples.n);
-            if (!hs.empty())
-                MP_HIP(hipMemcpy(hs.data(), d_samples.p, hs.size() * sizeof(float),
+        if (sink != nullptr && want_traj) {
+            std::unique_ptr<float[]> h(new float[d_samples.n]);
+            if (d_samples.n)
+                MP_HIP(hipMemcpy(h.get(), d_samples.p, d_samples.n * sizeof(float),
                                  hipMemcpyDeviceToHost));
-            o.samples.assign(hs.begin(), hs.end());
+            sink->take(h.get(), slot_particle, [](int64_t, int64_t sa) { return sa; });
         }
         if (want_ens) {
             o.ens.resize((size_t)S * 3);
@@ -1575,7 +1604,9 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     if (gemm != 0) {
         ss->cluster_block = 0;
         ss->dipolar = gemm;
+        UploadScope uploads;
         ss->groups.emplace_back(new ReplicaRun(sp, plan, traj, ens, gemm));
+        uploads.flush();
         return ss.release();
     }
     if (sp.dipolar == MP_DIPOLAR_GEMM_BF16X3 || sp.dipolar == MP_DIPOLAR_GEMM_F32)
@@ -1591,6 +1622,7 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     ss->dipolar = cluster_block && sp.interactions ? MP_DIPOLAR_PAIRS : 0;
     ss->cluster_block = cluster_block;
     ss->cluster_lanes = cluster_block ? layout.lanes : 0;
+    UploadScope uploads;
     for (const std::vector<int> &set : launch_sets(sp, plan, cluster_block != 0, in_arena)) {
         if (sp.precision == MP_PRECISION_FP32 && sp.scheme == MP_SCHEME_HEUN)
             ss->groups.emplace_back(
@@ -1599,6 +1631,7 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
             ss->groups.emplace_back(
                 new GroupRun<double>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
     }
+    uploads.flush();
     return ss.release();
 }
 
@@ -1632,40 +1665,23 @@ void session_finish(mp_session *ss, mp_ensemble_out &out)
     MP_HIP(hipSetDevice(ss->device));
     const HostCopy &h = ss->host;
     const Plan &plan = ss->plan;
-    const int64_t P = h.P, S = h.S;
+    const int64_t S = h.S;
     const bool want_traj = ss->want_traj && (out.mx || out.my || out.mz);
-    std::vector<double> state((size_t)P * 3), traj, ens;
-    std::vector<uint32_t> status((size_t)P, 0);
-    if (want_traj) traj.assign((size_t)S * 3 * (size_t)P, 0.0);
+    const SampleSink sink{{out.mx, out.my, out.mz}, plan, h};
+    std::vector<double> ens;
     if (out.ens_m && ss->want_ens) ens.assign((size_t)S * 3, 0.0);
     int64_t newton_iters = 0, newton_fail = 0;
     for (auto &run : ss->groups) {
-        GroupOut o = run->collect(ss->sg.s);
-        const int n = (int)o.particle_of.size();
-        for (int i = 0; i < n; ++i) {
-            const int64_t p = o.particle_of[(size_t)i];
-            if (p < 0) continue;
-            for (int d = 0; d < 3; ++d) state[(size_t)p * 3 + d] = o.state[(size_t)i * 3 + d];
-            status[(size_t)p] = o.status[(size_t)i];
-        }
+        const GroupOut o = run->collect(ss->sg.s, out.final_state, want_traj ? &sink : nullptr);
+        const std::vector<int64_t> &slots = run->slots();
+        if (out.status)
+            for (size_t i = 0; i < slots.size(); ++i)
+                if (slots[i] >= 0) out.status[slots[i]] = o.status[i];
         newton_iters += o.newton_iters;
         newton_fail += o.newton_fail;
         // samples recorded at the start step are the start state exactly as
         // given; samples before a resumed run's start step are not known
         const double nan = std::numeric_limits<double>::quiet_NaN();
-        if (want_traj)
-            for (int64_t s = 0; s < S; ++s)
-                for (int i = 0; i < n; ++i) {
-                    const int64_t p = o.particle_of[(size_t)i];
-                    if (p < 0) continue;
-                    const int64_t k = plan.sched[(size_t)o.group_of[(size_t)i]][(size_t)s];
-                    for (int d = 0; d < 3; ++d)
-                        traj[((size_t)s * 3 + d) * (size_t)P + (size_t)p] =
-                            k < h.start ? nan
-                            : k == h.start
-                                ? h.m0[(size_t)p * 3 + d]
-                                : o.samples[((size_t)s * 3 + d) * (size_t)n + (size_t)i];
-                }
         if (!ens.empty())
             for (int64_t s = 0; s < S; ++s) {
                 // what the set's groups recorded of sample s, and the start states
@@ -1678,11 +1694,12 @@ void session_finish(mp_session *ss, mp_ensemble_out &out)
                     all = all && k > h.start;
                 }
                 if (known && !all)
-                    for (int i = 0; i < n; ++i) {
-                        const int64_t p = o.particle_of[(size_t)i];
-                        if (p < 0 || plan.sched[(size_t)o.group_of[(size_t)i]][(size_t)s] > h.start)
+                    for (const int64_t p : slots) {
+                        if (p < 0) continue;
+                        const int64_t m = plan.member_of[(size_t)p];
+                        if (plan.sched[(size_t)plan.group_of[(size_t)m]][(size_t)s] > h.start)
                             continue;
-                        const double w = h.ms[(size_t)plan.member_of[(size_t)p]];
+                        const double w = h.ms[(size_t)m];
                         for (int d = 0; d < 3; ++d) v[d] += h.m0[(size_t)p * 3 + d] * w;
                     }
                 const bool recorded = all || run->set().size() > 1;
@@ -1708,20 +1725,7 @@ void session_finish(mp_session *ss, mp_ensemble_out &out)
         for (int64_t m = 0; m < h.M; ++m)
             fill_time_field(m, out.member_time ? out.member_time + m * S : nullptr,
                             out.member_field ? out.member_field + m * S : nullptr);
-    if (want_traj) {
-        double *dst[3] = {out.mx, out.my, out.mz};
-        for (int64_t p = 0; p < P; ++p) {
-            const double ms = h.ms[(size_t)plan.member_of[(size_t)p]];
-            for (int d = 0; d < 3; ++d) {
-                if (!dst[d]) continue;
-                for (int64_t s = 0; s < S; ++s)
-                    dst[d][p * S + s] = traj[((size_t)s * 3 + d) * (size_t)P + (size_t)p] * ms;
-            }
-        }
-    }
     if (out.ens_m && !ens.empty()) std::memcpy(out.ens_m, ens.data(), ens.size() * sizeof(double));
-    if (out.final_state) std::memcpy(out.final_state, state.data(), state.size() * sizeof(double));
-    if (out.status) std::memcpy(out.status, status.data(), status.size() * sizeof(uint32_t));
     out.n_steps = plan.group_steps[0];
     out.newton_iters = newton_iters;
     out.newton_failures = newton_fail;
@@ -1891,16 +1895,7 @@ int mp_session_state(mp_session *session, double *state, int64_t *step)
         if (!session || !state) throw simulation::Error(MP_ERR_ARG, "session and state are required");
         MP_HIP(hipSetDevice(session->device));
         MP_HIP(hipStreamSynchronize(session->sg.s));
-        for (size_t gi = 0; gi < session->groups.size(); ++gi) {
-            std::vector<double> st;
-            session->groups[gi]->state(st);
-            const std::vector<int64_t> &slots = session->groups[gi]->slots();
-            for (size_t i = 0; i < slots.size(); ++i) {
-                const int64_t p = slots[i];
-                if (p < 0) continue;
-                for (int d = 0; d < 3; ++d) state[p * 3 + d] = st[i * 3 + d];
-            }
-        }
+        for (auto &g : session->groups) g->state(state);
         if (step) *step = session->groups[0]->n_done;
     });
 }

@@ -623,4 +623,14 @@ static __global__ __launch_bounds__(256) void replica_stage2_kernel(ReplicaArgs 
     }
 }
 
+// The states of the live (replica, particle) elements as [reps n][3].
+static __global__ __launch_bounds__(256) void replica_pack_kernel(ReplicaArgs a, float *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= a.n * a.reps) return;
+    const size_t ox = (size_t)(i / a.n) * a.ld + replica_col(i % a.n, 0);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) out[3 * (size_t)i + d] = a.m[ox + 32 * d];
+}
+
 }  // namespace mp
