@@ -921,21 +921,36 @@ void dipole_tensor(const simulation::ReducedMember &r, const double *loc, double
         }
 }
 
-void split_host(const std::vector<double> &x, std::vector<__bf16> &hi, std::vector<__bf16> &lo)
+// The tensor as the product's fragments (replica_fragment): BF16 hi and lo, or FP32.
+std::vector<float> tensor_fragments(const std::vector<double> &D, int ld, int mode)
 {
-    hi.resize(x.size());
-    lo.resize(x.size());
-    for (size_t i = 0; i < x.size(); ++i) {
-        const float f = (float)x[i];
-        hi[i] = (__bf16)f;
-        lo[i] = (__bf16)(f - (float)hi[i]);
-    }
+    std::vector<float> out((size_t)ld * ld);
+    for (int pb = 0; pb < ld / 96; ++pb)
+        for (int ks = 0; ks < ld / 16; ++ks)
+            for (int u = 0; u < 3; ++u) {
+                char *const part[2] = {
+                    reinterpret_cast<char *>(out.data() + 4 * mp::replica_fragment(ld, pb, ks, u, 0)),
+                    reinterpret_cast<char *>(out.data() + 4 * mp::replica_fragment(ld, pb, ks, u, 1))};
+                for (int l = 0; l < mp::kWave; ++l)
+                    for (int j = 0; j < 8; ++j) {
+                        const int row = 96 * pb + 32 * u + (l & 31);
+                        const float x = (float)D[(size_t)row * ld + mp::replica_k(ks, l, j)];
+                        if (mode == MP_DIPOLAR_GEMM_F32) {
+                            std::memcpy(part[j >> 2] + 16 * l + 4 * (j & 3), &x, sizeof(x));
+                        } else {
+                            const __bf16 hi = (__bf16)x, lo = (__bf16)(x - (float)hi);
+                            std::memcpy(part[0] + 16 * l + 2 * j, &hi, sizeof(hi));
+                            std::memcpy(part[1] + 16 * l + 2 * j, &lo, sizeof(lo));
+                        }
+                    }
+            }
+    return out;
 }
 
 // Replica layout sizes: particles padded to a multiple of kParticlePad
-// (ld = 3 Np), replicas to a multiple of the 128-row block tile.
+// (ld = 3 Np), replicas to a multiple of the rows of a block.
 int replica_ld(int64_t n) { return 3 * pad_to(n, mp::kParticlePad); }
-int replica_rows(int64_t reps) { return pad_to(reps, mp::kBM); }
+int replica_rows(int64_t reps) { return pad_to(reps, mp::kReplicaPad); }
 
 // Which panels the blocks that one XCD runs share: 1 (default) the row
 // panels of the state, so each XCD reads an eighth of it and all of the
@@ -950,47 +965,69 @@ int replica_row_panels()
     return v;
 }
 
-// The BF16x3 product runs the Heun stages in its epilogue unless
+// The product runs the Heun stages in its epilogue unless
 // MAGPY_AMD_REPLICA_FUSED=0 when the run is created (then it writes the
-// field and separate stage kernels follow, as for the FP32 product; the two
-// give the same bits).
+// field and separate stage kernels follow; the two give the same bits).
 bool replica_fused()
 {
     const char *e = std::getenv("MAGPY_AMD_REPLICA_FUSED");
     return !(e != nullptr && std::string(e) == "0");
 }
 
-void launch_product(int mode, const float *a32, const float *b32, const __bf16 *b_hi,
-                    const __bf16 *b_lo, float *c, int rows, int ld, hipStream_t s)
+// One product with the epilogue `epi` (replica_product_kernel).  Blocks of four wave
+// pairs of 64 replicas share most, but a CU takes one: below a block per CU, blocks
+// of one pair; and where pairs of 32 replicas still fit the card at once (two waves
+// per SIMD), those, whose sums take half as long.  The sums are the same in all.
+// 512 steps, ms (start: blocks of 8 waves whatever the size, particles padded to 128)
+// with blocks of four pairs, pairs of 64 and pairs of 32 replicas:
+//   1,000 x 64   24.0   14.5  9.8  6.4      4,096 x 256  51.7  31.7  28.8  25.7
+//   64 x 400     58.7   42.1  22.3  13.9    2,048 x 512  74.4  51.6  45.0  43.0
+//   1,024 x 256  37.1   28.1  16.7  10.3    3,900 x 450  86.0    -   68.5  94.7
+//   4,096 x 512  92.4 (72.7 us a product)  70.9 (61 and 66 us), 75.5, -
+void launch_product(int mode, int epi, const float *state, const float *tensor,
+                    const mp::ReplicaArgs &a, int rows, int cus, int64_t step, float hstage,
+                    int64_t s_first, int n_rec, hipStream_t s)
 {
-    require(rows % mp::kBM == 0 && ld % mp::kBN == 0 && ld % mp::kGemmTile == 0 &&
-                ld % (6 * mp::kBK) == 0,
+    require(rows % mp::kReplicaPad == 0 && a.ld % (3 * mp::kParticlePad) == 0,
             "replica product: rows or ld do not fit the tiles");
-    if (mode == MP_DIPOLAR_GEMM_F32) {
-        const dim3 grid((unsigned)(rows / mp::kGemmTile), (unsigned)(ld / mp::kGemmTile));
-        hipLaunchKernelGGL(mp::gemm_f32_kernel, grid, dim3(256), 0, s, a32, b32, c, ld, ld);
-    } else {
-        const int nrb = rows / mp::kBM, ncb = ld / mp::kBN;
-        hipLaunchKernelGGL(mp::gemm_bf16x3_ksplit_kernel<0>, dim3((unsigned)(nrb * ncb)), dim3(512),
-                           0, s, a32, b_hi, b_lo, c, ld, ld, nrb, ncb, mp::ReplicaArgs{},
-                           (int64_t)0, 0.f, (int64_t)0, 0, replica_row_panels());
-    }
+    auto go = [&](auto kernel, auto w, auto t) {
+        constexpr int W = decltype(w)::value, KT = decltype(t)::value;
+        const int nrb = rows / (32 * KT * W), ncb = a.ld / (96 * W);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(nrb * ncb)), dim3(128 * W * W), 0, s, state,
+                           reinterpret_cast<const mp::f32x4 *>(tensor), a, step, hstage, s_first,
+                           n_rec, nrb, ncb, replica_row_panels());
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    auto with_epilogue = [&](auto m, auto w, auto t) {
+        constexpr int M = decltype(m)::value, W = decltype(w)::value, KT = decltype(t)::value;
+        if (epi == 0) go(mp::replica_product_kernel<M, 0, W, KT>, w, t);
+        else if (epi == 1) go(mp::replica_product_kernel<M, 1, W, KT>, w, t);
+        else go(mp::replica_product_kernel<M, 2, W, KT>, w, t);
+    };
+    const int64_t pairs = (int64_t)(rows / 64) * (a.ld / 96);
+    auto with_mode = [&](auto m) {
+        if (pairs >= 4 * (int64_t)cus) with_epilogue(m, Two{}, Two{});
+        else if (pairs > 2 * (int64_t)cus) with_epilogue(m, One{}, Two{});
+        else with_epilogue(m, One{}, One{});
+    };
+    if (mode == MP_DIPOLAR_GEMM_F32) with_mode(std::integral_constant<int, mp::kReplicaF32>{});
+    else with_mode(std::integral_constant<int, mp::kReplicaBf16x3>{});
+    MP_HIP(hipGetLastError());
 }
 
-// All members are one cluster replicated: state [rows][ld] replica-major,
-// four launches per Heun step (product, stage 1, product, stage 2); the
-// products read the FP32 state and split it to BF16 themselves.
+// All members are one cluster replicated: two products per Heun step, with the
+// stages in their epilogues or in kernels of their own.
 struct ReplicaRun : GroupBase {
-    int n = 0, reps = 0, ld = 0, rows = 0, mode = MP_DIPOLAR_GEMM_BF16X3, n_waves = 0;
+    int n = 0, reps = 0, ld = 0, rows = 0, mode = MP_DIPOLAR_GEMM_BF16X3, n_waves = 0, cus = 0;
     bool fused = false;
     int shape = MP_FIELD_CONSTANT;
     double happ = 0.0, fapp = 0.0, dt = 0.0;
     bool want_traj = false, want_ens = false;
     int64_t S = 0, s_next = 0;
     std::vector<int64_t> sched, slot_particle;
-    DevBuf<float> d_m, d_mt, d_h, d_nz, d_kex, d_key, d_kez, d_edx, d_edy, d_edz, d_sig, d_b32,
-        d_samples;
-    DevBuf<__bf16> d_bhi, d_blo;
+    DevBuf<float> d_m, d_mt, d_h, d_nz, d_kex, d_key, d_kez, d_edx, d_edy, d_edz, d_sig,
+        d_tensor, d_samples;
     DevBuf<uint32_t> d_key0, d_key1, d_status;
     DevBuf<double> d_msw, d_partial, d_ens;
     DevBuf<int64_t> d_sched;
@@ -999,7 +1036,8 @@ struct ReplicaRun : GroupBase {
     ReplicaRun(const simulation::EnsembleSpec &sp, const Plan &plan, bool traj, bool ens, int m)
     {
         mode = m;
-        fused = mode == MP_DIPOLAR_GEMM_BF16X3 && replica_fused();
+        cus = device_cus();
+        fused = replica_fused();
         reps = (int)sp.n_members;
         n = (int)(sp.member_offsets[1] - sp.member_offsets[0]);
         ld = replica_ld(n);
@@ -1050,24 +1088,17 @@ struct ReplicaRun : GroupBase {
         // dipole tensor and its split
         std::vector<double> D;
         dipole_tensor(r, sp.location, sp.magnetisation[0], (size_t)n, ld, D);
-        if (mode == MP_DIPOLAR_GEMM_F32) {
-            d_b32.upload(cast_vec<float>(D));
-        } else {
-            std::vector<__bf16> hi, lo;
-            split_host(D, hi, lo);
-            d_bhi.upload(hi);
-            d_blo.upload(lo);
-        }
-        // state, replica-major and zero padded
-        std::vector<double> m0((size_t)rows * ld, 0.0);
+        d_tensor.upload(tensor_fragments(D, ld, mode));
+        // state, zero padded
+        std::vector<float> m0((size_t)rows * ld, 0.f);
         const double *src = sp.start_state ? sp.start_state : sp.magnetisation_direction;
         for (int rr = 0; rr < reps; ++rr)
             for (int p = 0; p < n; ++p)
                 for (int c = 0; c < 3; ++c)
-                    m0[(size_t)rr * ld + mp::replica_col(p, c)] =
-                        src[3 * (sp.member_offsets[rr] + p) + c];
+                    m0[mp::replica_at(ld, rr, mp::replica_col(p, c))] =
+                        (float)src[3 * (sp.member_offsets[rr] + p) + c];
         n_done = std::min(sp.start_step, n_total);
-        d_m.upload(cast_vec<float>(m0));
+        d_m.upload(m0);
         d_mt.upload(std::vector<float>(m0.size(), 0.f));
         // the fused product keeps the field on chip and passes the step's
         // increments from stage 1 to stage 2; the separate stages pass the field
@@ -1076,9 +1107,9 @@ struct ReplicaRun : GroupBase {
         d_status.upload(std::vector<uint32_t>((size_t)reps * n, 0));
         d_sched.upload(sched);
         const int threads = reps * n;
-        const int grid = (threads + 255) / 256;
-        // the fused BF16x3 stages write one ensemble partial per product wave
-        n_waves = fused ? (rows / mp::kBM) * (ld / mp::kBN) * 8 : grid * 4;
+        // ensemble partials: one per 32 replicas x 32 particles of the product, or per
+        // wave of the stage kernels
+        n_waves = (rows / 32) * (ld / 96) * (fused ? 1 : 16);
         if (want_traj) d_samples.alloc((size_t)S * 3 * (size_t)threads);
         if (want_ens) {
             d_partial.alloc((size_t)S * 3 * (size_t)n_waves);
@@ -1115,8 +1146,7 @@ struct ReplicaRun : GroupBase {
     void enqueue(int64_t upto, hipStream_t s) override
     {
         upto = std::min(upto, n_total);
-        const int threads = reps * n;
-        const dim3 grid((unsigned)((threads + 255) / 256));
+        const dim3 grid((unsigned)((rows / 32) * (ld / 96) * 4));   // stage kernels
         while (n_done < upto) {
             const int64_t st = n_done;
             const double t1 = (double)(st + 1) * dt;
@@ -1126,21 +1156,12 @@ struct ReplicaRun : GroupBase {
             int n_rec = 0;
             while (s_next + n_rec < S && sched[(size_t)(s_next + n_rec)] == st + 1) ++n_rec;
             if (fused) {
-                // the stages run in the products' epilogues
-                require(rows % mp::kBM == 0 && ld % mp::kBN == 0 && ld % (6 * mp::kBK) == 0,
-                        "replica product: rows or ld do not fit the tiles");
-                const int nrb = rows / mp::kBM, ncb = ld / mp::kBN;
-                const dim3 pg((unsigned)(nrb * ncb)), pb(512);
-                hipLaunchKernelGGL(mp::gemm_bf16x3_ksplit_kernel<1>, pg, pb, 0, s, d_m.p, d_bhi.p,
-                                   d_blo.p, (float *)nullptr, ld, ld, nrb, ncb, a, st, h1,
-                                   (int64_t)0, 0, replica_row_panels());
-                hipLaunchKernelGGL(mp::gemm_bf16x3_ksplit_kernel<2>, pg, pb, 0, s, d_mt.p, d_bhi.p,
-                                   d_blo.p, (float *)nullptr, ld, ld, nrb, ncb, a, st, h2, s_next,
-                                   n_rec, replica_row_panels());
+                launch_product(mode, 1, d_m.p, d_tensor.p, a, rows, cus, st, h1, 0, 0, s);
+                launch_product(mode, 2, d_mt.p, d_tensor.p, a, rows, cus, st, h2, s_next, n_rec, s);
             } else {
-                launch_product(mode, d_m.p, d_b32.p, d_bhi.p, d_blo.p, d_h.p, rows, ld, s);
+                launch_product(mode, 0, d_m.p, d_tensor.p, a, rows, cus, st, 0.f, 0, 0, s);
                 hipLaunchKernelGGL(mp::replica_stage1_kernel, grid, dim3(256), 0, s, a, st, h1);
-                launch_product(mode, d_mt.p, d_b32.p, d_bhi.p, d_blo.p, d_h.p, rows, ld, s);
+                launch_product(mode, 0, d_mt.p, d_tensor.p, a, rows, cus, st, 0.f, 0, 0, s);
                 hipLaunchKernelGGL(mp::replica_stage2_kernel, grid, dim3(256), 0, s, a, st, h2,
                                    s_next, n_rec);
             }
@@ -1959,22 +1980,21 @@ int mp_dipolar_field(const double *location, const double *radius, const double 
             MP_HIP(hipGetLastError());
             MP_HIP(hipMemcpy(out.data(), dc.p, out.size() * sizeof(double), hipMemcpyDeviceToHost));
         } else {
-            DevBuf<float> a32, b32, c32((size_t)rows * ld);
-            DevBuf<__bf16> bhi, blo;
-            a32.upload(cast_vec<float>(ma));
-            if (mode == MP_DIPOLAR_GEMM_F32) {
-                b32.upload(cast_vec<float>(D));
-            } else {
-                std::vector<__bf16> hi, lo;
-                split_host(D, hi, lo);
-                bhi.upload(hi);
-                blo.upload(lo);
-            }
-            launch_product(mode, a32.p, b32.p, bhi.p, blo.p, c32.p, rows, ld, 0);
-            MP_HIP(hipGetLastError());
-            std::vector<float> o32(out.size());
-            MP_HIP(hipMemcpy(o32.data(), c32.p, o32.size() * sizeof(float), hipMemcpyDeviceToHost));
-            out.assign(o32.begin(), o32.end());
+            std::vector<float> tiled((size_t)rows * ld);
+            for (int rr = 0; rr < rows; ++rr)
+                for (int c = 0; c < ld; ++c)
+                    tiled[mp::replica_at(ld, rr, c)] = (float)ma[(size_t)rr * ld + c];
+            DevBuf<float> a32, tensor, c32((size_t)rows * ld);
+            a32.upload(tiled);
+            tensor.upload(tensor_fragments(D, ld, mode));
+            mp::ReplicaArgs a{};
+            a.ld = ld;
+            a.h = c32.p;
+            launch_product(mode, 0, a32.p, tensor.p, a, rows, device_cus(), 0, 0.f, 0, 0, 0);
+            MP_HIP(hipMemcpy(tiled.data(), c32.p, tiled.size() * sizeof(float), hipMemcpyDeviceToHost));
+            for (int rr = 0; rr < rows; ++rr)
+                for (int c = 0; c < ld; ++c)
+                    out[(size_t)rr * ld + c] = (double)tiled[mp::replica_at(ld, rr, c)];
         }
         for (size_t rr = 0; rr < reps; ++rr)
             for (size_t p = 0; p < n_particles; ++p)

@@ -13,17 +13,23 @@
 //
 // Columns are laid out component-blocked per 32 particles: particle i,
 // component a sits in column 96 (i / 32) + 32 a + i % 32 (replica_col), with
-// the particle count padded to a multiple of 128 so ld = 3 Np is a multiple
-// of 384.  The same permutation is applied to both indices of D, so the
-// product is unchanged; a 32-column MFMA tile then holds one component of 32
-// consecutive particles, and stage kernels read x, y, z as three coalesced
-// 128-byte rows.
+// the particle count padded to a multiple of 64.  The same permutation is applied
+// to both indices of D, so the product is unchanged; a 32-column MFMA tile then
+// holds one component of 32 consecutive particles.
+//
+// State, field and increments are stored in tiles of 32 replicas x 32 columns, in
+// the order in which a wave holds the tile as MFMA output with the tensor's rows as
+// the first operand (replica_at): lane l holds replica l % 32 and, in its 16
+// registers, particles 8 g + 4 (l / 32) + e.  The same 16 values in the same lane
+// are a fragment of the second operand, for a sum over k in that order, which the
+// tensor's fragments follow: what a lane computes is what it loads for the next
+// product, every access is 16 bytes per lane and 1 KB per wave, and no operand goes
+// through LDS.
 //
 // The product runs on MFMA in BF16 with the three-term split
 // x = x_hi + x_lo (x_hi = bf16(x), x_lo = bf16(x - x_hi)):
 //   Mt D^T ~ Mt_hi D_hi^T + Mt_hi D_lo^T + Mt_lo D_hi^T, FP32 accumulation,
-// or in FP32 on MFMA.  The BF16x3 product runs the Heun stages in its
-// epilogue; after the FP32 product they are elementwise kernels.
+// or in FP32 on MFMA, and the Heun stages run in its epilogue.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -38,39 +44,42 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-constexpr int kGemmTile = 128;  // block tile of the FP32 product: 4 waves of 64 x 64
-constexpr int kParticlePad = 128;  // particles per replica padded to a multiple of this
+constexpr int kParticlePad = 64;   // particles per replica padded to a multiple of this
+constexpr int kReplicaPad = 128;   // replicas padded to a multiple of this
 
 __host__ __device__ inline int replica_col(int i, int a) { return 96 * (i >> 5) + 32 * a + (i & 31); }
 
-__device__ inline void split_bf16(float x, __bf16 &hi, __bf16 &lo)
+// Place of (replica r, column c) in the state arrays: tiles of 1,024 values, rows
+// of tiles along the columns.
+__host__ __device__ inline size_t replica_at(int ld, int r, int c)
 {
-    hi = (__bf16)x;
-    lo = (__bf16)(x - (float)hi);
+    const int p = c & 31, lane = (r & 31) + 32 * ((p >> 2) & 1);
+    return (((size_t)(r >> 5) * (size_t)(ld >> 5) + (size_t)(c >> 5)) * 4 + (size_t)(p >> 3)) * 256 +
+           (size_t)(4 * lane + (p & 3));
 }
 
-// Store one 32x32 MFMA accumulator: element (row, col) of the tile is in lane
-// col + 32 * ((row / 4) % 2), register 4 * (row / 8) + row % 4.
-__device__ inline void store_tile32(float *C, int ldc, int r0, int c0, const f32x16 &acc)
+// Column of the tensor that lane l multiplies in slot j (0-7) of the product's step
+// ks (16 columns): the state's particles in the order above.
+__host__ __device__ inline int replica_k(int ks, int l, int j)
 {
-    const int l = threadIdx.x & 63;
-    const int col = c0 + (l & 31);
-#pragma unroll
-    for (int reg = 0; reg < 16; ++reg) {
-        const int row = r0 + 8 * (reg >> 2) + 4 * (l >> 5) + (reg & 3);
-        C[(size_t)row * ldc + col] = acc[reg];
-    }
+    return 32 * (ks >> 1) + 8 * (2 * (ks & 1) + (j >> 2)) + 4 * (l >> 5) + (j & 3);
+}
+
+// Place of part h (of two) of the tensor's fragments: particle block pb, step ks,
+// component u; 64 lanes of 16 bytes from there.  BF16: part 0 is hi and part 1 lo of
+// the eight slots of a lane; FP32: slots 0-3 and 4-7.
+__host__ __device__ inline size_t replica_fragment(int ld, int pb, int ks, int u, int h)
+{
+    return ((((size_t)pb * (size_t)(ld >> 4) + (size_t)ks) * 3 + (size_t)u) * 2 + (size_t)h) * 64;
 }
 
 // ------------------------------------------------------------------ Heun stages
-// Per-replica Heun stages around the product.  Thread = (replica r, particle
-// p), p fastest; state rows are replica-major with leading dimension ld
-// (>= 3N, padded).  The applied field of the two stage times is uniform and
-// passed in (h1, h2).
+// Per-replica Heun stages around the product.  The applied field of the two stage
+// times is uniform and passed in (h1, h2).
 struct ReplicaArgs {
     int n;                  // particles per replica
     int reps;               // replicas
-    int ld;                 // row length 3 Np (Np = n padded to a multiple of 128)
+    int ld;                 // columns 3 Np (Np = n padded to a multiple of kParticlePad)
     int n_waves;            // waves in the grid (ensemble partial stride)
     const float *kex, *key, *kez, *edx, *edy, *edz;  // per particle: k e, e dt
     const float *sig;       // per particle: sr sqrt(dt)
@@ -79,8 +88,8 @@ struct ReplicaArgs {
     const double *msw;             // per replica Ms
     uint32_t tag;
     int renorm;
-    float *m, *mt, *h;             // [reps][ld]: state, predictor, field
-    float *nz;                     // [reps][ld]: the step's scaled Wiener increments (fused
+    float *m, *mt, *h;             // replica_at: state, predictor, field
+    float *nz;                     // replica_at: the step's scaled Wiener increments (fused
                                    // product: stage 1 writes them, stage 2 reads them)
     uint32_t *status;              // [reps * n]
     // sampling
@@ -185,373 +194,310 @@ __device__ inline void replica_stage2_math(const ReplicaArgs &a, const ReplicaPa
     }
 }
 
-// Store m' of a live element and flag a non-finite state.
-__device__ inline void replica_store_state(const ReplicaArgs &a, int r, int p, size_t ox, float mx,
-                                           float my, float mz)
+// Flag a non-finite state.
+__device__ inline void replica_check(const ReplicaArgs &a, int r, int p, float mx, float my,
+                                     float mz)
 {
-    a.m[ox] = mx;
-    a.m[ox + 32] = my;
-    a.m[ox + 64] = mz;
     if (!(isfinite(mx) && isfinite(my) && isfinite(mz))) a.status[(size_t)r * a.n + p] |= 1u;
 }
 
-// Ht = Mt_hi D_hi^T + Mt_hi D_lo^T + Mt_lo D_hi^T with LDS staging; Mt is
-// read in FP32 and split on its way to LDS, D comes pre-split.  Block
-// tile 128 rows x 192 columns; each tile of 64 x 96 (2 x 3 MFMA tiles) is
-// computed by two waves (8 waves per block), one per 16-k half of every
-// 32-k stage, so each SIMD holds two waves and one can issue MFMAs while the
-// other waits on LDS or the barrier; the halves are added through LDS at the
-// end.  Stages are double-buffered in LDS and prefetched three stages ahead
-// in registers.  Blocks are numbered so that the blocks one XCD runs (block
-// ids b with equal b % 8) share panels: with row_panels, row panels of Mt
-// (each XCD reads an eighth of Mt and all of D), else column panels of D;
-// the shared panels then stay in that XCD's L2.  rows % 128 == 0,
-// cols % 192 == 0, K % 192 == 0 (stages come in sixes).  MFMAs are ordered so that six independent accumulators separate
-// dependent ones.
+// Ht = Mt D^T, and in the epilogue kEpi the Heun stage 1 or 2 on the tile that the
+// wave holds (kEpi 0: the field goes to a.h).  A pair of waves computes 32 particles
+// (three tiles of D's rows, one per component) x 32 kT replicas; the two (kh) take
+// alternate steps of 16 columns, so that 4,096 x 512 has two waves on each SIMD, and
+// each finishes half of the tile from the sums of both (exchanged through LDS).  A
+// block is kW x kW pairs, whose waves share operands in the CU's L1.  Operands go
+// from memory to registers, a step of up to 10 KB per wave ahead, with no LDS and no
+// barrier in the loop; the state is split to BF16 in registers.  Blocks are numbered
+// so that the blocks one XCD runs (block ids b with equal b % 8) share panels: with
+// row_panels, row panels of Mt (each XCD reads an eighth of Mt and all of D), else
+// column panels of D.
 //
-// kEpi selects the epilogue: 0 stores the product Ht to c; 1 and 2 run the
-// Heun stage 1 or 2 on the tile instead (ra, stage field hstage, step
-// n_step; stage 2 records the samples s_first .. s_first + n_rec - 1), so
-// the field never leaves the kernel.  A lane holds x, y and z of the same
-// (replica, particle) in its three column subtiles (u = 0, 1, 2), so the
-// stage is per lane; the two k halves each finish half of the registers
-// (kh = 0 the registers 0-7 of every subtile, kh = 1 the registers 8-15).
-constexpr int kBM = 128, kBN = 192, kBK = 32;
+// What bounds it (4,096 x 512, kW = kT = 2): 58 GFLOP of BF16 MFMA.  With operands
+// of ordinary values the chip's power holds MFMA alone to 1,750-1,800 TFLOP/s (33 us;
+// 24.5 on zeros) and a fed loop to about 1,130 (51 us), what a library product of
+// 8,192^3 reaches.  The product with its field stored takes 55 us (44 on zeros);
+// with both operands staged through LDS 61.4, the tensor alone 57.6, three steps
+// ahead 56.9, one wave per SIMD with twice the tile 53.1 (but then nothing draws
+// beside it, and the stages take longer alone).  With stage 1 61 us and with stage 2
+// 66 (both 72.7 with the operands through LDS and 4-byte accesses).
+enum ReplicaMode { kReplicaBf16x3, kReplicaF32 };
 
-template <int kEpi>
-static __global__ __launch_bounds__(512) void gemm_bf16x3_ksplit_kernel(
-    const float *__restrict__ a, const __bf16 *__restrict__ b_hi,
-    const __bf16 *__restrict__ b_lo, float *__restrict__ c, int K, int ldc, int n_row_blocks,
-    int n_col_blocks, ReplicaArgs ra, int64_t n_step, float hstage, int64_t s_first, int n_rec,
+template <int kMode, int kT>
+struct ReplicaStep {
+    f32x4 m[kT][2];    // state: replica tiles, groups 2 (ks % 2) and the next
+    f32x4 d[3][2];     // tensor: component, part
+
+    __device__ inline void load(const f32x4 *const state[kT], const f32x4 *tensor, int ks)
+    {
+#pragma unroll
+        for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) m[t][h] = state[t][ks * 128 + h * 64];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) d[u][h] = tensor[(ks * 6 + u * 2 + h) * 64];
+    }
+
+    __device__ inline void multiply(f32x16 acc[3][kT]) const
+    {
+        if constexpr (kMode == kReplicaBf16x3) {
+            bf16x8 x[2][kT], y[3][2];
+#pragma unroll
+            for (int t = 0; t < kT; ++t)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const float v = m[t][q >> 2][q & 3];
+                    const __bf16 hi = (__bf16)v;
+                    x[0][t][q] = hi;
+                    x[1][t][q] = (__bf16)(v - (float)hi);
+                }
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) y[u][h] = __builtin_bit_cast(bf16x8, d[u][h]);
+            // 3 kT independent accumulators between dependent instructions
+#pragma unroll
+            for (int term = 0; term < 3; ++term)
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+#pragma unroll
+                    for (int t = 0; t < kT; ++t)
+                        acc[u][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            y[u][term == 1 ? 1 : 0], x[term == 2 ? 1 : 0][t], acc[u][t], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+#pragma unroll
+                    for (int t = 0; t < kT; ++t)
+                        acc[u][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                            d[u][q >> 2][q & 3], m[t][q >> 2][q & 3], acc[u][t], 0, 0, 0);
+        }
+    }
+};
+
+template <int kMode, int kEpi, int kW, int kT>
+static __global__ __launch_bounds__(128 * kW * kW, 2) void replica_product_kernel(
+    const float *__restrict__ state, const f32x4 *__restrict__ tensor, ReplicaArgs a,
+    int64_t n_step, float hstage, int64_t s_first, int n_rec, int n_row_blocks, int n_col_blocks,
     int row_panels)
 {
-    constexpr int kLdsRow = kBK + 8;
-    constexpr int kPanelA = kBM * kLdsRow, kPanelB = kBN * kLdsRow;   // bf16 per panel
-    // one LDS array: [buffer][hi/lo] A panels, then B panels; reused at the
-    // end for the reduction of the two k halves
-    __shared__ __attribute__((aligned(16))) __bf16 lds[4 * kPanelA + 4 * kPanelB];
-    auto sa = [&](int buf, int h) { return lds + (2 * buf + h) * kPanelA; };
-    auto sb = [&](int buf, int h) { return lds + 4 * kPanelA + (2 * buf + h) * kPanelB; };
-    const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63;
-    const int kh = wave >> 2, w4 = wave & 3, wr = w4 >> 1, wc = w4 & 1;
+    constexpr int kPairs = kW * kW;
+    __shared__ f32x4 red[2 * kPairs][6 * kT * 64];
+    __shared__ f32x4 constants[7][8 * kW];     // of the block's particles, four at a time
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int kh = wave / kPairs, w = wave % kPairs, wr = w / kW, wc = w % kW;
     const int total = n_row_blocks * n_col_blocks;
     int logical = blockIdx.x;
     if (total % 8 == 0) logical = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
     const int cb = row_panels ? logical % n_col_blocks : logical / n_row_blocks;
     const int rb = row_panels ? logical / n_col_blocks : logical % n_row_blocks;
-    const int row0 = rb * kBM, col0 = cb * kBN;
-    f32x16 acc[2][3];
+    const int rt0 = kT * (kW * rb + wr), pb = kW * cb + wc;   // first replica tile, particle block
+    const int tiles = a.ld >> 5, steps = a.ld >> 4;
+    if constexpr (kEpi != 0) {
+        const float *src[7] = {a.kex, a.key, a.kez, a.edx, a.edy, a.edz, a.sig};
+        if (wave == 0 && l < 32 * kW) {
+            const int p = 32 * kW * cb + l;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[t][u][q] = 0.f;
-
-    // staging: A is FP32, 1024 chunks of 4 values (two per thread), split
-    // into hi/lo BF16 on the way to LDS; B 768 chunks of 8 BF16 per part
-    // (threads 0..255 take a second one); three stages in flight
-    typedef __attribute__((ext_vector_type(4))) uint32_t u32x4v;
-    typedef __attribute__((ext_vector_type(4))) float f32x4v;
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    f32x4v ga[3][2];
-    u32x4v gb[3][2][2];
-    const bool two_b = tid < 256;
-    const int n_stages = K / kBK;
-    auto load_stage = [&](auto set_c, int st) {
-        constexpr int R = decltype(set_c)::value;
-        if (st >= n_stages) return;
-        const int k0 = st * kBK;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int ch = tid + 512 * i, row = ch >> 3, kc = ch & 7;
-            ga[R][i] = *reinterpret_cast<const f32x4v *>(a + (size_t)(row0 + row) * K + k0 + 4 * kc);
+            for (int c = 0; c < 7; ++c)
+                reinterpret_cast<float *>(constants[c])[l] = src[c][p < a.n ? p : a.n - 1];
         }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            if (i == 1 && !two_b) break;
-            const int ch = tid + 512 * i, row = ch >> 2, kc = ch & 3;
-            const size_t off = (size_t)(col0 + row) * K + k0 + 8 * kc;
-            gb[R][0][i] = *reinterpret_cast<const u32x4v *>(b_hi + off);
-            gb[R][1][i] = *reinterpret_cast<const u32x4v *>(b_lo + off);
-        }
-    };
-    auto store_stage = [&](auto set_c, auto buf_c) {
-        constexpr int R = decltype(set_c)::value, B = decltype(buf_c)::value;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int ch = tid + 512 * i, row = ch >> 3, kc = ch & 7;
-            bf16x4 hi, lo;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float x = ga[R][i][q];
-                const __bf16 h = (__bf16)x;
-                hi[q] = h;
-                lo[q] = (__bf16)(x - (float)h);
-            }
-            *reinterpret_cast<bf16x4 *>(sa(B, 0) + row * kLdsRow + 4 * kc) = hi;
-            *reinterpret_cast<bf16x4 *>(sa(B, 1) + row * kLdsRow + 4 * kc) = lo;
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            if (i == 1 && !two_b) break;
-            const int ch = tid + 512 * i, row = ch >> 2, kc = ch & 3;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                *reinterpret_cast<u32x4v *>(sb(B, h) + row * kLdsRow + 8 * kc) = gb[R][h][i];
-        }
-    };
-    auto compute = [&](auto buf_c) {
-        constexpr int B = decltype(buf_c)::value;
-        const int kq = 16 * kh + 8 * (l >> 5);
-        bf16x8 xa[2][2], xb[2][3];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                xa[h][t] = *reinterpret_cast<const bf16x8 *>(
-                    sa(B, h) + (64 * wr + 32 * t + (l & 31)) * kLdsRow + kq);
-#pragma unroll
-        for (int u = 0; u < 3; ++u)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                xb[h][u] = *reinterpret_cast<const bf16x8 *>(
-                    sb(B, h) + (96 * wc + 32 * u + (l & 31)) * kLdsRow + kq);
-#pragma unroll
-        for (int term = 0; term < 3; ++term)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 3; ++u)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        xa[term == 2 ? 1 : 0][t], xb[term == 1 ? 1 : 0][u], acc[t][u], 0, 0, 0);
-    };
-    auto step = [&](auto s_c, int st) {
-        constexpr int S6 = decltype(s_c)::value;
-        compute(std::integral_constant<int, S6 % 2>{});
-        if (st + 1 < n_stages)
-            store_stage(std::integral_constant<int, (S6 + 1) % 3>{},
-                        std::integral_constant<int, (S6 + 1) % 2>{});
-        __syncthreads();
-        load_stage(std::integral_constant<int, (S6 + 1) % 3>{}, st + 4);
-    };
-    load_stage(std::integral_constant<int, 0>{}, 0);
-    store_stage(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-    __syncthreads();
-    load_stage(std::integral_constant<int, 1>{}, 1);
-    load_stage(std::integral_constant<int, 2>{}, 2);
-    load_stage(std::integral_constant<int, 0>{}, 3);
-    for (int st = 0; st < n_stages; st += 6) {
-        step(std::integral_constant<int, 0>{}, st);
-        step(std::integral_constant<int, 1>{}, st + 1);
-        step(std::integral_constant<int, 2>{}, st + 2);
-        step(std::integral_constant<int, 3>{}, st + 3);
-        step(std::integral_constant<int, 4>{}, st + 4);
-        step(std::integral_constant<int, 5>{}, st + 5);
     }
-    // the loop ends on a barrier: the staging LDS is free for the reduction
-    // of the two k halves (4 tiles x 6144 floats = 96 KB)
-    float *red = reinterpret_cast<float *>(lds);
-    static_assert(sizeof(lds) >= 4 * 6144 * sizeof(float), "reduction buffer");
-    if constexpr (kEpi == 0) {
-        float *mine = red + (size_t)w4 * 6144;
-        if (kh == 1) {
+    // Each wave of the pair finishes half of the tile: of two replica tiles the one
+    // kh, of one the groups 2 kh and 2 kh + 1 of four particles; the rest of its sums
+    // goes to its partner.  i counts a wave's groups, 16 bytes a lane each.
+    constexpr int kGroups = 2 * kT;
+    const int rt = rt0 + (kT == 2 ? kh : 0), g0 = kT == 2 ? 0 : 2 * kh;
+    const int r = 32 * rt + (l & 31);
+    const size_t at0 = ((size_t)rt * tiles + 3 * (size_t)pb) * 256 + (size_t)(64 * g0 + l);
+    auto place = [&](int u, int i) { return at0 + (size_t)(u * 256 + i * 64); };
+    auto get = [&](const float *p, int u, int i) {
+        return reinterpret_cast<const f32x4 *>(p)[place(u, i)];
+    };
+    auto put = [&](float *p, int u, int i, const f32x4 &v) {
+        reinterpret_cast<f32x4 *>(p)[place(u, i)] = v;
+    };
+    // particles of group i, counted in groups of four from the block's first
+    auto quad = [&](int i) { return 8 * wc + 2 * (g0 + i) + (l >> 5); };
+    const int rk = r < a.reps ? r : 0;
+    // Stage 1 draws the step's increments and stores them for both stages: one wave
+    // of a tile before its sums and the other after them, so that on each SIMD one
+    // draws (VALU) while the other multiplies: stage 1 of 4,096 x 512 70.7 -> 61.3 us.
+    auto draw = [&]() {
+        const uint32_t key0 = a.key0[rk], key1 = a.key1[rk];
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+        for (int i = 0; i < kGroups; ++i) {
+            const f32x4 sig = constants[6][quad(i)];
+            f32x4 inc[3];
 #pragma unroll
-                for (int u = 0; u < 3; ++u)
+            for (int e = 0; e < 4; ++e) {
+                float z[3];
+                replica_normals(key0, key1, a.tag, 32 * kW * cb + 4 * quad(i) + e, n_step, sig[e],
+                                z[0], z[1], z[2]);
 #pragma unroll
-                    for (int q = 0; q < 16; ++q) mine[((t * 3 + u) * 16 + q) * 64 + l] = acc[t][u][q];
-        }
-        __syncthreads();
-        if (kh == 0) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 3; ++u) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) acc[t][u][q] += mine[((t * 3 + u) * 16 + q) * 64 + l];
-                    store_tile32(c, ldc, row0 + 64 * wr + 32 * t, col0 + 96 * wc + 32 * u, acc[t][u]);
-                }
-        }
-    } else {
-        // each half sends the registers the other finishes.  The stage's
-        // loads of a lane's 8 elements per row tile (stage 1: state and
-        // Philox keys; stage 2: state, predictor and the increments stage 1
-        // drew) are issued together, the first tile's before the exchange
-        // barrier.
-        float *send = red + (size_t)(2 * w4 + kh) * 3072;
-        const float *recv = red + (size_t)(2 * w4 + 1 - kh) * 3072;
-        auto send_half = [&](auto qs_c) {
-            constexpr int QS = decltype(qs_c)::value;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 3; ++u)
-#pragma unroll
-                    for (int qq = 0; qq < 8; ++qq)
-                        send[((t * 3 + u) * 8 + qq) * 64 + l] = acc[t][u][QS + qq];
-        };
-        const int gcol = col0 + 96 * wc;             // x column of this wave's 32 particles
-        const int p = 32 * (gcol / 96) + (l & 31);   // particle of this lane's columns
-        const ReplicaParticle cp = replica_particle(ra, p < ra.n ? p : ra.n - 1);
-        const int qm = 8 * kh;                       // registers this half finishes
-        struct Batch {
-            float m[8][3], t[8][3], z[8][3];
-            uint32_t k0[8], k1[8];
-        };
-        auto row_of = [&](int t, int qq) {
-            const int q = qm + qq;
-            return row0 + 64 * wr + 32 * t + 8 * (q >> 2) + 4 * (l >> 5) + (q & 3);
-        };
-        auto load_batch = [&](int t, Batch &bt) {
-#pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-                const int r = row_of(t, qq);
-                const int rr = r < ra.reps ? r : 0;      // rows past the last replica: row 0
-                const size_t ox = (size_t)rr * ra.ld + gcol + (l & 31);
-#pragma unroll
-                for (int u = 0; u < 3; ++u) {
-                    bt.m[qq][u] = ra.m[ox + 32 * u];
-                    if constexpr (kEpi == 2) {
-                        bt.t[qq][u] = ra.mt[ox + 32 * u];
-                        bt.z[qq][u] = ra.nz[ox + 32 * u];
-                    }
-                }
-                if constexpr (kEpi == 1) {
-                    bt.k0[qq] = ra.key0[rr];
-                    bt.k1[qq] = ra.key1[rr];
-                }
+                for (int u = 0; u < 3; ++u) inc[u][e] = z[u];
             }
-        };
-        double ex = 0.0, ey = 0.0, ez = 0.0;
-        auto finish_batch = [&](auto qm_c, auto t_c, const Batch &bt) {
-            constexpr int QM = decltype(qm_c)::value, t = decltype(t_c)::value;
 #pragma unroll
-            for (int qq = 0; qq < 8; ++qq) {
-                float h[3];
+            for (int u = 0; u < 3; ++u) put(a.nz, u, i, inc[u]);
+        }
+    };
+    if constexpr (kEpi == 1) {
+        __syncthreads();   // the particles' constants
+        if (kh == 1) draw();
+    }
+    const f32x4 *st[kT];
 #pragma unroll
-                for (int u = 0; u < 3; ++u)
-                    h[u] = acc[t][u][QM + qq] + recv[((t * 3 + u) * 8 + qq) * 64 + l];
-                const int r = row_of(t, qq);
-                const bool live = r < ra.reps && p < ra.n;
-                if (!live) continue;
-                const size_t ox = (size_t)r * ra.ld + gcol + (l & 31);
-                if constexpr (kEpi == 1) {
-                    float sx, sy, sz, tx, ty, tz;
-                    replica_normals(bt.k0[qq], bt.k1[qq], ra.tag, p, n_step, cp.sig, sx, sy, sz);
-                    replica_stage1_math(ra, cp, sx, sy, sz, hstage, h[0], h[1], h[2], bt.m[qq][0],
-                                        bt.m[qq][1], bt.m[qq][2], tx, ty, tz);
-                    ra.mt[ox] = tx;
-                    ra.mt[ox + 32] = ty;
-                    ra.mt[ox + 64] = tz;
-                    ra.nz[ox] = sx;
-                    ra.nz[ox + 32] = sy;
-                    ra.nz[ox + 64] = sz;
-                } else {
-                    float mx, my, mz;
-                    replica_stage2_math(ra, cp, bt.z[qq][0], bt.z[qq][1], bt.z[qq][2], hstage, h[0],
-                                        h[1], h[2], bt.t[qq][0], bt.t[qq][1], bt.t[qq][2],
-                                        bt.m[qq][0], bt.m[qq][1], bt.m[qq][2], mx, my, mz);
-                    replica_store_state(ra, r, p, ox, mx, my, mz);
-                    if (n_rec > 0) {
-                        const double w = ra.msw[r];
-                        ex += (double)mx * w;
-                        ey += (double)my * w;
-                        ez += (double)mz * w;
-                        if (ra.samples != nullptr) {
-                            const size_t P = (size_t)ra.n * ra.reps, i = (size_t)r * ra.n + p;
-                            for (int k = 0; k < n_rec; ++k) {
-                                float *base = ra.samples + (size_t)(s_first + k) * 3 * P;
-                                base[i] = mx;
-                                base[P + i] = my;
-                                base[2 * P + i] = mz;
-                            }
+    for (int t = 0; t < kT; ++t)
+        st[t] = reinterpret_cast<const f32x4 *>(state) + (size_t)(rt0 + t) * tiles * 256 + l;
+    const f32x4 *dt0 = tensor + replica_fragment(a.ld, pb, 0, 0, 0) + l;
+    f32x16 acc[3][kT];
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+        for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[u][t][q] = 0.f;
+    // this wave's steps kh, kh + 2, ...: an even number (ld is a multiple of 192), each
+    // loaded while the one before is multiplied (the scheduler would otherwise move
+    // the loads down to their use); the load past the last is of the first step
+    ReplicaStep<kMode, kT> f[2];
+    const int mine = steps / 2;
+    f[0].load(st, dt0, kh);
+    for (int i = 0; i < mine; i += 2) {
+        f[1].load(st, dt0, 2 * (i + 1) + kh);
+        __builtin_amdgcn_sched_barrier(0);
+        f[0].multiply(acc);
+        f[0].load(st, dt0, 2 * (i + 2 < mine ? i + 2 : 0) + kh);
+        __builtin_amdgcn_sched_barrier(0);
+        f[1].multiply(acc);
+    }
+    f32x4 m[3][kGroups], mt[3][kGroups], nz[3][kGroups];
+    auto load_half = [&](int half) {
+#pragma unroll
+        for (int j = 0; j < kT; ++j)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const int i = half * kT + j;
+                m[u][i] = get(a.m, u, i);
+                nz[u][i] = get(a.nz, u, i);
+                if constexpr (kEpi == 2) mt[u][i] = get(a.mt, u, i);
+            }
+    };
+    if constexpr (kEpi == 1) {
+        if (kh == 0) draw();
+    }
+    if constexpr (kEpi != 0) load_half(0);
+    // the sum of group i, component u, of this wave (own) or its partner's groups
+    auto sum = [&](bool own, int u, int i, int e) {
+        const float first = acc[u][0][4 * i + e];
+        const float second = kT == 2 ? acc[u][kT - 1][4 * i + e] : acc[u][0][8 + 4 * i + e];
+        return (kh != 0) == own ? second : first;
+    };
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+        for (int i = 0; i < kGroups; ++i) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = sum(false, u, i, e);
+            red[wave][(u * kGroups + i) * 64 + l] = v;
+        }
+    __syncthreads();
+    const f32x4 *theirs = &red[kh ? wave - kPairs : wave + kPairs][l];
+    double ex = 0.0, ey = 0.0, ez = 0.0;
+    double msw = 0.0;
+    if constexpr (kEpi == 2) msw = n_rec > 0 ? a.msw[rk] : 0.0;
+#pragma unroll
+    for (int i = 0; i < kGroups; ++i) {
+        if constexpr (kEpi != 0)
+            if (i == kT - 1) load_half(1);
+        f32x4 h[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            h[u] = theirs[(u * kGroups + i) * 64];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[u][e] += sum(true, u, i, e);
+        }
+        if constexpr (kEpi == 0) {
+#pragma unroll
+            for (int u = 0; u < 3; ++u) put(a.h, u, i, h[u]);
+            continue;
+        }
+        f32x4 c[7], out[3];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) c[k] = constants[k][quad(i)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int p = 32 * kW * cb + 4 * quad(i) + e;
+            const ReplicaParticle cp{c[0][e], c[1][e], c[2][e], c[3][e], c[4][e], c[5][e], c[6][e]};
+            float x[3];
+            if constexpr (kEpi == 1) {
+                replica_stage1_math(a, cp, nz[0][i][e], nz[1][i][e], nz[2][i][e], hstage, h[0][e],
+                                    h[1][e], h[2][e], m[0][i][e], m[1][i][e], m[2][i][e], x[0],
+                                    x[1], x[2]);
+            } else {
+                replica_stage2_math(a, cp, nz[0][i][e], nz[1][i][e], nz[2][i][e], hstage, h[0][e],
+                                    h[1][e], h[2][e], mt[0][i][e], mt[1][i][e], mt[2][i][e],
+                                    m[0][i][e], m[1][i][e], m[2][i][e], x[0], x[1], x[2]);
+            }
+            const bool live = r < a.reps && p < a.n;
+            if constexpr (kEpi == 2) {
+                if (live) replica_check(a, r, p, x[0], x[1], x[2]);
+                if (n_rec > 0 && live) {
+                    ex += (double)x[0] * msw;
+                    ey += (double)x[1] * msw;
+                    ez += (double)x[2] * msw;
+                    if (a.samples != nullptr) {
+                        const size_t P = (size_t)a.n * a.reps, at = (size_t)r * a.n + p;
+                        for (int k = 0; k < n_rec; ++k) {
+                            float *base = a.samples + (size_t)(s_first + k) * 3 * P;
+                            base[at] = x[0];
+                            base[P + at] = x[1];
+                            base[2 * P + at] = x[2];
                         }
                     }
                 }
             }
-        };
-        Batch b0, b1;
-        load_batch(0, b0);
-        if (kh == 0) send_half(std::integral_constant<int, 8>{});
-        else send_half(std::integral_constant<int, 0>{});
-        __syncthreads();
-        // stage 1 holds both tiles' loads in flight; stage 2 loads twice as
-        // much per tile and issues the second tile's after the first
-        if constexpr (kEpi == 1) load_batch(1, b1);
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        using I8 = std::integral_constant<int, 8>;
-        if (kh == 0) finish_batch(I0{}, I0{}, b0);
-        else finish_batch(I8{}, I0{}, b0);
-        if constexpr (kEpi == 2) load_batch(1, b1);
-        if (kh == 0) finish_batch(I0{}, I1{}, b1);
-        else finish_batch(I8{}, I1{}, b1);
-        if constexpr (kEpi == 2) {
-            if (n_rec > 0 && ra.ens_partial != nullptr) {
-                wave_sum3<float>(ex, ey, ez);
-                if (l == 0) {
-                    const int wid = blockIdx.x * 8 + wave;
-                    for (int k = 0; k < n_rec; ++k) {
-                        double *dst = ra.ens_partial + (size_t)(s_first + k) * 3 * (size_t)ra.n_waves;
-                        dst[wid] = ex;
-                        dst[(size_t)ra.n_waves + wid] = ey;
-                        dst[2 * (size_t)ra.n_waves + wid] = ez;
-                    }
+            // the padding stays zero: it is an operand of the next product
+#pragma unroll
+            for (int u = 0; u < 3; ++u) out[u][e] = live ? x[u] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) put(kEpi == 1 ? a.mt : a.m, u, i, out[u]);
+    }
+    if constexpr (kEpi == 2) {
+        if (n_rec > 0 && a.ens_partial != nullptr) {
+            wave_sum3<float>(ex, ey, ez);
+            if constexpr (kT == 1) {   // one partial per 32 replicas x 32 particles
+                __shared__ double half[kPairs][3];
+                if (kh == 1 && l == 0) {
+                    half[w][0] = ex;
+                    half[w][1] = ey;
+                    half[w][2] = ez;
+                }
+                __syncthreads();
+                ex += half[w][0];
+                ey += half[w][1];
+                ez += half[w][2];
+            }
+            if (l == 0 && (kT == 2 || kh == 0)) {
+                const int wid = rt * (tiles / 3) + pb;
+                for (int k = 0; k < n_rec; ++k) {
+                    double *dst = a.ens_partial + (size_t)(s_first + k) * 3 * (size_t)a.n_waves;
+                    dst[wid] = ex;
+                    dst[(size_t)a.n_waves + wid] = ey;
+                    dst[2 * (size_t)a.n_waves + wid] = ez;
                 }
             }
         }
     }
 }
 
-// The same product in FP32 on MFMA (v_mfma_f32_32x32x2f32).  Each lane reads
-// four consecutive k of its rows per step of 8 and feeds them to four
-// instructions; A and B use the same k assignment, so the sum is complete.
-static __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__ a,
-                                                       const float *__restrict__ b,
-                                                       float *__restrict__ c, int K, int ldc)
-{
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int r0 = blockIdx.x * kGemmTile + (wave >> 1) * 64;
-    const int c0 = blockIdx.y * kGemmTile + (wave & 1) * 64;
-    const int lr = l & 31, kq = 4 * (l >> 5);
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[t][u][q] = 0.f;
-    const f32x4 *pa[2], *pb[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        pa[t] = reinterpret_cast<const f32x4 *>(a + (size_t)(r0 + 32 * t + lr) * K + kq);
-        pb[t] = reinterpret_cast<const f32x4 *>(b + (size_t)(c0 + 32 * t + lr) * K + kq);
-    }
-    for (int k = 0; k < K; k += 8) {
-        const int o = k / 4;
-        f32x4 xa[2], xb[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            xa[t] = pa[t][o];
-            xb[t] = pb[t][o];
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[t][q], xb[u][q], acc[t][u], 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) store_tile32(c, ldc, r0 + 32 * t, c0 + 32 * u, acc[t][u]);
-}
-
-// FP64 product on the VALU, one output per lane (reference for tests).
+// FP64 product on the VALU, one output per lane, of row-major matrices (reference
+// for tests).
 static __global__ void gemm_f64_kernel(const double *__restrict__ a, const double *__restrict__ b,
                                 double *__restrict__ c, int rows, int cols, int K)
 {
@@ -563,22 +509,37 @@ static __global__ void gemm_f64_kernel(const double *__restrict__ a, const doubl
     c[(size_t)r * cols + col] = s;
 }
 
-// The stages as elementwise kernels around an unfused product (FP32 MFMA
-// product): thread = (replica r, particle p), p fastest.
+// The stages as elementwise kernels around an unfused product: a thread per
+// (replica, particle), in the order of replica_at.
+struct ReplicaElement {
+    int r, p;
+    size_t at;     // of the x component; y and z are 1,024 and 2,048 further
+    bool live;
+    __device__ explicit ReplicaElement(const ReplicaArgs &a)
+    {
+        const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+        const int in = (int)(i & 1023), lane = (in >> 2) & 63, blocks = a.ld / 96;
+        const int tile = (int)(i >> 10), pb = tile % blocks;
+        r = 32 * (tile / blocks) + (lane & 31);
+        p = 32 * pb + 8 * (in >> 8) + 4 * (lane >> 5) + (in & 3);
+        at = ((size_t)(tile / blocks) * (size_t)(a.ld >> 5) + 3 * (size_t)pb) * 1024 + (size_t)in;
+        live = r < a.reps && p < a.n;
+    }
+};
+
 static __global__ __launch_bounds__(256) void replica_stage1_kernel(ReplicaArgs a, int64_t n_step, float h1)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n * a.reps) return;
-    const int r = i / a.n, p = i % a.n;
-    const size_t ox = (size_t)r * a.ld + replica_col(p, 0);
-    const ReplicaParticle c = replica_particle(a, p);
+    const ReplicaElement x(a);
+    if (!x.live) return;
+    const size_t y = x.at + 1024, z = x.at + 2048;
+    const ReplicaParticle c = replica_particle(a, x.p);
     float sx, sy, sz, tx, ty, tz;
-    replica_normals(a.key0[r], a.key1[r], a.tag, p, n_step, c.sig, sx, sy, sz);
-    replica_stage1_math(a, c, sx, sy, sz, h1, a.h[ox], a.h[ox + 32], a.h[ox + 64], a.m[ox],
-                        a.m[ox + 32], a.m[ox + 64], tx, ty, tz);
-    a.mt[ox] = tx;
-    a.mt[ox + 32] = ty;
-    a.mt[ox + 64] = tz;
+    replica_normals(a.key0[x.r], a.key1[x.r], a.tag, x.p, n_step, c.sig, sx, sy, sz);
+    replica_stage1_math(a, c, sx, sy, sz, h1, a.h[x.at], a.h[y], a.h[z], a.m[x.at], a.m[y], a.m[z],
+                        tx, ty, tz);
+    a.mt[x.at] = tx;
+    a.mt[y] = ty;
+    a.mt[z] = tz;
 }
 
 // stage 2 and the samples s_first .. s_first + n_rec - 1 (all recorded after
@@ -586,38 +547,40 @@ static __global__ __launch_bounds__(256) void replica_stage1_kernel(ReplicaArgs 
 static __global__ __launch_bounds__(256) void replica_stage2_kernel(ReplicaArgs a, int64_t n_step, float h2,
                                                              int64_t s_first, int n_rec)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = i < a.n * a.reps;
-    const int q = live ? i : a.n * a.reps - 1;
-    const int r = q / a.n, p = q % a.n;
-    const size_t ox = (size_t)r * a.ld + replica_col(p, 0);
+    const ReplicaElement x(a);
+    const size_t yy = x.at + 1024, zz = x.at + 2048;
+    const int p = x.live ? x.p : 0, r = x.live ? x.r : 0;
     const ReplicaParticle c = replica_particle(a, p);
     float sx, sy, sz, mx, my, mz;
     replica_normals(a.key0[r], a.key1[r], a.tag, p, n_step, c.sig, sx, sy, sz);
-    replica_stage2_math(a, c, sx, sy, sz, h2, a.h[ox], a.h[ox + 32], a.h[ox + 64], a.mt[ox],
-                        a.mt[ox + 32], a.mt[ox + 64], a.m[ox], a.m[ox + 32], a.m[ox + 64], mx, my,
-                        mz);
-    if (live) replica_store_state(a, r, p, ox, mx, my, mz);
+    replica_stage2_math(a, c, sx, sy, sz, h2, a.h[x.at], a.h[yy], a.h[zz], a.mt[x.at], a.mt[yy],
+                        a.mt[zz], a.m[x.at], a.m[yy], a.m[zz], mx, my, mz);
+    if (x.live) {
+        a.m[x.at] = mx;
+        a.m[yy] = my;
+        a.m[zz] = mz;
+        replica_check(a, r, p, mx, my, mz);
+    }
     for (int k = 0; k < n_rec; ++k) {
         const int64_t s = s_first + k;
-        if (a.samples != nullptr && live) {
-            const size_t P = (size_t)a.n * a.reps;
+        if (a.samples != nullptr && x.live) {
+            const size_t P = (size_t)a.n * a.reps, i = (size_t)r * a.n + p;
             float *base = a.samples + (size_t)s * 3 * P;
             base[i] = mx;
             base[P + i] = my;
             base[2 * P + i] = mz;
         }
         if (a.ens_partial != nullptr) {
-            double x = live ? (double)mx * a.msw[r] : 0.0;
-            double y = live ? (double)my * a.msw[r] : 0.0;
-            double z = live ? (double)mz * a.msw[r] : 0.0;
-            wave_sum3<float>(x, y, z);
+            double ex = x.live ? (double)mx * a.msw[r] : 0.0;
+            double ey = x.live ? (double)my * a.msw[r] : 0.0;
+            double ez = x.live ? (double)mz * a.msw[r] : 0.0;
+            wave_sum3<float>(ex, ey, ez);
             if ((threadIdx.x & (kWave - 1)) == 0) {
                 const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
                 double *dst = a.ens_partial + (size_t)s * 3 * (size_t)a.n_waves;
-                dst[wave] = x;
-                dst[(size_t)a.n_waves + wave] = y;
-                dst[2 * (size_t)a.n_waves + wave] = z;
+                dst[wave] = ex;
+                dst[(size_t)a.n_waves + wave] = ey;
+                dst[2 * (size_t)a.n_waves + wave] = ez;
             }
         }
     }
@@ -628,9 +591,9 @@ static __global__ __launch_bounds__(256) void replica_pack_kernel(ReplicaArgs a,
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n * a.reps) return;
-    const size_t ox = (size_t)(i / a.n) * a.ld + replica_col(i % a.n, 0);
+    const size_t at = replica_at(a.ld, i / a.n, replica_col(i % a.n, 0));
 #pragma unroll
-    for (int d = 0; d < 3; ++d) out[3 * (size_t)i + d] = a.m[ox + 32 * d];
+    for (int d = 0; d < 3; ++d) out[3 * (size_t)i + d] = a.m[at + 1024 * (size_t)d];
 }
 
 }  // namespace mp
