@@ -696,15 +696,15 @@ struct GroupRun : GroupBase {
         else launch_cluster_lanes<1, false>(s, htab);
     }
 
-    // Partners whose geometry the two-lane FP32 kernel caches per lane (in
-    // workgroups of at most 256 lanes): 16, or 0 with MAGPY_AMD_CLUSTER_CACHE=0.
-    // Results do not depend on it.
+    // Partners whose geometry the two-lane kernel caches per lane (in workgroups of
+    // at most 256 lanes): 16 in FP32 and 8 in FP64, or 0 with
+    // MAGPY_AMD_CLUSTER_CACHE=0.  Results do not depend on it.
     int cluster_cache() const
     {
-        if (sizeof(T) != 4 || lanes != 2 || block > 256 || array_noise) return 0;
+        if (lanes != 2 || block > 256 || array_noise) return 0;
         if (const char *env = std::getenv("MAGPY_AMD_CLUSTER_CACHE"))
             if (std::atoi(env) == 0) return 0;
-        return 16;
+        return sizeof(T) == 4 ? 16 : 8;
     }
 
     template <bool kArray>
@@ -743,8 +743,14 @@ struct GroupRun : GroupBase {
     template <int L, bool kArray>
     void launch_cluster_lanes(hipStream_t s, const float *htab)
     {
+        if constexpr (L == 2 && !kArray && sizeof(T) == 8) {
+            if (cluster_cache() != 0) {
+                launch_cluster_variant<L, kArray, 8, 0>(s, htab);
+                return;
+            }
+        }
         if constexpr (L == 2 && !kArray && sizeof(T) == 4) {
-            if (cluster_cache() == 16) {
+            if (cluster_cache() != 0) {
                 if (cluster_lds_cache()) launch_cluster_variant<L, kArray, 16, 16>(s, htab);
                 else launch_cluster_variant<L, kArray, 16, 0>(s, htab);
                 return;

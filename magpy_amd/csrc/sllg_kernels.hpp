@@ -287,6 +287,46 @@ __device__ inline void group_normals(int64_t g, uint32_t pid, uint32_t tag, cons
     }
 }
 
+// The value of the even (kOdd = 0) or odd lane of the caller's pair of lanes
+template <int kOdd>
+__device__ inline double of_pair(double v)
+{
+    constexpr int kPerm = kOdd ? 0xf5 : 0xa0;   // quad_perm 1133, 0022
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), kPerm, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), kPerm, 0xf, 0xf, true));
+}
+
+// group_normals where the two lanes of a pair (half 0 and 1) want the same twelve:
+// each draws six, from the first (second) half of the three Philox calls, and the
+// lanes exchange them.  All lanes of the wave call it together.  FP64 only: in FP32,
+// where a pair of normals is 25 instructions, the exchange ties the draws to the
+// step chain and costs more than it saves (4,096 clusters: 13.1 -> 15.0 ms).
+__device__ inline void shared_normals(int64_t g, int half, uint32_t pid, uint32_t tag,
+                                      const PhiloxKeys &keys, double sig, double z[12])
+{
+    const uint64_t outer = (uint64_t)(3 * g + 2 * half), middle = (uint64_t)(3 * g + 1);
+    const u32x4 w = philox4x32_10(u32x4{(uint32_t)outer, (uint32_t)(outer >> 32), pid, tag}, keys);
+    const u32x4 v =
+        philox4x32_10(u32x4{(uint32_t)middle, (uint32_t)(middle >> 32), pid, tag}, keys);
+    const uint32_t v0 = half ? v.z : v.x, v1 = half ? v.w : v.y;
+    double own[6];
+    Num<double>::box_muller(w.x, w.y, own[0], own[1]);
+    Num<double>::box_muller(w.z, w.w, own[2], own[3]);
+    Num<double>::box_muller(v0, v1, own[4], own[5]);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) own[i] *= sig;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z[i] = of_pair<0>(own[i]);
+        z[8 + i] = of_pair<1>(own[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        z[4 + i] = of_pair<0>(own[4 + i]);
+        z[6 + i] = of_pair<1>(own[4 + i]);
+    }
+}
+
 // One block of steps [n0, n1) for independent particles.  Steps are walked in
 // groups of four, whose twelve normals come from three Philox calls.  The
 // state chain of one step depends on the previous step, so with one wave per
@@ -698,6 +738,13 @@ struct alignas(16) Vec4 {
     T x, y, z, w;
 };
 
+template <typename T>
+__device__ inline T rsqrt_pair(T r2)
+{
+    if constexpr (sizeof(T) == 4) return __builtin_amdgcn_rsqf(r2);
+    else return rsqrt_normal(r2);
+}
+
 // One dipolar pair term: the field at pi of the moment mj (weight pj.w) at
 // pj, added to (ax, ay, az); `skip` masks the particle's own lane.
 template <typename T>
@@ -707,9 +754,7 @@ __device__ inline void dipolar_term(const Vec4<T> &pi, const Vec4<T> &pj, const 
 #pragma clang fp contract(off)
     const T dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
     const T r2 = skip ? T(1) : fmad(dx, dx, fmad(dy, dy, dz * dz));
-    T rinv;
-    if constexpr (sizeof(T) == 4) rinv = __builtin_amdgcn_rsqf(r2);
-    else rinv = rsqrt_normal(r2);
+    const T rinv = rsqrt_pair(r2);
     const T rinv2 = rinv * rinv;
     const T c = skip ? T(0) : pj.w * rinv2 * rinv;
     const T t = T(3) * fmad(mj.x, dx, fmad(mj.y, dy, mj.z * dz)) * rinv2;
@@ -798,7 +843,7 @@ __device__ inline void pair_cache_init(const Vec4<T> *pos, int self, int jb, int
         const bool skip = !in || j == self;
         const T dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
         const T r2 = skip ? T(1) : fmad(dx, dx, fmad(dy, dy, dz * dz));
-        const T rinv = __builtin_amdgcn_rsqf(r2);
+        const T rinv = rsqrt_pair(r2);
         const T rinv2 = rinv * rinv;
         pc.dx[k] = skip ? T(0) : dx;
         pc.dy[k] = skip ? T(0) : dy;
@@ -882,9 +927,9 @@ __device__ inline void dipolar_field_cached(const Vec4<T> *pos, const Vec4<T> *m
             for (int u = 0; u < 2; ++u) {
                 const T dx = pj[u].x - pi.x, dy = pj[u].y - pi.y, dz = pj[u].z - pi.z;
                 const T t = T(3) * fmad(mj[u].x, dx, fmad(mj[u].y, dy, mj[u].z * dz)) * g[u].y;
-                x = fmad(g[u].x, fmad(t, dx, -mj[u].x), x);
-                y = fmad(g[u].x, fmad(t, dy, -mj[u].y), y);
-                z = fmad(g[u].x, fmad(t, dz, -mj[u].z), z);
+                x = fmad(T(g[u].x), fmad(t, dx, -mj[u].x), x);
+                y = fmad(T(g[u].x), fmad(t, dy, -mj[u].y), y);
+                z = fmad(T(g[u].x), fmad(t, dz, -mj[u].z), z);
             }
         }
     }
@@ -910,10 +955,15 @@ __device__ inline void dipolar_field_cached(const Vec4<T> *pos, const Vec4<T> *m
 // the even lane alone writes the shared state, samples and results.  With
 // kArrayNoise the Wiener normals are the caller's ([step][slot][3], the
 // reference's RngArray, lib/rng.cpp:67-94) instead of the Philox stream.
-// kCache (two lanes, FP32) caches the first kCache partners' geometry per
-// lane (PairCache): workgroups of at most 256 lanes then, for the registers;
-// kLds more partners keep their weights in LDS after the three state arrays
-// (kLds x lanes float2).
+// kCache (two lanes) caches the first kCache partners' geometry per lane
+// (PairCache): workgroups of at most 256 lanes then, for the registers; kLds more
+// partners (FP32) keep their weights in LDS after the three state arrays (kLds x
+// lanes float2).  In FP64 the two lanes also draw half of the normals each.
+// Ensembles that run with two lanes have few waves: a SIMD's time is the
+// instructions of one or two, of which a FP64 pair term computed anew takes some 45
+// and from the cache 10, and a bound of 256 lanes leaves room for 512 registers (at
+// 1,024 it spilled).  FP64, 600 clusters of 2-12, 1,000 steps: 3.4 -> 1.6 ms; of 2-64,
+// 400 steps: 3.6 -> 2.6.
 template <typename T, int kShape, bool kTable, bool kRenorm, int kLanes, bool kArrayNoise,
           int kCache = 0, int kLds = 0>
 __global__ __launch_bounds__(kCache > 0 ? 256 : 1024, kLds > 0 ? 2 : 1) void heun_cluster_kernel(
@@ -948,8 +998,8 @@ __global__ __launch_bounds__(kCache > 0 ? 256 : 1024, kLds > 0 ? 2 : 1) void heu
     const int64_t n0 = a.n0, n1 = a.n1;
     const int64_t tab0 = 4 * (n0 >> 2);
     if (lead) pos[tid] = Vec4<T>{ca.px[p], ca.py[p], ca.pz[p], ca.w[p]};
-    static_assert(kCache == 0 || (kLanes == 2 && sizeof(T) == 4), "cache: two lanes, FP32");
-    static_assert(kLds == 0 || kCache > 0, "LDS partners follow the register-cached ones");
+    static_assert(kCache == 0 || kLanes == 2, "cache: two lanes");
+    static_assert(kLds == 0 || (kCache > 0 && sizeof(T) == 4), "LDS partners follow the register-cached ones");
     PairCache<T, (kCache > 0 ? kCache : 4)> pc;
     float2 *geo = reinterpret_cast<float2 *>(mb1 + slots) + threadIdx.x;
     if constexpr (kCache > 0) {
@@ -964,9 +1014,13 @@ __global__ __launch_bounds__(kCache > 0 ? 256 : 1024, kLds > 0 ? 2 : 1) void heu
     // the normals of step group g+1 are drawn while group g is integrated
     T zc[12], zn[12];
     const int64_t g_begin = n0 >> 2, g_end = (n1 + 3) >> 2;
-    if constexpr (!kArrayNoise) group_normals(g_begin, pid, a.tag, keys, sig, zc);
+    auto draw = [&](int64_t g, T z[12]) {
+        if constexpr (kLanes == 2 && sizeof(T) == 8) shared_normals(g, half, pid, a.tag, keys, sig, z);
+        else group_normals(g, pid, a.tag, keys, sig, z);
+    };
+    if constexpr (!kArrayNoise) draw(g_begin, zc);
     for (int64_t g = g_begin; g < g_end; ++g) {
-        if constexpr (!kArrayNoise) group_normals(g + 1, pid, a.tag, keys, sig, zn);
+        if constexpr (!kArrayNoise) draw(g + 1, zn);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int64_t n = 4 * g + u;
