@@ -102,15 +102,18 @@ int64_t env_steps_per_launch()
 }
 
 // Length of the segments whose maps are computed in parallel: the checkpoint
-// interval, or the smallest whole part of it that is a multiple of 4 steps and at
-// least 200.  Short segments give small ensembles more lanes (300 particles,
-// 20,000 steps: 4.6 -> 3.7 ms) and let the maps' waves, some of which share a SIMD
-// with a forward wave, even out; each costs a transfer of 168 bytes per particle.
-// Above 2^16 particles one segment of every particle fills the card, and the states
-// kept for shorter ones (two blocks of up to 2^16 steps) would take over 1 GiB.
-int64_t segment_steps(int64_t particles, int64_t checkpoint_interval)
+// interval, or in FP64 the smallest whole part of it that is a multiple of 4 steps and
+// at least 200.  Short segments give small ensembles more lanes and let the maps'
+// waves, some of which share a SIMD with a forward wave, even out (3,000 particles,
+// FP64, 20,000 steps: 9.8 -> 8.1 ms); each costs a transfer of 168 bytes per particle.
+// Not in FP32 (16,384 particles: 8.5 -> 7.1): a map starts at the identity, where each
+// step's small change is rounded to the last place of one, and the gradient was 1.8
+// times as far from FP64.  Above 2^16 particles one segment of every particle fills
+// the card, and the states kept for shorter ones (two blocks of up to 2^16 steps)
+// would take over 1 GiB.
+int64_t segment_steps(int64_t particles, int64_t checkpoint_interval, bool fp64)
 {
-    if (particles > (int64_t)1 << 16) return checkpoint_interval;
+    if (!fp64 || particles > (int64_t)1 << 16) return checkpoint_interval;
     const int64_t groups = checkpoint_interval / 4;
     for (int64_t parts = groups; parts > 1; --parts)
         if (groups % parts == 0 && checkpoint_interval / parts >= 200)
@@ -119,15 +122,17 @@ int64_t segment_steps(int64_t particles, int64_t checkpoint_interval)
 }
 
 // Segments of C steps per forward launch: about 2^16 steps.  A run of fewer than
-// eight such blocks is cut into eight, so that the maps of one block overlap the
-// forward steps of the next, as long as a block's maps (a lane per segment and
-// particle) keep three waves on each SIMD of the card.
-int64_t block_segments(int64_t particles, int64_t segments, int64_t C)
+// eight (FP32: four) such blocks is cut into as many, so that the maps of one block
+// overlap the forward steps of the next, as long as a block's maps (a lane per segment
+// and particle) keep three (two) waves on each SIMD of the card.  Long FP32 segments
+// fill the card less evenly in small blocks: 9.5 ms in eight, 8.5 in four.
+int64_t block_segments(int64_t particles, int64_t segments, int64_t C, bool fp64)
 {
     if (const int64_t env = env_steps_per_launch()) return std::max<int64_t>(1, env / C);
     const int64_t most = std::max<int64_t>(1, ((int64_t)1 << 16) / C);
-    const int64_t fill = (3 * ((int64_t)1 << 16) + particles - 1) / particles;
-    return std::min(most, std::max((segments + 7) / 8, fill));
+    const int64_t blocks = fp64 ? 8 : 4, waves = fp64 ? 3 : 2;
+    const int64_t fill = (waves * ((int64_t)1 << 16) + particles - 1) / particles;
+    return std::min(most, std::max((segments + blocks - 1) / blocks, fill));
 }
 
 // lanes (segment x particle) per adjoint-map launch
@@ -228,10 +233,10 @@ struct AdjointRun final : AdjointBase {
         device = s.device;
         P = sp.n_particles;
         N = sp.n_steps;
-        C = segment_steps(P, sp.checkpoint_interval);
+        C = segment_steps(P, sp.checkpoint_interval, sizeof(T) == 8);
         S = sp.n_samples;
         n_ck = (N + C - 1) / C;
-        segs_per_block = block_segments(P, n_ck, C);
+        segs_per_block = block_segments(P, n_ck, C, sizeof(T) == 8);
         spl = segs_per_block * C;
         shape.assign(sp.radius_shape, sp.radius_shape + P);
         m0.assign(sp.magnetisation_direction, sp.magnetisation_direction + 3 * P);

@@ -395,8 +395,8 @@ struct TransferArgs {
 // its states and normals are in registers.  Keeping every step's state and
 // normals instead (24 bytes per step, written and read back through HBM) waited
 // on those reads.  Bound: VALU issue, ~640 instructions per step.  16,384
-// particles, FP32: 20,000 steps 10.8 -> 7.1 ms with the forward pass, 200,000
-// steps 84 -> 57.8 ms; 3,000 particles, FP64, 20,000 steps: 24.2 -> 8.1 ms.
+// particles, FP32: 20,000 steps 10.9 -> 8.6 ms with the forward pass, 200,000
+// steps 85 -> 63.8 ms; 3,000 particles, FP64, 20,000 steps: 24.2 -> 8.1 ms.
 // The next group's state and field values load while a group is worked on.
 // Registers: three waves per SIMD in FP32 (168; four spill: 4.05 against 3.16
 // ms per 163,840 lanes and 1,000 steps), two in FP64.
