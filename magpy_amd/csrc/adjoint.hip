@@ -279,6 +279,7 @@ struct AdjointRun final : AdjointBase {
             k1[p] = (uint32_t)(sd >> 32);
         }
         MP_HIP(hipSetDevice(device));
+        UploadScope uploads;
         ex.upload(hx);
         ey.upload(hy);
         ez.upload(hz);
@@ -306,6 +307,7 @@ struct AdjointRun final : AdjointBase {
         d_piece_start.upload(pt.start);
         d_piece_new.upload(pt.is_new);
         d_piece_iv.upload(pt.iv);
+        uploads.flush();
         inj.alloc(pt.bounds.size());
     }
 
