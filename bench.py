@@ -530,7 +530,7 @@ def library_gemm(args):
         out[name + "_tflops"] = 2.0 * M * N * K / us / 1e6
     # this library's BF16x3 product of the replica workload (4,096 states of
     # the 512-particle cluster), 10 calls: each uploads its operands, so only
-    # a kernel trace times the product itself (gemm_bf16x3_ksplit_kernel<0>)
+    # a kernel trace times the product itself (replica_product_kernel, epilogue 0)
     import magpy_amd
     inp = replica_inputs(M)
     n = 512

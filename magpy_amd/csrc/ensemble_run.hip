@@ -989,7 +989,7 @@ bool replica_fused()
 //   1,000 x 64   24.0   14.5  9.8  6.4      4,096 x 256  51.7  31.7  28.8  25.7
 //   64 x 400     58.7   42.1  22.3  13.9    2,048 x 512  74.4  51.6  45.0  43.0
 //   1,024 x 256  37.1   28.1  16.7  10.3    3,900 x 450  86.0    -   68.5  94.7
-//   4,096 x 512  92.4 (72.7 us a product)  70.9 (61 and 66 us), 75.5, -
+//   4,096 x 512  92.4  70.9  75.5  -  (with the state's copy: 70.7 -> 63.8 us a product)
 void launch_product(int mode, int epi, const float *state, const float *tensor,
                     const mp::ReplicaArgs &a, int rows, int cus, int64_t step, float hstage,
                     int64_t s_first, int n_rec, hipStream_t s)

@@ -220,7 +220,8 @@ __device__ inline void replica_check(const ReplicaArgs &a, int r, int p, float m
 // with both operands staged through LDS 61.4, the tensor alone 57.6, three steps
 // ahead 56.9, one wave per SIMD with twice the tile 53.1 (but then nothing draws
 // beside it, and the stages take longer alone).  With stage 1 61 us and with stage 2
-// 66 (both 72.7 with the operands through LDS and 4-byte accesses).
+// 66 in a trace; in a run 63.8 on average (70.7 with the operands through LDS and
+// 4-byte accesses).
 enum ReplicaMode { kReplicaBf16x3, kReplicaF32 };
 
 template <int kMode, int kT>
