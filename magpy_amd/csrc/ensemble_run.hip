@@ -212,11 +212,10 @@ struct SampleSink {
     const Plan &plan;
     const HostCopy &host;
 
-    // Samples of every slot from the records src [records][3][n]; slot_particle[i]
-    // is the particle (-1: padding) and record(i, s) the record of its sample s.
-    // Tiles of particles and samples keep both sides in cache.
-    template <typename T, typename Record>
-    void take(const T *src, const std::vector<int64_t> &slot_particle, Record record) const
+    // Samples of every slot from src [S][3][n]; slot_particle[i] is the particle
+    // (-1: padding).  Tiles of particles and samples keep both sides in cache.
+    template <typename T>
+    void take(const T *src, const std::vector<int64_t> &slot_particle) const
     {
         constexpr int64_t kTile = 16;
         const int64_t n = (int64_t)slot_particle.size(), S = host.S;
@@ -231,7 +230,7 @@ struct SampleSink {
                     const std::vector<int64_t> &k = plan.sched[(size_t)plan.group_of[(size_t)m]];
                     for (int64_t sa = s0; sa < std::min(S, s0 + kTile); ++sa) {
                         const int64_t at = k[(size_t)sa];
-                        const T *row = at > host.start ? src + record(i, sa) * 3 * n + i : nullptr;
+                        const T *row = at > host.start ? src + sa * 3 * n + i : nullptr;
                         for (int d = 0; d < 3; ++d) {
                             if (!dst[d]) continue;
                             const double v = row != nullptr       ? (double)row[d * n]
@@ -251,6 +250,10 @@ struct GroupBase {
     virtual void state(double *out) = 0;               // its particles' rows of [P][3]
     virtual const std::vector<int64_t> &slots() const = 0;
     virtual const std::vector<int> &set() const = 0;   // its schedule groups
+    // Device memory for one launch's records, which the sets of a run share: each
+    // launch's records are taken from it before the next launch of any set
+    virtual size_t record_bytes() const { return 0; }
+    virtual void use_records(void *) {}
     virtual GroupOut collect(hipStream_t s, double *state_out, const SampleSink *samples) = 0;
 };
 
@@ -371,7 +374,9 @@ std::vector<int64_t> union_schedule(const Plan &plan, const std::vector<int> &se
 // can have a schedule group per member: one launch of one particle after the
 // other (300 members, 2,000 FP64 steps: 178 ms).  A launch set records the union
 // of its groups' sample steps, which differ by a step here and there, and each
-// member's samples are picked from it.  Sets hold groups of equal step count whose
+// member's samples (and each group's sums) are picked from it after each launch, so
+// that a run keeps its samples as it would with a launch per group, and the records
+// of one set beside them.  Sets hold groups of equal step count whose
 // kernels run the same code for them: FP64 and the implicit scheme, whose lanes
 // all evaluate their own field; FP32 constant fields; and FP32 groups of
 // independent particles that read their field from a table, as many rows of it.
@@ -440,6 +445,8 @@ struct GroupRun : GroupBase {
     // The schedule groups of this launch set.  With several, the kernels record
     // the union of their sample steps (S of them, S_out samples per group) and
     // pick[g][s] is the record of group g's sample s (-1: at or before the start).
+    // take_records keeps of them what the run asked for: the samples, in d_samples
+    // as a single group's, and a sum per sample and group, in d_partial.
     std::vector<int> groups;
     int64_t S = 0, S_out = 0, s_next = 0, spl = 1;
     std::vector<int64_t> sched, slot_particle;
@@ -459,6 +466,8 @@ struct GroupRun : GroupBase {
     int64_t tab_stride = 0;
     DevBuf<int64_t> d_toff;                   // per slot: start of its row (several rows)
     DevBuf<int32_t> d_pick, d_slot_group;
+    DevBuf<int32_t> d_group_slots, d_group_first;   // the slots of each group
+    T *records = nullptr;
     mp::IndepArgs<T> a{};
 
     // cluster_block == 0: one slot per particle of the group (independent
@@ -631,19 +640,34 @@ struct GroupRun : GroupBase {
                        : 0;
         // the one-wave kernel reads one table row
         if (several && uniform_field) two_wave = std::max(two_wave, 1);
-        if (want_traj || (several && want_ens)) d_samples.alloc((size_t)S * 3 * (size_t)n);
+        if (want_traj) d_samples.alloc((size_t)S_out * 3 * (size_t)n);
         if (want_ens) {
             // each recorded sample writes all of its (component, wave) slots;
             // slots of samples taken at step 0 are replaced on the host.  Several
-            // schedules: the sums are taken from the samples
-            if (!several) d_partial.alloc((size_t)S * 3 * (size_t)n_waves);
+            // schedules: a slot per group, zero where the group took no sample
+            d_partial.alloc((size_t)S_out * 3 * (several ? set.size() : (size_t)n_waves));
             d_ens.alloc((size_t)S_out * 3);
             if (several) {
-                std::vector<int32_t> flat;
-                for (const auto &row : pick) flat.insert(flat.end(), row.begin(), row.end());
-                d_pick.upload(flat);
-                d_slot_group.upload(std::vector<int32_t>(slot_group.begin(), slot_group.end()));
+                MP_HIP(hipMemset(d_partial.p, 0, d_partial.n * sizeof(double)));
+                MP_HIP(hipStreamSynchronize(nullptr));
+                std::vector<int32_t> first(set.size() + 1, 0), slots;
+                for (int g : slot_group)
+                    if (g >= 0) ++first[(size_t)g + 1];
+                for (size_t g = 0; g < set.size(); ++g) first[g + 1] += first[g];
+                slots.resize((size_t)first.back());
+                std::vector<int32_t> at(first.begin(), first.end() - 1);
+                for (int i = 0; i < n; ++i)
+                    if (slot_group[(size_t)i] >= 0)
+                        slots[(size_t)at[(size_t)slot_group[(size_t)i]]++] = i;
+                d_group_first.upload(first);
+                d_group_slots.upload(slots);
             }
+        }
+        if (several && (want_traj || want_ens)) {
+            std::vector<int32_t> flat;
+            for (const auto &row : pick) flat.insert(flat.end(), row.begin(), row.end());
+            d_pick.upload(flat);
+            d_slot_group.upload(std::vector<int32_t>(slot_group.begin(), slot_group.end()));
         }
         if (array_noise) {
             std::vector<double> nz((size_t)n_total * (size_t)n * 3, 0.0);
@@ -668,8 +692,8 @@ struct GroupRun : GroupBase {
         a.status = d_status.p;
         a.sched = d_sched.p;
         a.S = S;
-        a.samples = d_samples.p;
-        a.ens_partial = d_partial.p;
+        a.samples = several ? nullptr : d_samples.p;   // several: use_records
+        a.ens_partial = several ? nullptr : d_partial.p;
         a.tag = sp.noise_tag;
         a.renorm = sp.renorm ? 1 : 0;
         a.noise = array_noise ? d_noise.p : nullptr;
@@ -678,6 +702,53 @@ struct GroupRun : GroupBase {
 
     const std::vector<int64_t> &slots() const override { return slot_particle; }
     const std::vector<int> &set() const override { return groups; }
+
+    size_t record_bytes() const override
+    {
+        return groups.size() > 1 && (want_traj || want_ens) ? (size_t)S * 3 * (size_t)n * sizeof(T)
+                                                            : 0;
+    }
+    void use_records(void *p) override
+    {
+        if (record_bytes() == 0) return;
+        records = static_cast<T *>(p);
+        a.samples = records;
+    }
+
+    // The samples and sums of the records that a launch of the steps up to n1 wrote:
+    // those from s_next on.  A group takes a sample at one step, so that its sum has
+    // all its terms here and does not depend on how a run is cut into launches.
+    void take_records(int64_t n1, hipStream_t s)
+    {
+        const int32_t first = (int32_t)s_next,
+                      end = (int32_t)(std::upper_bound(sched.begin() + s_next, sched.end(), n1) -
+                                      sched.begin());
+        if (first == end) return;
+        int64_t lo = S_out, hi = 0;   // the samples that any group has there
+        for (const auto &row : pick) {
+            lo = std::min<int64_t>(lo, std::lower_bound(row.begin(), row.end(), first) - row.begin());
+            hi = std::max<int64_t>(hi, std::lower_bound(row.begin(), row.end(), end) - row.begin());
+        }
+        if (lo >= hi) return;
+        const int64_t G = (int64_t)groups.size(), most = 16 * (int64_t)device_cus();
+        auto blocks = [&](int64_t threads) {
+            return dim3((unsigned)std::min((threads + mp::kBlock - 1) / mp::kBlock, most));
+        };
+        const mp::RecordArgs<T> r{records, d_pick.p, n, S_out, lo, hi, first, end};
+        if (want_traj) {
+            hipLaunchKernelGGL(mp::pick_samples_kernel<T>, blocks((hi - lo) * n), dim3(mp::kBlock), 0,
+                               s, r, d_slot_group.p, d_samples.p);
+            MP_HIP(hipGetLastError());
+        }
+        if (want_ens) {
+            int team = 1;   // lanes per sum: the slots of a group on average, to a wave
+            while (team < mp::kWave && team * G < (int64_t)d_group_slots.n) team *= 2;
+            hipLaunchKernelGGL(mp::group_sums_kernel<T>, blocks((hi - lo) * G * team),
+                               dim3(mp::kBlock), 0, s, r, d_group_slots.p, d_group_first.p, (int)G,
+                               team, d_msw.p, d_partial.p);
+            MP_HIP(hipGetLastError());
+        }
+    }
 
     unsigned long long *newton_iters() const { return d_newton.p; }
     unsigned long long *newton_fails() const { return d_newton.p ? d_newton.p + n : nullptr; }
@@ -833,6 +904,7 @@ struct GroupRun : GroupBase {
                 launch_shape<T, false>(shape_kind, a, scheme, eps, max_iter, newton_iters(), newton_fails(), grid, s,
                                        htab, two_wave);
             MP_HIP(hipGetLastError());
+            if (records != nullptr) take_records(n1, s);
             ++launches;
             n_done = n1;
         }
@@ -852,15 +924,10 @@ struct GroupRun : GroupBase {
     GroupOut collect(hipStream_t s, double *state_out, const SampleSink *sink) override
     {
         GroupOut o;
-        const bool several = groups.size() > 1;
         if (want_ens) {
-            if (several)
-                hipLaunchKernelGGL(mp::ens_pick_kernel<T>, dim3((unsigned)(S_out * 3)),
-                                   dim3(mp::kBlock), 0, s, d_samples.p, d_pick.p, d_slot_group.p,
-                                   d_msw.p, n, (int)S_out, d_ens.p);
-            else
-                hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)),
-                                   dim3(mp::kBlock), 0, s, d_partial.p, n_waves, S * 3, d_ens.p);
+            const int parts = groups.size() > 1 ? (int)groups.size() : n_waves;
+            hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S_out * 3)), dim3(mp::kBlock),
+                               0, s, d_partial.p, parts, S_out * 3, d_ens.p);
             MP_HIP(hipGetLastError());
         }
         MP_HIP(hipStreamSynchronize(s));
@@ -881,12 +948,7 @@ struct GroupRun : GroupBase {
             if (d_samples.n)
                 MP_HIP(hipMemcpy(h.get(), d_samples.p, d_samples.n * sizeof(T),
                                  hipMemcpyDeviceToHost));
-            if (several)
-                sink->take(h.get(), slot_particle, [&](int64_t i, int64_t sa) {
-                    return (int64_t)pick[(size_t)slot_group[(size_t)i]][(size_t)sa];
-                });
-            else
-                sink->take(h.get(), slot_particle, [](int64_t, int64_t sa) { return sa; });
+            sink->take(h.get(), slot_particle);
         }
         if (want_ens) {
             o.ens.resize((size_t)S_out * 3);
@@ -1214,7 +1276,7 @@ struct ReplicaRun : GroupBase {
             if (d_samples.n)
                 MP_HIP(hipMemcpy(h.get(), d_samples.p, d_samples.n * sizeof(float),
                                  hipMemcpyDeviceToHost));
-            sink->take(h.get(), slot_particle, [](int64_t, int64_t sa) { return sa; });
+            sink->take(h.get(), slot_particle);
         }
         if (want_ens) {
             o.ens.resize((size_t)S * 3);
@@ -1255,6 +1317,7 @@ struct mp_session {
     Plan plan;
     HostCopy host;
     std::vector<std::unique_ptr<GroupBase>> groups;
+    DevBuf<char> records;   // shared by the launch sets of several schedules
     StreamGuard sg;
     // own_stream false: launches go to the null stream and nothing is created
     explicit mp_session(bool own_stream = true) : sg(own_stream) {}
@@ -1659,6 +1722,10 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
                 new GroupRun<double>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
     }
     uploads.flush();
+    size_t record_bytes = 0;
+    for (auto &g : ss->groups) record_bytes = std::max(record_bytes, g->record_bytes());
+    ss->records.alloc(record_bytes);
+    for (auto &g : ss->groups) g->use_records(ss->records.p);
     return ss.release();
 }
 

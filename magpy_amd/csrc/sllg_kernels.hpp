@@ -1745,31 +1745,70 @@ static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int
     if (threadIdx.x == 0) out[r] = buf[0];
 }
 
-// Ensemble sums of a launch set of several schedules: out[s][c] = sum over slots
-// of Ms m, each slot's sample s being record pick[group][s] (-1: none), in a
-// fixed order.  Bound by the read of the records once.
+// Of a launch set of several schedules: the records [first, end) that a launch has
+// just written, records[u][component][slot]; pick[group][s] is the record of the
+// group's sample s (-1: none), and samples [lo, hi) are those that any group has there.
 template <typename T>
-static __global__ __launch_bounds__(kBlock) void ens_pick_kernel(const T *samples,
-                                                                 const int32_t *pick,
-                                                                 const int32_t *slot_group,
-                                                                 const double *msw, int n, int S,
-                                                                 double *out)
+struct RecordArgs {
+    const T *records;
+    const int32_t *pick;
+    int n;
+    int64_t S, lo, hi;
+    int32_t first, end;
+};
+
+// samples[s][component][slot] of every slot whose sample s is one of the records.
+// Bound by its reads and writes, 48 bytes (FP64) a sample and slot.
+template <typename T>
+static __global__ __launch_bounds__(kBlock) void pick_samples_kernel(RecordArgs<T> a,
+                                                                     const int32_t *slot_group,
+                                                                     T *samples)
 {
-    const int s = blockIdx.x / 3, c = blockIdx.x % 3;
-    __shared__ double buf[kBlock];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += kBlock) {
+    const size_t n = (size_t)a.n, total = (size_t)(a.hi - a.lo) * n;
+    for (size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x; t < total;
+         t += (size_t)gridDim.x * kBlock) {
+        const size_t s = (size_t)a.lo + t / n, i = t % n;
         const int g = slot_group[i];
-        const int u = g < 0 ? -1 : pick[(size_t)g * S + s];
-        if (u >= 0) acc += (double)samples[((size_t)u * 3 + c) * (size_t)n + i] * msw[i];
+        if (g < 0) continue;
+        const int32_t u = a.pick[(size_t)g * (size_t)a.S + s];
+        if (u < a.first || u >= a.end) continue;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) samples[(s * 3 + c) * n + i] = a.records[((size_t)u * 3 + c) * n + i];
     }
-    buf[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) buf[threadIdx.x] += buf[threadIdx.x + w];
-        __syncthreads();
+}
+
+// partial[s][component][group] = sum of Ms m over the group's slots
+// slots[first_slot[g] .. first_slot[g + 1]) for every sample s of the group that is
+// one of the records, by `team` (a power of two up to 64) lanes each, in a fixed order.
+template <typename T>
+static __global__ __launch_bounds__(kBlock) void group_sums_kernel(RecordArgs<T> a,
+                                                                   const int32_t *slots,
+                                                                   const int32_t *first_slot, int G,
+                                                                   int team, const double *msw,
+                                                                   double *partial)
+{
+    const size_t n = (size_t)a.n, total = (size_t)(a.hi - a.lo) * (size_t)G;
+    const int lane = threadIdx.x & (team - 1);
+    for (size_t t = ((size_t)blockIdx.x * kBlock + threadIdx.x) / team; t < total;
+         t += (size_t)gridDim.x * kBlock / team) {
+        const size_t s = (size_t)a.lo + t / (size_t)G, g = t % (size_t)G;
+        const int32_t u = a.pick[g * (size_t)a.S + s];
+        if (u < a.first || u >= a.end) continue;
+        const T *row = a.records + (size_t)u * 3 * n;
+        double sum[3] = {0.0, 0.0, 0.0};
+        for (int k = first_slot[g] + lane; k < first_slot[g + 1]; k += team) {
+            const size_t i = (size_t)slots[k];
+            const double w = msw[i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sum[c] += (double)row[c * n + i] * w;
+        }
+        for (int x = team / 2; x > 0; x /= 2)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sum[c] += __shfl_xor(sum[c], x);
+        if (lane == 0)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) partial[(s * 3 + c) * (size_t)G + g] = sum[c];
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = buf[0];
 }
 
 // normals j0 .. j0+n-1 of one particle's stream, one lane per normal
