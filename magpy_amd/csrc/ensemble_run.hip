@@ -26,6 +26,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "cluster_layout.hpp"
 #include "host_util.hpp"
 #include "simulation.hpp"
 #include "replica_kernels.hpp"
@@ -1434,13 +1435,6 @@ void validate(const EnsembleSpec &sp)
 
 namespace {
 
-// Layout of the interacting-cluster kernel: `block` lanes per workgroup and
-// `lanes` (1 or 2) lanes per particle slot, so a workgroup holds
-// block / lanes slots, which must take the largest cluster.
-struct ClusterLayout {
-    int block = 0, lanes = 1;
-};
-
 // The smallest power-of-two block of at least one wave whose slots hold the
 // largest cluster (0: none up to max_block lanes).
 int cluster_min_block(int64_t nmax, int lanes, int max_block = 1024)
@@ -1506,30 +1500,28 @@ ClusterLayout cluster_layout(int64_t nmax, int64_t particles, ClusterLimits lim 
 }
 
 // Autotuner of the cluster layout: for runs long enough to repay it, time a
-// few trial steps of the first schedule group with every candidate (one and
+// few trial steps of the launch set with the most particles with every candidate (one and
 // two lanes per slot, unless MAGPY_AMD_CLUSTER_LANES fixes it, each with the
 // power-of-two blocks from the smallest that holds the largest cluster up to
 // 1024 lanes) on throw-away copies of the state, and keep the fastest.
-// Results are cached per (largest cluster, particles, precision) for the
-// life of the process.  Trials run from the group's own first step (a
-// resumed run starts at start_step), and a group too short to time them
-// keeps the untimed layout, uncached.
+// Results are cached (LayoutKey) for the life of the process.  Trials run
+// from the run's own first step (a resumed run starts at start_step), and a
+// run too short to time them keeps the untimed layout, uncached.
 ClusterLayout autotune_cluster_layout(const simulation::EnsembleSpec &sp, const Plan &plan,
+                                      const std::vector<int> &set, int64_t set_particles,
                                       int64_t nmax, hipStream_t s)
 {
-    static std::map<std::tuple<int64_t, int64_t, int, int>, ClusterLayout> cache;
+    static LayoutCache cache;
     const int forced = env_cluster_lanes();
-    const auto key = std::make_tuple(nmax, (int64_t)plan.perm.size(), (int)sp.precision, forced);
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
+    const LayoutKey key{sp.device, nmax, set_particles, (int)sp.precision, forced};
+    ClusterLayout best;
+    if (cache.find(key, best)) return best;
     const int64_t trial_steps = 64;
-    const int64_t first = std::min(sp.start_step, plan.group_steps[0]);
-    if (plan.group_steps[0] - first < 4 + trial_steps)
-        return cluster_layout(nmax, (int64_t)plan.perm.size());
+    const int64_t steps = plan.group_steps[(size_t)set[0]], first = std::min(sp.start_step, steps);
+    if (steps - first < 4 + trial_steps) return cluster_layout(nmax, (int64_t)plan.perm.size());
     hipEvent_t e0, e1;
     MP_HIP(hipEventCreate(&e0));
     MP_HIP(hipEventCreate(&e1));
-    ClusterLayout best;
     float best_ms = 0.f;
     for (int lanes = 1; lanes <= 2; ++lanes) {
         if (forced != 0 && lanes != forced) continue;
@@ -1537,9 +1529,9 @@ ClusterLayout autotune_cluster_layout(const simulation::EnsembleSpec &sp, const 
         for (int b = b0; b != 0 && b <= 1024; b *= 2) {
             std::unique_ptr<GroupBase> g;
             if (sp.precision == MP_PRECISION_FP32)
-                g.reset(new GroupRun<float>(sp, plan, {0}, false, false, b, lanes));
+                g.reset(new GroupRun<float>(sp, plan, set, false, false, b, lanes));
             else
-                g.reset(new GroupRun<double>(sp, plan, {0}, false, false, b, lanes));
+                g.reset(new GroupRun<double>(sp, plan, set, false, false, b, lanes));
             g->enqueue(g->n_done + 4, s);  // warm the code object
             MP_HIP(hipEventRecord(e0, s));
             g->enqueue(g->n_done + trial_steps, s);
@@ -1556,7 +1548,7 @@ ClusterLayout autotune_cluster_layout(const simulation::EnsembleSpec &sp, const 
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    cache[key] = best;
+    cache.keep(key, best);
     return best;
 }
 
@@ -1703,17 +1695,21 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
         throw simulation::Error(MP_ERR_UNSUPPORTED,
                                 "the dipolar product needs an FP32 Heun ensemble of replicas of "
                                 "one cluster with the Philox stream");
+    const std::vector<std::vector<int>> sets = launch_sets(sp, plan, cluster_block != 0, in_arena);
     // pair sums: pick the block size by timing the candidates on long runs
     if (cluster_block != 0 && std::getenv("MAGPY_AMD_CLUSTER_BLOCK") == nullptr &&
-        sp.noise == MP_NOISE_PHILOX && sp.scheme == MP_SCHEME_HEUN &&
-        plan.group_steps[0] >= 20000 && !in_arena)
-        layout = autotune_cluster_layout(sp, plan, nmax, ss->sg.s);
+        sp.noise == MP_NOISE_PHILOX && sp.scheme == MP_SCHEME_HEUN && !in_arena) {
+        int64_t particles = 0;
+        const std::vector<int> &timed = sets[largest_set(sets, plan.group_begin, &particles)];
+        if (plan.group_steps[(size_t)timed[0]] >= 20000)
+            layout = autotune_cluster_layout(sp, plan, timed, particles, nmax, ss->sg.s);
+    }
     cluster_block = layout.block;
     ss->dipolar = cluster_block && sp.interactions ? MP_DIPOLAR_PAIRS : 0;
     ss->cluster_block = cluster_block;
     ss->cluster_lanes = cluster_block ? layout.lanes : 0;
     UploadScope uploads;
-    for (const std::vector<int> &set : launch_sets(sp, plan, cluster_block != 0, in_arena)) {
+    for (const std::vector<int> &set : sets) {
         if (sp.precision == MP_PRECISION_FP32 && sp.scheme == MP_SCHEME_HEUN)
             ss->groups.emplace_back(
                 new GroupRun<float>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
