@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <mutex>
 #include <tuple>
 #include <vector>
 
@@ -40,19 +41,27 @@ inline size_t largest_set(const std::vector<std::vector<int>> &sets,
 // the timed set, precision, lanes forced by the environment (0: none).
 using LayoutKey = std::tuple<int, int64_t, int64_t, int, int>;
 
-// Tuned layouts, for the life of the process
+// Tuned layouts, for the life of the process.  Threads create sessions at the same
+// time (the Python binding releases the interpreter lock), so every access is locked;
+// two that tune one key at once keep the later's layout.
 class LayoutCache {
   public:
     bool find(const LayoutKey &key, ClusterLayout &out) const
     {
+        std::lock_guard<std::mutex> lock(m);
         auto it = known.find(key);
         if (it == known.end()) return false;
         out = it->second;
         return true;
     }
-    void keep(const LayoutKey &key, const ClusterLayout &l) { known[key] = l; }
+    void keep(const LayoutKey &key, const ClusterLayout &l)
+    {
+        std::lock_guard<std::mutex> lock(m);
+        known[key] = l;
+    }
 
   private:
+    mutable std::mutex m;
     std::map<LayoutKey, ClusterLayout> known;
 };
 
