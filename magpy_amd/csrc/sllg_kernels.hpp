@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "cluster_norm.h"
 #include "linalg3.h"
 #include "normal64.h"
 #include "philox.h"
@@ -1371,8 +1372,8 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
 // particles is F: the effective field at every iterate includes the dipolar
 // sum over the cluster's iterates, exchanged through LDS each iteration; and
 // the tolerance eps |guess|_2 and the step norm |delta|_2 are taken over the
-// whole cluster (lib/optimisation.cpp:98, 142), summed over its members in
-// component order, so the lanes of a cluster iterate together.  A singular
+// whole cluster (lib/optimisation.cpp:98, 142), summed in one order for every
+// layout (cluster_square), so the lanes of a cluster iterate together.  A singular
 // block makes the whole system singular: dgesv then leaves its right-hand
 // side -F as the result for every particle of the cluster.  Each particle's
 // drift Jacobian reads the field Jacobian at hj + 3n, n its index in the
@@ -1596,30 +1597,14 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock, 3) void i
 
     // The sum over the cluster of |v|^2: kT lanes add theirs by lane swaps and
     // the first stores the sum (put_square), then every lane adds the cluster's
-    // sums (cluster_sum): up to 64 of four lanes each, eight LDS reads in flight,
-    // or the few of two.
+    // sums (cluster_square).
     auto put_square = [&](const double *v) {
         double q = live ? fmad(v[0], v[0], fmad(v[1], v[1], v[2] * v[2])) : 0.0;
         q += swap_lanes<1>(q);
         if constexpr (kT == 4) q += swap_lanes<2>(q);
         if ((tid & (kT - 1)) == 0) red[tid / kT] = q;
     };
-    auto cluster_sum = [&]() {
-        double sum = 0.0;
-        if constexpr (kT == 2) {
-            for (int k = cb; k < ce; k += 2) sum += red[k / 2];
-            return sum;
-        }
-        for (int k = cb; k < ce; k += 8 * kT) {
-            double v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = red[(k + u * kT < ce ? k + u * kT : cb) / kT];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = k + u * kT < ce ? v[u] : 0.0;
-            sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-        }
-        return sum;
-    };
+    auto cluster_sum = [&]() { return cluster_square<kT>(red, cb, ce); };
     // the field of the state m, the dipolar sum of the published states added
     auto field = [&](const double *m, double applied, double *h) {
         single_field(m, e, k, applied, h);
