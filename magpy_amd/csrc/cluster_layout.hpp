@@ -1,5 +1,6 @@
 // cluster_layout.hpp -- host rules of the cluster kernels' layout that need no
-// device: which launch set the autotuner times and what it remembers.
+// device: which launch set the autotuner times and what it remembers, and how many
+// lanes of the implicit kernel share their pair sums.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -7,6 +8,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 namespace mp_host {
@@ -64,5 +66,30 @@ class LayoutCache {
     mutable std::mutex m;
     std::map<LayoutKey, ClusterLayout> known;
 };
+
+// Lanes of the implicit cluster kernel that share their pair sums (shared_field), 2 or
+// 4, for the members (particle ranges) of a launch; the results are the same.  Four
+// are the faster for clusters of 9 and more, but a small member's helper lanes then
+// take slots of their own.  So: two with no cluster above 8; four where all slots are
+// at most a wave on every SIMD (one_wave), since the largest cluster's wave then takes
+// the launch's time; else four if the slots that helpers add are a sixth of the large
+// clusters' particles or fewer.  us per step with 2 / 4 lanes, 32 steps (helpers /
+// large particles): 65,536 dimers 38 / 105; and one cluster of 9 with them 62 / 115;
+// 6,000 of 9 and 10,000 dimers (0.37) 85 / 96; 2,000 of 64 and 20,000 dimers (0.31)
+// 373 / 409, 8,000 dimers (0.13) 363 / 330; 6,000 of 16 and 3,000 dimers (0.06) 140 /
+// 122.  A wave per SIMD or fewer: 64 of 32 and 512 dimers 116 / 98, one of 9 and 64
+// dimers 49 / 43.
+inline int field_targets(const std::vector<std::pair<int64_t, int64_t>> &members, int64_t one_wave)
+{
+    int64_t slots = 0, helpers = 0, large = 0;
+    for (const auto &m : members) {
+        const int64_t n = m.second - m.first, two = (n + 1) / 2 * 2, four = (n + 3) / 4 * 4;
+        slots += four;
+        if (n > 8) large += n;
+        else helpers += four - two;
+    }
+    if (large == 0) return 2;
+    return slots <= one_wave || 6 * helpers <= large ? 4 : 2;
+}
 
 }  // namespace mp_host

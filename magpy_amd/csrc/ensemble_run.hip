@@ -315,14 +315,6 @@ void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int 
     }
 }
 
-// Lanes of the implicit cluster kernel that share their pair sums (shared_field)
-int field_targets(const std::vector<std::pair<int64_t, int64_t>> &members)
-{
-    int64_t nmax = 1;
-    for (const auto &m : members) nmax = std::max(nmax, m.second - m.first);
-    return nmax > 8 ? 4 : 2;
-}
-
 // The applied field of a schedule group: whether all of its particles see the
 // same one (shape, reduced amplitude, cycles per step), and which.
 struct GroupField {
@@ -509,7 +501,8 @@ struct GroupRun : GroupBase {
             // workgroups that fill every SIMD once
             const size_t run =
                 (size_t)std::max(1, 4 * device_cus() / ((block + mp::kWave - 1) / mp::kWave));
-            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT) targets = field_targets(members);
+            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT)
+                targets = field_targets(members, 4 * (int64_t)device_cus() * mp::kWave);
             pack_clusters(members, block / lanes, targets, run, slot_particle, cbase, csize);
         } else {
             for (int gi : set)

@@ -1403,9 +1403,10 @@ constexpr int kImplicitClusterBlock = 256;   // largest workgroup, so largest cl
 // independent work.  A source was two 32-byte vectors per term; it is 48 bytes
 // for kT terms.  Bound: FP64 issue, ~33 instructions per term, under the card's
 // power limit (2.1 GHz).  kT = 4 is the faster from 9 particles up; in smaller
-// clusters helper lanes and idle residues cost more than the reads (us per
-// iteration, kT 2 / 4: 65,536 dimers 1.64 / 3.5, 8,192 of 8 2.18 / 2.20, 2,048
-// of 64 13.4 / 13.0).  4,096 clusters of 2 to 64, 32 steps, on a warm card:
+// clusters helper lanes and idle residues cost more than the reads (us per step,
+// kT 2 / 4: 65,536 dimers 38 / 105, 16,384 of 8 80 / 88, 14,563 of 9 141 / 141,
+// 8,192 of 16 137 / 122, 2,048 of 64 367 / 333; field_targets has the mixtures).
+// 4,096 clusters of 2 to 64, 32 steps, on a warm card:
 // 11.4 -> 10.65 ms a pass; one dimer, 1,000 steps: 24.6 -> 21.0 ms.
 struct Source {
     double px, py, pz, mx, my, mz;   // position, w m
