@@ -427,7 +427,9 @@ std::vector<std::vector<int>> launch_sets(const simulation::EnsembleSpec &sp, co
 
 template <typename T>
 struct GroupRun : GroupBase {
-    int n = 0, grid = 0, block = mp::kBlock, n_waves = 0, scheme = 0, shape_kind = -1;
+    // n: slots of the arrays, of which a cluster's workgroups have n_slots (implicit
+    // clusters: also helpers and padding, with no place in the arrays)
+    int n = 0, n_slots = 0, grid = 0, block = mp::kBlock, n_waves = 0, scheme = 0, shape_kind = -1;
     int max_iter = 1000;
     double eps = 1e-9;
     bool array_noise = false, want_traj = false, want_ens = false, cluster = false;
@@ -448,7 +450,7 @@ struct GroupRun : GroupBase {
     DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_m, d_samples;   // d_m: x, y, z, each n
     DevBuf<T> d_px, d_py, d_pz, d_w;
     DevBuf<double> d_fred, d_fdt, d_dtd, d_msw, d_noise, d_partial, d_ens;
-    DevBuf<int> d_shape, d_cbase, d_csize;
+    DevBuf<int> d_shape, d_cbase, d_csize, d_row, d_cell;
     DevBuf<uint32_t> d_key0, d_key1, d_pid, d_status;
     DevBuf<int64_t> d_sched;
     DevBuf<unsigned long long> d_newton;      // per slot: iterations, then failures
@@ -504,6 +506,24 @@ struct GroupRun : GroupBase {
             if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT)
                 targets = field_targets(members, 4 * (int64_t)device_cus() * mp::kWave);
             pack_clusters(members, block / lanes, targets, run, slot_particle, cbase, csize);
+            n_slots = (int)slot_particle.size();
+            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT) {
+                // arrays hold the particles alone; 8 bytes a slot find them
+                std::vector<int> row((size_t)n_slots, 0), cell((size_t)n_slots, 0);
+                std::vector<int64_t> particles;
+                for (int i = 0; i < n_slots; ++i) {
+                    cell[(size_t)i] = cbase[(size_t)i] | csize[(size_t)i] << 16;
+                    if (slot_particle[(size_t)i] >= 0) {
+                        row[(size_t)i] = (int)particles.size();
+                        particles.push_back(slot_particle[(size_t)i]);
+                    } else if (csize[(size_t)i] > 0) {   // a helper reads its neighbour's row
+                        row[(size_t)i] = (int)particles.size() - 1;
+                    }
+                }
+                slot_particle = std::move(particles);
+                d_row.upload(row);
+                d_cell.upload(cell);
+            }
         } else {
             for (int gi : set)
                 slot_particle.insert(slot_particle.end(),
@@ -601,12 +621,13 @@ struct GroupRun : GroupBase {
         d_k.upload(cast_vec<T>(k));
         d_al.upload(cast_vec<T>(al));
         d_dt.upload(cast_vec<T>(dt));
-        d_sig.upload(cast_vec<T>(sig));
+        const bool implicit = scheme == MP_SCHEME_IMPLICIT_MIDPOINT;
+        if (!implicit) d_sig.upload(cast_vec<T>(sig));
         d_sr.upload(cast_vec<T>(sr));
         d_happ.upload(cast_vec<T>(happ));
         d_m.upload(cast_vec<T>(m_now));
         d_fred.upload(fred);
-        d_fdt.upload(fdt);
+        if (!implicit) d_fdt.upload(fdt);
         d_dtd.upload(dt);
         d_msw.upload(msw);
         d_shape.upload(shape);
@@ -615,18 +636,20 @@ struct GroupRun : GroupBase {
         d_pid.upload(pid);
         d_status.upload(std::vector<uint32_t>((size_t)n, 0));
         d_sched.upload(sched);
-        if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT)
+        if (implicit)
             d_newton.upload(std::vector<unsigned long long>(2 * (size_t)n, 0));
         if (cluster) {
             d_px.upload(cast_vec<T>(px));
             d_py.upload(cast_vec<T>(py));
             d_pz.upload(cast_vec<T>(pz));
             d_w.upload(cast_vec<T>(w));
-            d_cbase.upload(cbase);
-            d_csize.upload(csize);
+            if (!implicit) {
+                d_cbase.upload(cbase);
+                d_csize.upload(csize);
+            }
         }
         // cluster slots come in whole blocks of block / lanes
-        grid = cluster ? n / (block / lanes) : (n + block - 1) / block;
+        grid = cluster ? n_slots / (block / lanes) : (n + block - 1) / block;
         n_waves = (grid * block) / mp::kWave;
         const bool several = set.size() > 1;
         two_wave = !cluster && !array_noise && scheme == MP_SCHEME_HEUN
@@ -776,8 +799,8 @@ struct GroupRun : GroupBase {
     void launch_implicit_cluster(hipStream_t s)
     {
         mp::ImplicitClusterArgs ia{
-            mp::ClusterArgs<double>{a, d_px.p, d_py.p, d_pz.p, d_w.p, d_cbase.p, d_csize.p}, eps,
-            max_iter, newton_iters(), newton_fails(), interactions ? 1 : 0};
+            mp::ClusterArgs<double>{a, d_px.p, d_py.p, d_pz.p, d_w.p, nullptr, nullptr}, d_row.p,
+            d_cell.p, eps, max_iter, newton_iters(), newton_fails(), interactions ? 1 : 0};
         // a source per slot, a sum per `targets` slots, a flag per slot
         const size_t shmem = (size_t)block * (sizeof(mp::Source) + sizeof(int)) +
                              (size_t)(block / targets) * sizeof(double);

@@ -1385,11 +1385,14 @@ __global__ __launch_bounds__(kBlock) void implicit_indep_kernel(ImplicitArgs ia)
 // interactions the dipolar sums are left out and the cluster still shares
 // its norms, as the reference's 3N system does.
 struct ImplicitClusterArgs {
-    ClusterArgs<double> c;
+    ClusterArgs<double> c;              // (cbase and csize are in cell)
+    const int *row;                     // [slots]: the particle's row of the arrays
+    const int *cell;                    // [slots]: the cluster's first slot in the workgroup,
+                                        // and its size above 16 bits (0: padding)
     double eps;
     int max_iter;
-    unsigned long long *newton_iters;   // [slots]
-    unsigned long long *newton_fail;    // [slots]
+    unsigned long long *newton_iters;   // [n]
+    unsigned long long *newton_fail;    // [n]
     int interactions;                   // 0: no dipolar sums (norms stay per cluster)
 };
 
@@ -1541,10 +1544,12 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock, 3) void i
     int *sing = reinterpret_cast<int *>(red + slots / kT);  // a cluster's first slot: singular block
 
     const int tid = threadIdx.x;
-    const int p = blockIdx.x * slots + tid;   // the grid covers all slots exactly
-    // padding: cn = 0; a helper lane: past the end of its cluster
-    const int cn = ca.csize[p];
-    const int cb = cn > 0 ? ca.cbase[p] : tid, ce = cb + cn;
+    const int slot = blockIdx.x * slots + tid;   // the grid covers all slots exactly
+    // padding: cn = 0; a helper lane: past the end of its cluster.  The arrays hold the
+    // particles alone (with helpers in them a run of singles took twice the memory);
+    // both read a particle's row, which a helper shares with its neighbour
+    const int p = ia.row[slot], cell = ia.cell[slot], cn = cell >> 16;
+    const int cb = cn > 0 ? cell & 0xffff : tid, ce = cb + cn;
     const bool live = tid < ce;
     const bool leader = live && tid == cb;
 
@@ -1579,7 +1584,7 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock, 3) void i
     double c_half[3], e0[3];
     {
         const int nn = live ? cn : 1, idx = live ? tid - cb : 0;
-        const int first = blockIdx.x * slots + cb;
+        const int first = live ? p - idx : p;   // a cluster's rows follow each other
         const double k0 = a.k[first];
         e0[0] = a.ex[first];
         e0[1] = a.ey[first];
