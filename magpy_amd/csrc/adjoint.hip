@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "adjoint_kernels.hpp"
+#include "adjoint_plan.hpp"
 #include "host_util.hpp"
 
 using namespace mp_host;
@@ -255,25 +256,14 @@ struct AdjointRun final : AdjointBase {
         pt.build(sched, N, C);
         n_waves = (int)((P + mp::kWave - 1) / mp::kWave);
         // transfer batches: up to 2^20 lanes (launches of a few waves per SIMD
-        // leave their last round half empty), scratch at most 8 GiB, the block's
-        // segments split evenly
+        // leave their last round half empty)
         const int64_t seg_len = std::min(C, N);
-        const int64_t by_lanes = std::max<int64_t>(1, env_batch_lanes() / P);
-        const int64_t by_bytes = std::max<int64_t>(
-            1, ((int64_t)8 << 30) / ((seg_len + 3) / 4 * 3 * P * (int64_t)sizeof(T)));
-        const int64_t most = std::min({segs_per_block, by_lanes, by_bytes});
-        const int64_t n_batches = (segs_per_block + most - 1) / most;
-        batch_segs = (segs_per_block + n_batches - 1) / n_batches;
-        max_batch_pieces = 1;
-        for (int64_t b0 = 0; b0 < n_ck; b0 += segs_per_block) {
-            const int64_t b1 = std::min(n_ck, b0 + segs_per_block);
-            for (int64_t j0 = b0; j0 < b1; j0 += batch_segs) {
-                const int64_t j1 = std::min(b1, j0 + batch_segs);
-                const int64_t np = (j1 < n_ck ? pt.seg_first[(size_t)j1] : (int64_t)pt.start.size()) -
-                                   pt.seg_first[(size_t)j0];
-                max_batch_pieces = std::max(max_batch_pieces, np);
-            }
-        }
+        const MapBatch batch = map_batch(
+            pt.seg_first, (int64_t)pt.start.size(), segs_per_block, P, env_batch_lanes(),
+            (seg_len + 3) / 4 * 3 * P * (int64_t)sizeof(T),
+            (int64_t)mp::kTransfer * P * (int64_t)sizeof(double));
+        batch_segs = batch.segments;
+        max_batch_pieces = batch.pieces;
         std::vector<T> hx(P), hy(P), hz(P);
         std::vector<uint32_t> k0(P), k1(P);
         for (int64_t p = 0; p < P; ++p) {
@@ -476,7 +466,8 @@ struct AdjointRun final : AdjointBase {
         const int64_t n_a = j0 * C, n_end = std::min(N, j1 * C);
         table(ftab_tr, tr.s, T(1), n_a, n_end - n_a + 2);
         const int64_t piece0 = pt.seg_first[(size_t)j0];
-        const int64_t piece1 = j1 < n_ck ? pt.seg_first[(size_t)j1] : (int64_t)pt.start.size();
+        const int64_t piece1 =
+            piece0 + pieces_of(pt.seg_first, (int64_t)pt.start.size(), j0, j1);
         mp::TransferArgs<T> t{};
         t.n = (int)P;
         t.ex = ex.p;
