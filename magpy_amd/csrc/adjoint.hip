@@ -107,6 +107,8 @@ int64_t env_steps_per_launch()
 // at least 200.  Short segments give small ensembles more lanes and let the maps'
 // waves, some of which share a SIMD with a forward wave, even out (3,000 particles,
 // FP64, 20,000 steps: 9.8 -> 8.1 ms); each costs a transfer of 168 bytes per particle.
+// Against extended precision (15 ensembles of 48 particles, 20,000 steps) the FP64
+// gradient's rms error is 2.7e-14 with segments of 200 steps and 2.9e-14 of 1,000.
 // Not in FP32 (16,384 particles: 8.5 -> 7.1): a map starts at the identity, where each
 // step's small change is rounded to the last place of one, and the gradient was 1.8
 // times as far from FP64.  Above 2^16 particles one segment of every particle fills

@@ -594,7 +594,9 @@ struct GroupRun : GroupBase {
         if (uniform_field) {
             // groups of four aligned below n0, one entry past the last step, and
             // the next group's prefetch: 4 * groups + 5 <= spl + 12
-            if (set.size() > 1)   // at most 64 MB of rows, or rows of 4,096 steps
+            // several: 64 MB of rows, or rows of 4,096 steps where those are more (16 KB a
+            // group; a launch per group had rows of 512 KB)
+            if (set.size() > 1)
                 spl = std::min(spl, std::max((int64_t)4096, ((int64_t)1 << 24) / (int64_t)set.size()));
             tab_stride = spl + 16;
             std::vector<int> row_shape;
