@@ -944,10 +944,13 @@ struct GroupRun : GroupBase {
     {
         GroupOut o;
         if (want_ens) {
-            const int parts = groups.size() > 1 ? (int)groups.size() : n_waves;
-            hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S_out * 3)), dim3(mp::kBlock),
-                               0, s, d_partial.p, parts, S_out * 3, d_ens.p);
-            MP_HIP(hipGetLastError());
+            auto go = [&](auto kernel, int parts) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(S_out * 3)), dim3(mp::kBlock), 0, s,
+                                   d_partial.p, parts, S_out * 3, d_ens.p);
+                MP_HIP(hipGetLastError());
+            };
+            if (groups.size() > 1) go(mp::ens_reduce_kernel<true>, (int)groups.size());
+            else go(mp::ens_reduce_kernel<false>, n_waves);
         }
         MP_HIP(hipStreamSynchronize(s));
         if (state_out) state(state_out);
@@ -1281,7 +1284,7 @@ struct ReplicaRun : GroupBase {
     {
         GroupOut o;
         if (want_ens) {
-            hipLaunchKernelGGL(mp::ens_reduce_kernel, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
+            hipLaunchKernelGGL(mp::ens_reduce_kernel<false>, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
                                s, d_partial.p, n_waves, S * 3, d_ens.p);
             MP_HIP(hipGetLastError());
         }

@@ -1719,21 +1719,42 @@ __global__ __launch_bounds__(kOneWave ? kWave : kImplicitClusterBlock, 3) void i
     }
 }
 
-// Sum per-wave partials of each (sample, component) in a fixed order.
+// x += y with the addition's rounding error added to e (Knuth's two-sum)
+__device__ inline void add_with_error(double &x, double &e, double y)
+{
+#pragma clang fp contract(off)
+    const double s = x + y, b = s - x;
+    e += (x - (s - b)) + (y - b);
+    x = s;
+}
+
+// Sum per-wave partials of each (sample, component) in a fixed order.  kErrors: the
+// partials are those of a launch set's groups, often of one particle each; their sum
+// carries its rounding errors along.
+template <bool kErrors>
 static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int64_t rows, double *out)
 {
+#pragma clang fp contract(off)
     const int64_t r = blockIdx.x;
     if (r >= rows) return;
-    __shared__ double buf[kBlock];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n_waves; i += blockDim.x) acc += partial[r * n_waves + i];
+    __shared__ double buf[kBlock], low[kBlock];
+    auto add = [](double &x, double &e, double y) {
+        if constexpr (kErrors) add_with_error(x, e, y);
+        else x += y;
+    };
+    double acc = 0.0, err = 0.0;
+    for (int i = threadIdx.x; i < n_waves; i += blockDim.x) add(acc, err, partial[r * n_waves + i]);
     buf[threadIdx.x] = acc;
+    low[threadIdx.x] = err;
     __syncthreads();
     for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) buf[threadIdx.x] += buf[threadIdx.x + w];
+        if ((int)threadIdx.x < w) {
+            add(buf[threadIdx.x], low[threadIdx.x], buf[threadIdx.x + w]);
+            low[threadIdx.x] += low[threadIdx.x + w];
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[r] = buf[0];
+    if (threadIdx.x == 0) out[r] = kErrors ? buf[0] + low[0] : buf[0];
 }
 
 // Of a launch set of several schedules: the records [first, end) that a launch has
@@ -1770,7 +1791,8 @@ static __global__ __launch_bounds__(kBlock) void pick_samples_kernel(RecordArgs<
 
 // partial[s][component][group] = sum of Ms m over the group's slots
 // slots[first_slot[g] .. first_slot[g + 1]) for every sample s of the group that is
-// one of the records, by `team` (a power of two up to 64) lanes each, in a fixed order.
+// one of the records, by `team` (a power of two up to 64) lanes each, in a fixed order
+// and with the additions' rounding errors.
 template <typename T>
 static __global__ __launch_bounds__(kBlock) void group_sums_kernel(RecordArgs<T> a,
                                                                    const int32_t *slots,
@@ -1786,19 +1808,23 @@ static __global__ __launch_bounds__(kBlock) void group_sums_kernel(RecordArgs<T>
         const int32_t u = a.pick[g * (size_t)a.S + s];
         if (u < a.first || u >= a.end) continue;
         const T *row = a.records + (size_t)u * 3 * n;
-        double sum[3] = {0.0, 0.0, 0.0};
+        double sum[3] = {0.0, 0.0, 0.0}, err[3] = {0.0, 0.0, 0.0};
         for (int k = first_slot[g] + lane; k < first_slot[g + 1]; k += team) {
             const size_t i = (size_t)slots[k];
             const double w = msw[i];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) sum[c] += (double)row[c * n + i] * w;
+            for (int c = 0; c < 3; ++c) add_with_error(sum[c], err[c], (double)row[c * n + i] * w);
         }
         for (int x = team / 2; x > 0; x /= 2)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) sum[c] += __shfl_xor(sum[c], x);
+            for (int c = 0; c < 3; ++c) {
+                const double other = __shfl_xor(sum[c], x), low = __shfl_xor(err[c], x);
+                add_with_error(sum[c], err[c], other);
+                err[c] += low;
+            }
         if (lane == 0)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) partial[(s * 3 + c) * (size_t)G + g] = sum[c];
+            for (int c = 0; c < 3; ++c) partial[(s * 3 + c) * (size_t)G + g] = sum[c] + err[c];
     }
 }
 
