@@ -22,7 +22,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -258,63 +257,6 @@ struct GroupBase {
     virtual GroupOut collect(hipStream_t s, double *state_out, const SampleSink *samples) = 0;
 };
 
-// Cluster packing: members of a group sorted by size (largest first), each
-// placed in the first block with room; a member never straddles blocks.
-// Returns slot -> particle (-1 padding), and per slot the block-relative
-// start lane of its member and the member size.  A member takes a multiple of
-// `align` slots: those past its size are its helpers (slot_particle -1, with the
-// member's start and size), so every member starts on a multiple of align.
-// Blocks come out largest member first.  The dispatcher deals workgroups round
-// the XCDs, their CUs and SIMDs, so those `run` apart share a SIMD; a
-// workgroup's time goes with its largest member, and every second run of blocks
-// is reversed so that a SIMD gets a long and a short one.
-void pack_clusters(const std::vector<std::pair<int64_t, int64_t>> &members, int block,
-                   int align, size_t run, std::vector<int64_t> &slot_particle,
-                   std::vector<int> &cbase, std::vector<int> &csize)
-{
-    auto taken = [align](int size) { return (size + align - 1) / align * align; };
-    std::vector<size_t> order(members.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) {
-        return members[x].second - members[x].first > members[y].second - members[y].first;
-    });
-    std::vector<int> fill;                       // lanes used per block
-    std::vector<std::vector<size_t>> content;    // members per block
-    size_t first_open = 0;
-    for (size_t oi : order) {
-        const int sz = taken((int)(members[oi].second - members[oi].first));
-        size_t bi = first_open;
-        while (bi < fill.size() && fill[bi] + sz > block) ++bi;
-        if (bi == fill.size()) {
-            fill.push_back(0);
-            content.emplace_back();
-        }
-        fill[bi] += sz;
-        content[bi].push_back(oi);
-        while (first_open < fill.size() && fill[first_open] == block) ++first_open;
-    }
-    for (size_t b = run; b < content.size(); b += 2 * run)
-        std::reverse(content.begin() + (ptrdiff_t)b,
-                     content.begin() + (ptrdiff_t)std::min(content.size(), b + run));
-    const size_t nslots = fill.size() * (size_t)block;
-    slot_particle.assign(nslots, -1);
-    cbase.assign(nslots, 0);
-    csize.assign(nslots, 0);
-    for (size_t bi = 0; bi < content.size(); ++bi) {
-        int lane = 0;
-        for (size_t oi : content[bi]) {
-            const int sz = (int)(members[oi].second - members[oi].first);
-            for (int j = 0; j < taken(sz); ++j) {
-                const size_t slot = bi * (size_t)block + (size_t)(lane + j);
-                if (j < sz) slot_particle[slot] = members[oi].first + j;
-                cbase[slot] = lane;
-                csize[slot] = sz;
-            }
-            lane += taken(sz);
-        }
-    }
-}
-
 // The applied field of a schedule group: whether all of its particles see the
 // same one (shape, reduced amplitude, cycles per step), and which.
 struct GroupField {
@@ -503,11 +445,12 @@ struct GroupRun : GroupBase {
             // workgroups that fill every SIMD once
             const size_t run =
                 (size_t)std::max(1, 4 * device_cus() / ((block + mp::kWave - 1) / mp::kWave));
-            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT)
-                targets = field_targets(members, 4 * (int64_t)device_cus() * mp::kWave);
-            pack_clusters(members, block / lanes, targets, run, slot_particle, cbase, csize);
+            const bool implicit = scheme == MP_SCHEME_IMPLICIT_MIDPOINT;
+            if (implicit) targets = field_targets(members, 4 * (int64_t)device_cus() * mp::kWave);
+            pack_clusters(members, block / lanes, targets, run, reversed_runs(implicit, lanes),
+                          slot_particle, cbase, csize);
             n_slots = (int)slot_particle.size();
-            if (scheme == MP_SCHEME_IMPLICIT_MIDPOINT) {
+            if (implicit) {
                 // arrays hold the particles alone; 8 bytes a slot find them
                 std::vector<int> row((size_t)n_slots, 0), cell((size_t)n_slots, 0);
                 std::vector<int64_t> particles;
