@@ -405,6 +405,7 @@ struct GroupRun : GroupBase {
     DevBuf<int32_t> d_pick, d_slot_group;
     DevBuf<int32_t> d_group_slots, d_group_first;   // the slots of each group
     T *records = nullptr;
+    bool sums_clear = false;
     mp::IndepArgs<T> a{};
 
     // cluster_block == 0: one slot per particle of the group (independent
@@ -610,8 +611,6 @@ struct GroupRun : GroupBase {
             d_partial.alloc((size_t)S_out * 3 * (several ? set.size() : (size_t)n_waves));
             d_ens.alloc((size_t)S_out * 3);
             if (several) {
-                MP_HIP(hipMemset(d_partial.p, 0, d_partial.n * sizeof(double)));
-                MP_HIP(hipStreamSynchronize(nullptr));
                 std::vector<int32_t> first(set.size() + 1, 0), slots;
                 for (int g : slot_group)
                     if (g >= 0) ++first[(size_t)g + 1];
@@ -675,6 +674,14 @@ struct GroupRun : GroupBase {
         if (record_bytes() == 0) return;
         records = static_cast<T *>(p);
         a.samples = records;
+    }
+
+    // The sums of samples that a group takes at or before the start are zero
+    void clear_sums(hipStream_t s)
+    {
+        if (sums_clear || groups.size() == 1 || !want_ens) return;
+        MP_HIP(hipMemsetAsync(d_partial.p, 0, d_partial.n * sizeof(double), s));
+        sums_clear = true;
     }
 
     // The samples and sums of the records that a launch of the steps up to n1 wrote:
@@ -838,6 +845,7 @@ struct GroupRun : GroupBase {
     void enqueue(int64_t upto, hipStream_t s) override
     {
         upto = std::min(upto, n_total);
+        clear_sums(s);
         while (n_done < upto) {
             const int64_t n1 = std::min(upto, n_done + spl);
             while (s_next < S && sched[(size_t)s_next] < n_done + 1) ++s_next;
@@ -886,6 +894,7 @@ struct GroupRun : GroupBase {
     GroupOut collect(hipStream_t s, double *state_out, const SampleSink *sink) override
     {
         GroupOut o;
+        clear_sums(s);
         if (want_ens) {
             auto go = [&](auto kernel, int parts) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)(S_out * 3)), dim3(mp::kBlock), 0, s,
