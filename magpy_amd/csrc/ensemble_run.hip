@@ -391,7 +391,7 @@ struct GroupRun : GroupBase {
     std::vector<std::vector<int32_t>> pick;
     DevBuf<T> d_ex, d_ey, d_ez, d_k, d_al, d_dt, d_sig, d_sr, d_happ, d_m, d_samples;   // d_m: x, y, z, each n
     DevBuf<T> d_px, d_py, d_pz, d_w;
-    DevBuf<double> d_fred, d_fdt, d_dtd, d_msw, d_noise, d_partial, d_ens;
+    DevBuf<double> d_fred, d_fdt, d_dtd, d_msw, d_noise, d_partial;   // d_partial: then the sums
     DevBuf<int> d_shape, d_cbase, d_csize, d_row, d_cell;
     DevBuf<uint32_t> d_key0, d_key1, d_pid, d_status;
     DevBuf<int64_t> d_sched;
@@ -404,15 +404,15 @@ struct GroupRun : GroupBase {
     DevBuf<int64_t> d_toff;                   // per slot: start of its row (several rows)
     DevBuf<int32_t> d_pick, d_slot_group;
     DevBuf<int32_t> d_group_slots, d_group_first;   // the slots of each group
-    T *records = nullptr;
-    bool sums_clear = false;
+    T *records = nullptr;      // at the end of d_samples, or the run's (use_records)
+    size_t n_samples = 0;      // values of d_samples that are samples
     mp::IndepArgs<T> a{};
 
     // cluster_block == 0: one slot per particle of the group (independent
     // particles); otherwise members packed into blocks of cluster_block lanes,
-    // cluster_lanes (1 or 2) lanes per slot.
+    // cluster_lanes (1 or 2) lanes per slot.  sole_set: no other set shares its records.
     GroupRun(const simulation::EnsembleSpec &sp, const Plan &plan, const std::vector<int> &set,
-             bool traj, bool ens, int cluster_block, int cluster_lanes = 1)
+             bool traj, bool ens, int cluster_block, int cluster_lanes = 1, bool sole_set = false)
         : groups(set)
     {
         const int64_t P = sp.member_offsets[sp.n_members];
@@ -603,13 +603,15 @@ struct GroupRun : GroupBase {
                        : 0;
         // the one-wave kernel reads one table row
         if (several && uniform_field) two_wave = std::max(two_wave, 1);
-        if (want_traj) d_samples.alloc((size_t)S_out * 3 * (size_t)n);
+        if (want_traj) n_samples = (size_t)S_out * 3 * (size_t)n;
+        const size_t own_records = sole_set ? record_bytes() / sizeof(T) : 0;
+        if (n_samples + own_records) d_samples.alloc(n_samples + own_records);
+        if (own_records) records = d_samples.p + n_samples;
         if (want_ens) {
             // each recorded sample writes all of its (component, wave) slots;
             // slots of samples taken at step 0 are replaced on the host.  Several
-            // schedules: a slot per group, zero where the group took no sample
-            d_partial.alloc((size_t)S_out * 3 * (several ? set.size() : (size_t)n_waves));
-            d_ens.alloc((size_t)S_out * 3);
+            // schedules: a slot per group
+            d_partial.alloc((size_t)S_out * 3 * ((several ? set.size() : (size_t)n_waves) + 1));
             if (several) {
                 std::vector<int32_t> first(set.size() + 1, 0), slots;
                 for (int g : slot_group)
@@ -653,7 +655,7 @@ struct GroupRun : GroupBase {
         a.status = d_status.p;
         a.sched = d_sched.p;
         a.S = S;
-        a.samples = several ? nullptr : d_samples.p;   // several: use_records
+        a.samples = several ? records : d_samples.p;
         a.ens_partial = several ? nullptr : d_partial.p;
         a.tag = sp.noise_tag;
         a.renorm = sp.renorm ? 1 : 0;
@@ -666,8 +668,8 @@ struct GroupRun : GroupBase {
 
     size_t record_bytes() const override
     {
-        return groups.size() > 1 && (want_traj || want_ens) ? (size_t)S * 3 * (size_t)n * sizeof(T)
-                                                            : 0;
+        const bool shared = groups.size() > 1 && (want_traj || want_ens) && records == nullptr;
+        return shared ? (size_t)S * 3 * (size_t)n * sizeof(T) : 0;
     }
     void use_records(void *p) override
     {
@@ -675,14 +677,8 @@ struct GroupRun : GroupBase {
         records = static_cast<T *>(p);
         a.samples = records;
     }
-
-    // The sums of samples that a group takes at or before the start are zero
-    void clear_sums(hipStream_t s)
-    {
-        if (sums_clear || groups.size() == 1 || !want_ens) return;
-        MP_HIP(hipMemsetAsync(d_partial.p, 0, d_partial.n * sizeof(double), s));
-        sums_clear = true;
-    }
+    // the sums [S_out][3] of the set, behind its partial sums
+    double *ens_sums() const { return d_partial.p + (d_partial.n - (size_t)S_out * 3); }
 
     // The samples and sums of the records that a launch of the steps up to n1 wrote:
     // those from s_next on.  A group takes a sample at one step, so that its sum has
@@ -700,23 +696,18 @@ struct GroupRun : GroupBase {
         }
         if (lo >= hi) return;
         const int64_t G = (int64_t)groups.size(), most = 16 * (int64_t)device_cus();
-        auto blocks = [&](int64_t threads) {
-            return dim3((unsigned)std::min((threads + mp::kBlock - 1) / mp::kBlock, most));
+        auto blocks = [&](bool wanted, int64_t threads) {
+            return wanted ? (int)std::min((threads + mp::kBlock - 1) / mp::kBlock, most) : 0;
         };
         const mp::RecordArgs<T> r{records, d_pick.p, n, S_out, lo, hi, first, end};
-        if (want_traj) {
-            hipLaunchKernelGGL(mp::pick_samples_kernel<T>, blocks((hi - lo) * n), dim3(mp::kBlock), 0,
-                               s, r, d_slot_group.p, d_samples.p);
-            MP_HIP(hipGetLastError());
-        }
-        if (want_ens) {
-            int team = 1;   // lanes per sum: the slots of a group on average, to a wave
-            while (team < mp::kWave && team * G < (int64_t)d_group_slots.n) team *= 2;
-            hipLaunchKernelGGL(mp::group_sums_kernel<T>, blocks((hi - lo) * G * team),
-                               dim3(mp::kBlock), 0, s, r, d_group_slots.p, d_group_first.p, (int)G,
-                               team, d_msw.p, d_partial.p);
-            MP_HIP(hipGetLastError());
-        }
+        int team = 1;   // lanes per sum: the slots of a group on average, to a wave
+        while (team < mp::kWave && team * G < (int64_t)d_group_slots.n) team *= 2;
+        const mp::GroupSums q{d_group_slots.p, d_group_first.p, (int)G, team, d_msw.p, d_partial.p};
+        const int sample_blocks = blocks(want_traj, (hi - lo) * n);
+        const int sum_blocks = blocks(want_ens, (hi - lo) * G * team);
+        hipLaunchKernelGGL(mp::take_records_kernel<T>, dim3((unsigned)(sample_blocks + sum_blocks)),
+                           dim3(mp::kBlock), 0, s, r, d_slot_group.p, d_samples.p, sample_blocks, q);
+        MP_HIP(hipGetLastError());
     }
 
     unsigned long long *newton_iters() const { return d_newton.p; }
@@ -845,7 +836,6 @@ struct GroupRun : GroupBase {
     void enqueue(int64_t upto, hipStream_t s) override
     {
         upto = std::min(upto, n_total);
-        clear_sums(s);
         while (n_done < upto) {
             const int64_t n1 = std::min(upto, n_done + spl);
             while (s_next < S && sched[(size_t)s_next] < n_done + 1) ++s_next;
@@ -894,11 +884,10 @@ struct GroupRun : GroupBase {
     GroupOut collect(hipStream_t s, double *state_out, const SampleSink *sink) override
     {
         GroupOut o;
-        clear_sums(s);
         if (want_ens) {
             auto go = [&](auto kernel, int parts) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)(S_out * 3)), dim3(mp::kBlock), 0, s,
-                                   d_partial.p, parts, S_out * 3, d_ens.p);
+                                   d_partial.p, parts, S_out * 3, ens_sums(), d_pick.p);
                 MP_HIP(hipGetLastError());
             };
             if (groups.size() > 1) go(mp::ens_reduce_kernel<true>, (int)groups.size());
@@ -918,15 +907,15 @@ struct GroupRun : GroupBase {
             }
         }
         if (sink != nullptr && want_traj) {
-            std::unique_ptr<T[]> h(new T[d_samples.n]);
-            if (d_samples.n)
-                MP_HIP(hipMemcpy(h.get(), d_samples.p, d_samples.n * sizeof(T),
+            std::unique_ptr<T[]> h(new T[n_samples]);
+            if (n_samples)
+                MP_HIP(hipMemcpy(h.get(), d_samples.p, n_samples * sizeof(T),
                                  hipMemcpyDeviceToHost));
             sink->take(h.get(), slot_particle);
         }
         if (want_ens) {
             o.ens.resize((size_t)S_out * 3);
-            MP_HIP(hipMemcpy(o.ens.data(), d_ens.p, o.ens.size() * sizeof(double),
+            MP_HIP(hipMemcpy(o.ens.data(), ens_sums(), o.ens.size() * sizeof(double),
                              hipMemcpyDeviceToHost));
         }
         return o;
@@ -1237,7 +1226,7 @@ struct ReplicaRun : GroupBase {
         GroupOut o;
         if (want_ens) {
             hipLaunchKernelGGL(mp::ens_reduce_kernel<false>, dim3((unsigned)(S * 3)), dim3(mp::kBlock), 0,
-                               s, d_partial.p, n_waves, S * 3, d_ens.p);
+                               s, d_partial.p, n_waves, S * 3, d_ens.p, nullptr);
             MP_HIP(hipGetLastError());
         }
         MP_HIP(hipStreamSynchronize(s));
@@ -1685,10 +1674,12 @@ mp_session *session_create(const simulation::EnsembleSpec &sp, bool traj, bool e
     for (const std::vector<int> &set : sets) {
         if (sp.precision == MP_PRECISION_FP32 && sp.scheme == MP_SCHEME_HEUN)
             ss->groups.emplace_back(
-                new GroupRun<float>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
+                new GroupRun<float>(sp, plan, set, traj, ens, cluster_block, layout.lanes,
+                                    sets.size() == 1));
         else
             ss->groups.emplace_back(
-                new GroupRun<double>(sp, plan, set, traj, ens, cluster_block, layout.lanes));
+                new GroupRun<double>(sp, plan, set, traj, ens, cluster_block, layout.lanes,
+                                     sets.size() == 1));
     }
     uploads.flush();
     size_t record_bytes = 0;

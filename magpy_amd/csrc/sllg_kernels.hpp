@@ -1728,22 +1728,28 @@ __device__ inline void add_with_error(double &x, double &e, double y)
     x = s;
 }
 
-// Sum per-wave partials of each (sample, component) in a fixed order.  kErrors: the
-// partials are those of a launch set's groups, often of one particle each; their sum
-// carries its rounding errors along.
-template <bool kErrors>
-static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int64_t rows, double *out)
+// Sum per-wave partials of each (sample, component) in a fixed order.  kGroups: the
+// partials are those of a launch set's groups, often of one particle each, without
+// those that took no record of the sample (pick[group][rows / 3]); their sum carries its
+// rounding errors along.
+template <bool kGroups>
+static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int64_t rows, double *out,
+                                         const int32_t *pick)
 {
 #pragma clang fp contract(off)
     const int64_t r = blockIdx.x;
     if (r >= rows) return;
     __shared__ double buf[kBlock], low[kBlock];
     auto add = [](double &x, double &e, double y) {
-        if constexpr (kErrors) add_with_error(x, e, y);
+        if constexpr (kGroups) add_with_error(x, e, y);
         else x += y;
     };
     double acc = 0.0, err = 0.0;
-    for (int i = threadIdx.x; i < n_waves; i += blockDim.x) add(acc, err, partial[r * n_waves + i]);
+    for (int i = threadIdx.x; i < n_waves; i += blockDim.x) {
+        if constexpr (kGroups)
+            if (pick[(size_t)i * (size_t)(rows / 3) + (size_t)(r / 3)] < 0) continue;
+        add(acc, err, partial[r * n_waves + i]);
+    }
     buf[threadIdx.x] = acc;
     low[threadIdx.x] = err;
     __syncthreads();
@@ -1754,7 +1760,7 @@ static __global__ void ens_reduce_kernel(const double *partial, int n_waves, int
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[r] = kErrors ? buf[0] + low[0] : buf[0];
+    if (threadIdx.x == 0) out[r] = kGroups ? buf[0] + low[0] : buf[0];
 }
 
 // Of a launch set of several schedules: the records [first, end) that a launch has
@@ -1772,13 +1778,11 @@ struct RecordArgs {
 // samples[s][component][slot] of every slot whose sample s is one of the records.
 // Bound by its reads and writes, 48 bytes (FP64) a sample and slot.
 template <typename T>
-static __global__ __launch_bounds__(kBlock) void pick_samples_kernel(RecordArgs<T> a,
-                                                                     const int32_t *slot_group,
-                                                                     T *samples)
+__device__ inline void pick_samples(const RecordArgs<T> &a, size_t first, size_t step,
+                                    const int32_t *slot_group, T *samples)
 {
     const size_t n = (size_t)a.n, total = (size_t)(a.hi - a.lo) * n;
-    for (size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x; t < total;
-         t += (size_t)gridDim.x * kBlock) {
+    for (size_t t = first; t < total; t += step) {
         const size_t s = (size_t)a.lo + t / n, i = t % n;
         const int g = slot_group[i];
         if (g < 0) continue;
@@ -1793,29 +1797,32 @@ static __global__ __launch_bounds__(kBlock) void pick_samples_kernel(RecordArgs<
 // slots[first_slot[g] .. first_slot[g + 1]) for every sample s of the group that is
 // one of the records, by `team` (a power of two up to 64) lanes each, in a fixed order
 // and with the additions' rounding errors.
+struct GroupSums {
+    const int32_t *slots, *first_slot;
+    int G, team;
+    const double *msw;
+    double *partial;
+};
+
 template <typename T>
-static __global__ __launch_bounds__(kBlock) void group_sums_kernel(RecordArgs<T> a,
-                                                                   const int32_t *slots,
-                                                                   const int32_t *first_slot, int G,
-                                                                   int team, const double *msw,
-                                                                   double *partial)
+__device__ inline void group_sums(const RecordArgs<T> &a, size_t first, size_t step,
+                                  const GroupSums &q)
 {
-    const size_t n = (size_t)a.n, total = (size_t)(a.hi - a.lo) * (size_t)G;
-    const int lane = threadIdx.x & (team - 1);
-    for (size_t t = ((size_t)blockIdx.x * kBlock + threadIdx.x) / team; t < total;
-         t += (size_t)gridDim.x * kBlock / team) {
-        const size_t s = (size_t)a.lo + t / (size_t)G, g = t % (size_t)G;
+    const size_t n = (size_t)a.n, G = (size_t)q.G, total = (size_t)(a.hi - a.lo) * G;
+    const int lane = threadIdx.x & (q.team - 1);
+    for (size_t t = first / q.team; t < total; t += step / q.team) {
+        const size_t s = (size_t)a.lo + t / G, g = t % G;
         const int32_t u = a.pick[g * (size_t)a.S + s];
         if (u < a.first || u >= a.end) continue;
         const T *row = a.records + (size_t)u * 3 * n;
         double sum[3] = {0.0, 0.0, 0.0}, err[3] = {0.0, 0.0, 0.0};
-        for (int k = first_slot[g] + lane; k < first_slot[g + 1]; k += team) {
-            const size_t i = (size_t)slots[k];
-            const double w = msw[i];
+        for (int k = q.first_slot[g] + lane; k < q.first_slot[g + 1]; k += q.team) {
+            const size_t i = (size_t)q.slots[k];
+            const double w = q.msw[i];
 #pragma unroll
             for (int c = 0; c < 3; ++c) add_with_error(sum[c], err[c], (double)row[c * n + i] * w);
         }
-        for (int x = team / 2; x > 0; x /= 2)
+        for (int x = q.team / 2; x > 0; x /= 2)
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const double other = __shfl_xor(sum[c], x), low = __shfl_xor(err[c], x);
@@ -1824,8 +1831,25 @@ static __global__ __launch_bounds__(kBlock) void group_sums_kernel(RecordArgs<T>
             }
         if (lane == 0)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) partial[(s * 3 + c) * (size_t)G + g] = sum[c] + err[c];
+            for (int c = 0; c < 3; ++c) q.partial[(s * 3 + c) * G + g] = sum[c] + err[c];
     }
+}
+
+// What a run asked for of the records: the first sample_blocks workgroups take the
+// samples, the rest the sums (one launch, since a small ensemble's time is its launches).
+template <typename T>
+static __global__ __launch_bounds__(kBlock) void take_records_kernel(RecordArgs<T> a,
+                                                                     const int32_t *slot_group,
+                                                                     T *samples, int sample_blocks,
+                                                                     GroupSums q)
+{
+    const int b = blockIdx.x, sum_blocks = gridDim.x - sample_blocks;
+    if (b < sample_blocks)
+        pick_samples(a, (size_t)b * kBlock + threadIdx.x, (size_t)sample_blocks * kBlock, slot_group,
+                     samples);
+    else
+        group_sums(a, (size_t)(b - sample_blocks) * kBlock + threadIdx.x,
+                   (size_t)sum_blocks * kBlock, q);
 }
 
 // normals j0 .. j0+n-1 of one particle's stream, one lane per normal
